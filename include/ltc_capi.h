@@ -317,10 +317,16 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
  * more rows than one launch of at most one workgroup per CU holds, one
  * launch per NCL * NB rows, then 1 when the module forward's sensory launch
  * walks one list per neuron over all of D (64 < D <= 256 with many rows)
- * instead of per 64-input chunk. Returns the number of values written, or
- * -1 for invalid sizes. The plan depends on the current device's CU count.
+ * instead of per 64-input chunk, then five fields of the register-resident
+ * forward clusters (128 < H <= 512 where the geometry above would stream its
+ * operands): workgroups per cluster (0: not used, and the forward runs in the
+ * geometry above), columns per workgroup, rows per cluster, launches per call
+ * and LDS bytes per workgroup. They keep the state's NaN treatment of the
+ * geometry they replace (cmp_fwd above). Returns the number of values
+ * written, or -1 for invalid sizes. The plan depends on the current device's
+ * CU count.
  */
-#define LTC_PLAN_FIELDS 28
+#define LTC_PLAN_FIELDS 33
 int ltc_launch_plan(int B, int T, int D, int H, int ode_unfolds, long long* out, int n);
 
 /*

@@ -196,10 +196,46 @@ bool plan_cluster(ltc::Plan& p, int ncu) {
   return false;
 }
 
+// Register-resident clusters for 128 < Hp <= 512 where the plan above has no
+// register-resident form: a forward member's 1024 threads hold the compacted
+// synapses of 64 columns or 32, at most 20 or 16 each at any mask density, so
+// no operand is streamed. When the batch leaves a cluster to every row, one
+// row per cluster (ode_fwd_own_kernel); else the fewest rows per cluster of
+// the two-group form that take the batch in one launch of at most one
+// workgroup per CU, and past eight rows as many launches as the batch needs.
+void plan_reg_clusters(ltc::Plan& p, int ncu) {
+  p.rf = ltc::RegCluster{};
+  if (p.Hp <= 128 || p.Hp > 512 || p.B < 1) return;
+  if (p.CP > 0 && p.Hp == 256 && p.KS == 16 && p.RC == 16) return;
+  ltc::RegCluster g{};
+  auto geom = [&](int jw) {
+    g.JW = jw;
+    g.CP = p.Hp / jw;
+    g.KS = 1024 / jw;
+    g.RC = p.Hp / g.KS;
+  };
+  geom(p.Hp <= 320 ? 64 : 32);
+  g.NB = 1;
+  if (p.B * g.CP > ncu) {
+    geom(p.Hp <= 256 ? 64 : 32);
+    const int slots = ncu / g.CP;
+    if (slots < 1) return;
+    for (int nb : {2, 4, 8}) {
+      g.NB = nb;
+      if ((p.B + nb - 1) / nb <= slots) break;
+    }
+  }
+  const int need = (p.B + g.NB - 1) / g.NB, slots = ncu / g.CP;
+  g.NCL = need < slots ? need : slots;
+  g.L = (p.B + g.NCL * g.NB - 1) / (g.NCL * g.NB);
+  g.xcd = (g.NCL + 7) / 8 * 8 * g.CP <= ncu;
+  if (ltc::reg_fwd_lds(g, p.Hp) <= chain_lds_limit()) p.rf = g;
+}
+
 // ---------------------------------------------------------------------------
 // Launch plan
 // ---------------------------------------------------------------------------
-ltc::Plan make_plan_uncached(int B, int T, int D, int H, int U, int ncu) {
+ltc::Plan make_plan_uncached(int B, int T, int D, int H, int U, int ncu, bool reg) {
   ltc::Plan p{};
   p.B = B;
   p.T = T;
@@ -285,6 +321,7 @@ ltc::Plan make_plan_uncached(int B, int T, int D, int H, int U, int ncu) {
   p.JWB = 64;
   p.LCH = p.LCHB = 1;
   plan_cluster(p, ncu);
+  if (reg) plan_reg_clusters(p, ncu);
   // Recurrent parameter-gradient chunks: about 1024 workgroups, at least 32
   // unfold instances each, at most 64 partials per synapse.
   if (p.FUSE) {
@@ -325,8 +362,11 @@ ltc::Plan make_plan_uncached(int B, int T, int D, int H, int U, int ncu) {
 // The plans of the last few sizes asked for on this thread: a training step
 // asks for the same sizes several times (saved-buffer and workspace sizes,
 // then the call itself, forward and backward).
-ltc::Plan make_plan(int B, int T, int D, int H, int U, int ncu = device_cus()) {
-  constexpr int kKey = 7;
+// `reg` false: without the register-resident clusters (the no-allocation
+// forward falls back to it where their images would not fit its scratch).
+ltc::Plan make_plan(int B, int T, int D, int H, int U, bool reg = true) {
+  constexpr int kKey = 8;
+  const int ncu = device_cus();
   struct Entry {
     int key[kKey];
     ltc::Plan p;
@@ -335,7 +375,7 @@ ltc::Plan make_plan(int B, int T, int D, int H, int U, int ncu = device_cus()) {
   thread_local Entry cache[kEntries];
   thread_local int used = 0, next = 0;
   // the plan also depends on the device's per-workgroup LDS limit
-  const int key[kKey] = {B, T, D, H, U, ncu, (int)chain_lds_limit()};
+  const int key[kKey] = {B, T, D, H, U, ncu, (int)chain_lds_limit(), reg ? 1 : 0};
   for (int i = 0; i < used; ++i) {
     const Entry& e = cache[i];
     bool hit = true;
@@ -344,7 +384,7 @@ ltc::Plan make_plan(int B, int T, int D, int H, int U, int ncu = device_cus()) {
   }
   Entry& e = cache[next];
   for (int i = 0; i < kKey; ++i) e.key[i] = key[i];
-  e.p = make_plan_uncached(B, T, D, H, U, ncu);
+  e.p = make_plan_uncached(B, T, D, H, U, ncu, reg);
   next = (next + 1) % kEntries;
   if (used < kEntries) ++used;
   return e.p;
@@ -373,7 +413,7 @@ std::atomic<long long> g_spin{ltc::kDefaultSpinTicks};
 // Compacted images of the register-resident cluster kernels (forward / chain).
 void carve_cmp(const ltc::Plan& p, Carver& c, ltc::Prepped& pp, bool fwd, bool bwd) {
   const long long n = (long long)p.Hp * p.Hp;
-  if (fwd && ltc::cmp_fwd(p)) {
+  if (fwd && ltc::fwd_image_cmp(p)) {
     pp.cF = c.take<float4>(n);
     pp.cFi = c.take<int>(n);
     pp.cFn = c.take<int>(p.Hp);
@@ -387,7 +427,7 @@ void carve_cmp(const ltc::Plan& p, Carver& c, ltc::Prepped& pp, bool fwd, bool b
 
 ltc::ClusterBuf carve_cluster(const ltc::Plan& p, Carver& c, bool bwd) {
   ltc::ClusterBuf cb{nullptr, nullptr, g_spin.load(std::memory_order_relaxed)};
-  if (p.CP > 0) {
+  if (bwd ? ltc::bwd_clusters(p) : ltc::fwd_clusters(p)) {
     cb.xch = c.take<unsigned long long>(bwd ? ltc::cluster_words_bwd(p) : ltc::cluster_words(p));
     cb.status = c.take<int>(1);
   }
@@ -737,7 +777,10 @@ long long ltc_bwd_workspace_bytes(int B, int T, int D, int H, int ode_unfolds) {
   return round_up(c.off, 256);
 }
 
-int ltc_full_forward(const float* x, long long sxb, long long sxt, long long sxd,
+namespace {
+
+// ltc_full_forward, with or without the register-resident clusters.
+int full_forward(bool reg, const float* x, long long sxb, long long sxt, long long sxd,
                      const float* state, const float* w_pos, const float* w_erev,
                      const float* mu, const float* sigma, const float* sensory_mu,
                      const float* sensory_sigma, const float* sensory_erev,
@@ -754,7 +797,7 @@ int ltc_full_forward(const float* x, long long sxb, long long sxt, long long sxd
   if (B > 0 && (!state || !h_final)) return fail(LTC_EINVAL, "state/h_final pointer is NULL");
   if ((long long)B * T > 0 && (!x || !out)) return fail(LTC_EINVAL, "x/out pointer is NULL");
   if (save_intermediates && !saved) return fail(LTC_EINVAL, "saved pointer is NULL");
-  const ltc::Plan p = make_plan(B, T, D, H, ode_unfolds);
+  const ltc::Plan p = make_plan(B, T, D, H, ode_unfolds, reg);
   Carver need{nullptr};
   carve_fwd(p, need);
   if (workspace_bytes < need.off || (need.off > 0 && !workspace))
@@ -788,7 +831,7 @@ int ltc_full_forward(const float* x, long long sxb, long long sxt, long long sxd
                                w.cb, s);
   });
   if (e != hipSuccess) return hip_fail("ODE forward launch", e);
-  if (p.CP > 0) {
+  if (ltc::fwd_clusters(p)) {
     ltc::FillList fl = poison_list(w.cb);
     ltc::fill_add(fl, out, nullptr, (long long)B * T * H);
     ltc::fill_add(fl, h_final, nullptr, (long long)B * H);
@@ -796,6 +839,22 @@ int ltc_full_forward(const float* x, long long sxb, long long sxt, long long sxd
     return run_fill(fl, s);
   }
   return LTC_OK;
+}
+
+}  // namespace
+
+int ltc_full_forward(const float* x, long long sxb, long long sxt, long long sxd,
+                     const float* state, const float* w_pos, const float* w_erev,
+                     const float* mu, const float* sigma, const float* sensory_mu,
+                     const float* sensory_sigma, const float* sensory_erev,
+                     const float* sensory_w_pos, const float* cm_t, const float* gleak_pos,
+                     const float* vleak, int B, int T, int D, int H, int ode_unfolds,
+                     float epsilon, int save_intermediates, float* out, float* h_final,
+                     float* saved, void* workspace, long long workspace_bytes, void* stream) {
+  return full_forward(true, x, sxb, sxt, sxd, state, w_pos, w_erev, mu, sigma, sensory_mu,
+                      sensory_sigma, sensory_erev, sensory_w_pos, cm_t, gleak_pos, vleak, B, T, D,
+                      H, ode_unfolds, epsilon, save_intermediates, out, h_final, saved, workspace,
+                      workspace_bytes, stream);
 }
 
 int ltc_full_forward_noalloc(const float* x, long long sxb, long long sxt, long long sxd,
@@ -811,6 +870,13 @@ int ltc_full_forward_noalloc(const float* x, long long sxb, long long sxt, long 
   if (rc != LTC_OK) return rc;
   Carver need{nullptr};
   carve_fwd(make_plan(B, T, D, H, ode_unfolds), need);
+  // The register-resident clusters' images take a little more than the dense
+  // ones: sizes that only fit without them run without them.
+  const bool reg = need.off <= LTC_NOALLOC_SCRATCH_BYTES;
+  if (!reg) {
+    need = Carver{nullptr};
+    carve_fwd(make_plan(B, T, D, H, ode_unfolds, false), need);
+  }
   if (need.off > LTC_NOALLOC_SCRATCH_BYTES)
     return fail(LTC_EUNSUPPORTED,
                 "these sizes need " + std::to_string(need.off) +
@@ -819,7 +885,7 @@ int ltc_full_forward_noalloc(const float* x, long long sxb, long long sxt, long 
                     " (use ltc_full_forward with a workspace)");
   void* ws = noalloc_scratch();
   if (ws == nullptr) return LTC_EHIP;
-  return ltc_full_forward(x, sxb, sxt, sxd, state, w_pos, w_erev, mu, sigma, sensory_mu,
+  return full_forward(reg, x, sxb, sxt, sxd, state, w_pos, w_erev, mu, sigma, sensory_mu,
                           sensory_sigma, sensory_erev, sensory_w_pos, cm_t, gleak_pos, vleak, B,
                           T, D, H, ode_unfolds, epsilon, save_intermediates, out, h_final, saved,
                           ws, LTC_NOALLOC_SCRATCH_BYTES, stream);
@@ -1052,7 +1118,7 @@ int ltc_module_forward(const float* x, long long sxb, long long sxt, long long s
                                densave, wfw.cb, s);
   });
   if (e != hipSuccess) return hip_fail("ODE forward launch", e);
-  if (p.CP > 0) {
+  if (ltc::fwd_clusters(p)) {
     ltc::FillList fl = poison_list(wfw.cb);
     ltc::fill_add(fl, out, nullptr, (long long)B * T * H);
     ltc::fill_add(fl, h_final, nullptr, (long long)B * H);
@@ -1458,7 +1524,7 @@ int ltc_ode_unfold_fwd(const float* state, const float* w_pos, const float* w_er
     e = ltc::launch_copy_rows(vsave, p.Hp, v_buffer, H, (long long)ode_unfolds * B, H, s);
     if (e != hipSuccess) return hip_fail("copy launch", e);
   }
-  if (p.CP > 0) {
+  if (ltc::fwd_clusters(p)) {
     ltc::FillList fl = poison_list(w.f.cb);
     ltc::fill_add(fl, state_out, nullptr, (long long)B * H);
     ltc::fill_add(fl, v_buffer, nullptr, save_intermediates ? (long long)ode_unfolds * B * H : 0);
@@ -1554,10 +1620,11 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
                                 ltc::kFinRec);
   });
   if (e != hipSuccess) return hip_fail("finalize launch", e);
-  if (p.CP > 0) {
+  {
     // Either the recompute (forward) or the chain may have given up; both
     // status words gate the same fill.
     for (const ltc::ClusterBuf* cb : {&w.f.cb, &w.b.cb}) {
+      if (cb->status == nullptr) continue;  // no clusters in that launch
       ltc::FillList fl = poison_list(*cb);
       for (float* z : {grad_v, grad_w_num_sensory, grad_w_den_sensory})
         ltc::fill_add(fl, z, nullptr, (long long)B * H);
@@ -1587,7 +1654,8 @@ int ltc_launch_plan(int B, int T, int D, int H, int ode_unfolds, long long* out,
       p.CP > 0 ? (long long)p.NCLB * p.CPB : (B + p.NB - 1) / p.NB,
       ltc::cmp_fwd(p) ? 1 : 0, ltc::cmp_bwd(p) ? 1 : 0, ltc::prep_sens_fused(p) ? 1 : 0,
       ltc::row_bwd_fused(p) ? 1 : 0, ltc::row128_rec_fused(p) ? 1 : 0, p.LCH, p.LCHB,
-      ltc::sens_full_list(p) ? 1 : 0};
+      ltc::sens_full_list(p) ? 1 : 0,
+      p.rf.CP, p.rf.JW, p.rf.NB, p.rf.L, p.rf.CP > 0 ? ltc::reg_fwd_lds(p.rf, p.Hp) : 0};
   const int m = n < LTC_PLAN_FIELDS ? n : LTC_PLAN_FIELDS;
   for (int i = 0; i < m; ++i) out[i] = v[i];
   return m;

@@ -3907,9 +3907,8 @@ struct FwdCK {
   const int* cidx;
   const int* ccnt;
   int R0;  // first batch row of this launch (launches take NCL * NB rows each)
+  int NCL; // register-resident clusters: clusters of this launch (the grid may hold more)
 };
-
-
 
 // RCP = 16 (Hp = 256): the compacted image (CMP). Thread (o, ks) holds the
 // entries ks, ks + 16, ... of column c's active rows, and the wave runs as
@@ -4086,21 +4085,35 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl_kernel(FwdCK k) {
 // unfold and alternate the two slots, so a slot is overwritten only after
 // every partner has published the group's following state, which it does
 // after it has gathered the slot's words. Waits are bounded as there.
-template <int NB>
+//
+// Members of JW = 64 columns (16 chunks) or 32 (32 chunks, two per wave), each
+// thread at most RC = Hp / KS <= 16 compacted synapses. NF keeps the dense
+// kernels' treatment of a NaN state where a dense kernel ran before: the
+// synapses that the image leaves out have weight zero, and 0 * NaN is NaN, so
+// a NaN in a row's state v^n makes every neuron of that row NaN at v^{n+1}.
+// Each state value is tested when it is written to LDS, and a row flag by
+// unfold parity carries the result to the owners.
+template <int NB, int JW = kClW, bool NF = false>
 __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
   static_assert(NB == 2 || NB == 4 || NB == 8, "two groups of rows");
-  constexpr int HB = NB / 2, RCP = 16, PER = NB * kClW, PERG = HB * kClW;
+  constexpr int HB = NB / 2, RCP = 16, PER = NB * JW, PERG = HB * JW;
+  // gather words per thread and group: (CP - 1) * PERG <= XW * 1024
+  constexpr int XW = JW == 32 && HB == 4 ? 2 : 1;
   extern __shared__ float4 lds4[];
   __shared__ int gave_up;
+  __shared__ int nanrow[2][NB];  // NF: the row's state of that unfold parity holds a NaN
   const int Hp = k.Hp, H = k.H, KS = k.KS, B = k.B, T = k.T, U = k.U, CP = k.CP;
   float* vs = reinterpret_cast<float*>(lds4);                          // [Hp][NB]
-  float2* red = reinterpret_cast<float2*>(vs + NB * Hp);               // [2][KS][HB][64]
-  int4* slot_tab = reinterpret_cast<int4*>(red + 2 * KS * HB * kClW);  // [4][threads]
+  float2* red = reinterpret_cast<float2*>(vs + NB * Hp);               // [2][KS][HB][JW]
+  int4* slot_tab = reinterpret_cast<int4*>(red + 2 * KS * HB * JW);    // [4][threads]
   const int tid = threadIdx.x, nthr = blockDim.x;
-  const int ks = __builtin_amdgcn_readfirstlane(tid >> 6), o = tid & 63;
+  // with JW = 64 ks is uniform across each wave; with JW = 32 a wave holds two
+  const int ks = JW == 64 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid / JW;
+  const int o = tid % JW;
   int p, cl;
   cluster_coords(blockIdx.x, CP, k.xcd_local != 0, p, cl);
-  const int c = p * kClW + o;
+  if (NF && cl >= k.NCL) return;  // grid padded to whole rounds of the XCDs
+  const int c = p * JW + o;
   const int b0 = k.R0 + cl * NB;
   const bool owner = ks < NB;  // finishes row bo = ks of column c (the plan keeps KS >= NB)
   const int bo = ks, og = ks / HB;
@@ -4109,23 +4122,32 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
   const float C = k.neuron[c], G = k.neuron[Hp + c], L = k.neuron[2 * Hp + c];
   const float GL = G * L, CG = C + G;
 
+  if (NF && tid < 2 * NB) nanrow[tid / NB][tid % NB] = 0;  // before balanced_lane's barriers
+
   // Synapse lane in balanced order, as in ode_fwd_cl_kernel.
   float4 preg[RCP];
+  // chunks of a column, and slots of a chunk (16 each at Hp = 256)
+  const int NCK = NF ? KS : kCmpChunks, RC = NF ? k.RC : RCP;
   int nslot, sks, so;
   {
     int* perm = reinterpret_cast<int*>(slot_tab + (RCP / 4) * nthr);
     const int cnt0 = k.ccnt[c];
-    const int lane_id = balanced_lane(cnt0 > ks ? (cnt0 - 1 - ks) / kCmpChunks + 1 : 0, tid,
+    const int lane_id = balanced_lane(cnt0 > ks ? (cnt0 - 1 - ks) / NCK + 1 : 0, tid,
                                       nthr, perm, perm + nthr);
-    sks = lane_id >> 6;
-    so = lane_id & 63;
-    const int sc = p * kClW + so;
+    sks = lane_id / JW;
+    so = lane_id % JW;
+    const int sc = p * JW + so;
     const int cnt = k.ccnt[sc];
-    nslot = wave_max(cnt > sks ? (cnt - 1 - sks) / kCmpChunks + 1 : 0);
+    nslot = wave_max(cnt > sks ? (cnt - 1 - sks) / NCK + 1 : 0);
     int ix[RCP];
 #pragma unroll
     for (int rr = 0; rr < RCP; ++rr) {
-      const long long a = (long long)(sks * RCP + rr) * Hp + sc;
+      if (NF && rr >= RC) {  // fewer slots per chunk than registers
+        preg[rr] = make_float4(0.f, 0.f, 0.f, 0.f);
+        ix[rr] = 0;
+        continue;
+      }
+      const long long a = (long long)(sks * RC + rr) * Hp + sc;
       preg[rr] = k.cimg[a];
       ix[rr] = k.cidx[a] * NB * 4;
     }
@@ -4136,21 +4158,28 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
   if (tid == 0) gave_up = 0;
   for (int e = tid; e < NB * Hp; e += nthr) {
     const int b = e / Hp, j = e - b * Hp;
-    vs[j * NB + b] = (k.state0 != nullptr && b0 + b < B && j < H)
-                         ? k.state0[(long long)(b0 + b) * H + j]
-                         : 0.f;
+    const float v = (k.state0 != nullptr && b0 + b < B && j < H)
+                        ? k.state0[(long long)(b0 + b) * H + j]
+                        : 0.f;
+    vs[j * NB + b] = v;
+    if (NF && v != v) nanrow[0][b] = 1;
   }
   lds_barrier();
 
-  // This thread's word of a group gather (threads below (CP - 1) * PERG):
-  // partner member gm, row gr of the group, column gc.
-  const bool gth = tid < (CP - 1) * PERG;
-  int gm = 0, gr = 0, gc = 0;
-  if (gth) {
-    const int q = tid / PERG, r = tid - q * PERG;
-    gm = q + (q >= p ? 1 : 0);
-    gr = r / kClW;
-    gc = r - gr * kClW;
+  // This thread's words of a group gather (threads below (CP - 1) * PERG): the
+  // word's offset in a slot and its state's place in LDS, both for group 0.
+  // (1024 is a multiple of PERG, so a second word lies 1024 / PERG partners on.)
+  static_assert(XW == 1 || 1024 % PERG == 0, "a thread's words share row and column");
+  bool gth[XW];
+  unsigned gwo[XW];
+  int gvo[XW];
+#pragma unroll
+  for (int x = 0; x < XW; ++x) {
+    const int q = (tid + x * 1024) / PERG, gr = tid % PERG / JW, gc = tid % JW;
+    const int gm = q + (q >= p ? 1 : 0);
+    gth[x] = q < CP - 1;
+    gwo[x] = (unsigned)(gm * PER + gr * JW + gc);
+    gvo[x] = (gm * JW + gc) * NB + gr;
   }
   const long long N = (long long)T * U;
   float snr = 0.f, sdr = 0.f;  // owners: their row's sensory sums at the current step
@@ -4172,13 +4201,14 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
   auto finish = [&](bool publish) {
     const int t = pt, u = pu;
     const float vold = vs[c * NB + bo];
-    const float den = CG + (pnq.y + sdr) + k.eps;
+    float den = CG + (pnq.y + sdr) + k.eps;
+    if (NF && nanrow[pn & 1][bo] != 0) den = __builtin_nanf("");
     const float num = C * vold + GL + (pnq.x + snr);
     const float rden = __builtin_amdgcn_rcpf(den);
     const float vnew = c < H ? num * rden : 0.f;
     if (publish) {
       const unsigned tag = (unsigned)(pn + 1);
-      xch_put(xbase + (long long)(tag & 1) * CP * PER + p * PER + bo * kClW + o, vnew, tag);
+      xch_put(xbase + (long long)(tag & 1) * CP * PER + p * PER + bo * JW + o, vnew, tag);
     }
     if (k.vsave != nullptr && live) {
       const long long e = (pn * B + b0 + bo) * Hp + c;
@@ -4186,6 +4216,7 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
       k.densave[e] = rden;
     }
     vs[c * NB + bo] = vnew;
+    if (NF && vnew != vnew) nanrow[(pn + 1) & 1][bo] = 1;
     vlast = vnew;
     if (u == U - 1) {
       if (live && c < H) k.out[((long long)(b0 + bo) * T + t) * H + c] = vnew;
@@ -4214,9 +4245,11 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
       const int gg = 1 - g;
       const long long gtag = g == 1 ? n + 1 : n;
       const bool need = g == 1 ? n + 1 < N : n > 0;
-      unsigned long long* gw = xbase + (long long)(gtag & 1) * CP * PER + gm * PER +
-                               (gg * HB + gr) * kClW + gc;
-      unsigned long long w = 0;
+      unsigned long long* gslot =
+          xbase + (long long)(gtag & 1) * CP * PER + gg * HB * JW;
+      unsigned long long w[XW];
+#pragma unroll
+      for (int x = 0; x < XW; ++x) w[x] = 0;
       float na[HB], qa[HB];
 #pragma unroll
       for (int b = 0; b < HB; ++b) na[b] = qa[b] = 0.f;
@@ -4226,7 +4259,11 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
       asm volatile("" : "+s"(nsl));
 #pragma unroll
       for (int q = 0; q < RCP / 4; ++q) {
-        if (q == RCP / 8 && need && gth) w = xch_get(gw);
+        if (q == RCP / 8) {
+#pragma unroll
+          for (int x = 0; x < XW; ++x)
+            if (need && gth[x]) w[x] = xch_get(gslot + gwo[x]);
+        }
         if (4 * q < nsl) {
           const int4 of = slot_tab[q * nthr + tid];
           fwd_synapses_cmp<HB>(preg + 4 * q, vs + g * HB, of.x, of.y, na, qa);
@@ -4234,25 +4271,32 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
             fwd_synapses_cmp<HB>(preg + 4 * q + 2, vs + g * HB, of.z, of.w, na, qa);
         }
       }
-      float2* rg = red + g * KS * HB * kClW;
+      float2* rg = red + g * KS * HB * JW;
 #pragma unroll
-      for (int b = 0; b < HB; ++b) rg[(sks * HB + b) * kClW + so] = make_float2(na[b], qa[b]);
+      for (int b = 0; b < HB; ++b) rg[(sks * HB + b) * JW + so] = make_float2(na[b], qa[b]);
       if (k.spin <= 0) {
         gave_up = 1;  // a budget of 0: give up at the first wait, as xch_gather does
-      } else if (need && gth) {
-        const long long t0 = wall_clock64();
-        bool ok = true;
-        while ((unsigned)(w >> 32) != (unsigned)gtag) {
-          if (wall_clock64() - t0 > k.spin) {
-            ok = false;
-            break;
+      } else {
+#pragma unroll
+        for (int x = 0; x < XW; ++x) {
+          if (!need || !gth[x]) continue;
+          const long long t0 = wall_clock64();
+          bool ok = true;
+          while ((unsigned)(w[x] >> 32) != (unsigned)gtag) {
+            if (wall_clock64() - t0 > k.spin) {
+              ok = false;
+              break;
+            }
+            w[x] = xch_get(gslot + gwo[x]);
           }
-          w = xch_get(gw);
+          if (ok) {
+            const float v = __uint_as_float((unsigned)w[x]);
+            vs[gvo[x] + gg * HB] = v;
+            if (NF && v != v) nanrow[gtag & 1][gg * HB + gvo[x] % NB] = 1;
+          } else {
+            gave_up = 1;
+          }
         }
-        if (ok)
-          vs[(gm * kClW + gc) * NB + gg * HB + gr] = __uint_as_float((unsigned)w);
-        else
-          gave_up = 1;
       }
       lds_barrier();
       if (gave_up) {
@@ -4261,7 +4305,14 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
         return;
       }
       if (owner && og == g) {
-        pnq = ks_sum_wide(rg + (bo - g * HB) * kClW + o, HB * kClW, KS);
+        const float2* rb = rg + (bo - g * HB) * JW + o;
+        if constexpr (JW == 32) {  // 32 chunks, eight reads in flight
+          pnq = tree_sum<8>(rb, HB * JW);
+#pragma unroll
+          for (int s = 8; s < 32; s += 8) pnq += tree_sum<8>(rb + s * HB * JW, HB * JW);
+        } else {
+          pnq = ks_sum_wide(rb, HB * JW, KS);
+        }
         pn = n;
         pt = t;
         pu = u;
@@ -4274,6 +4325,194 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
   if (live) {
     if (c < H) k.hfin[(long long)(b0 + bo) * H + c] = vlast;
     if (k.vsave != nullptr) k.vsave[((long long)T * U * B + b0 + bo) * Hp + c] = vlast;
+  }
+}
+
+// Sum of x over LPC consecutive lanes (16 or 32), in every one of them: DPP
+// rotations within the 16-lane rows, then gfx950's row swap. Each step is a
+// butterfly, so both lanes of a pair add the same two values.
+template <int LPC>
+__device__ __forceinline__ float lane_group_sum(float v) {
+  static_assert(LPC == 16 || LPC == 32, "one or two 16-lane rows");
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false));
+  if constexpr (LPC == 32) {
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                    false);
+    v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  }
+  return v;
+}
+
+// Wave-owned register-resident forward, one batch row per cluster of CP
+// workgroups, for batches that leave a cluster to every row. Bound by the
+// latency of an unfold: 16 waves of 64 / LPC columns, LPC consecutive lanes
+// holding one column's compacted synapses (chunk = lane % LPC), up to RCP >=
+// Hp / LPC each in registers with their LDS row offsets packed two per
+// register. A column's sums finish inside its wave, whose lead lane publishes
+// the new state at once; the partners' words go into the other of two LDS
+// state rows, so an unfold has one barrier. Members are as wide as the
+// registers allow (an exchange costs more the more members take part: Hp =
+// 320, 1.9-2.2 us an unfold with 5 members of 64 columns, 2.5 with 10, 3.6
+// with 20). NaN states and waits as in ode_fwd_cl2_kernel.
+template <int LPC, int RCP>
+__global__ __launch_bounds__(1024) void ode_fwd_own_kernel(FwdCK k) {
+  constexpr int NT = 1024, CW = 64 / LPC, JW = NT / LPC, ZG = 4;
+  static_assert(RCP % ZG == 0, "slots come four at a time");
+  extern __shared__ float4 lds4[];
+  __shared__ int gave_up;
+  __shared__ int nanrow[2];  // the state of that unfold parity holds a NaN
+  const int Hp = k.Hp, H = k.H, T = k.T, U = k.U, CP = k.CP, RC = k.RC;
+  float* vs = reinterpret_cast<float*>(lds4);  // [2][Hp], the state by unfold parity
+  const int tid = threadIdx.x, lane = tid & 63;
+  int p, cl;
+  cluster_coords(blockIdx.x, CP, k.xcd_local != 0, p, cl);
+  if (cl >= k.NCL) return;  // grid padded to whole rounds of the XCDs
+  const int b0 = __builtin_amdgcn_readfirstlane(k.R0 + cl);
+  const int ck = lane % LPC;                         // chunk of the column
+  const unsigned c = (unsigned)(p * JW + (tid >> 6) * CW + lane / LPC);
+  const bool lead = ck == 0, col = (int)c < H;
+  unsigned long long* xbase = k.xch + (long long)cl * 2 * Hp;
+  const float C = k.neuron[c], G = k.neuron[Hp + c], L = k.neuron[2 * Hp + c];
+  const float GL = G * L, CG = C + G;
+  const int cnt = k.ccnt[c];
+  const int nslot = wave_max(cnt > ck ? (cnt - 1 - ck) / LPC + 1 : 0);
+  float4 preg[RCP];
+  unsigned ix[RCP / 2];
+#pragma unroll
+  for (int rr = 0; rr < RCP; ++rr) {
+    preg[rr] = make_float4(0.f, 0.f, 0.f, 0.f);
+    unsigned o = 0;
+    if (rr < RC) {
+      const int a = (ck * RC + rr) * Hp + c;
+      preg[rr] = k.cimg[a];
+      o = (unsigned)k.cidx[a] * 4u;
+    }
+    ix[rr >> 1] = (rr & 1) ? (ix[rr >> 1] | (o << 16)) : o;
+  }
+  if (tid == 0) gave_up = nanrow[0] = nanrow[1] = 0;
+  __syncthreads();
+  for (int j = tid; j < Hp; j += NT) {
+    const float s = (k.state0 != nullptr && j < H) ? k.state0[(long long)b0 * H + j] : 0.f;
+    vs[j] = s;
+    if (s != s) nanrow[0] = 1;
+  }
+  // This thread's word of the gather: column gj of a partner.
+  const bool gth = tid < Hp - JW;
+  const int gj = tid + (tid >= p * JW ? JW : 0);
+  // rows of global memory through wave-uniform bases and the lane's column
+  const long long srow = (long long)b0 * T * Hp;
+  float snn = (k.sn + srow)[c], sdn = (k.sd + srow)[c];
+  float snr = 0.f, sdr = 0.f;
+  lds_barrier();
+  float v = vs[c];
+  const long long N = (long long)T * U;
+  int t = 0, u = 0;
+  for (long long n = 0; n < N; ++n) {
+    if (u == 0) {
+      snr = snn;
+      sdr = sdn;
+      if (t + 1 < T) {
+        const long long e = srow + (long long)(t + 1) * Hp;
+        snn = (k.sn + e)[c];
+        sdn = (k.sd + e)[c];
+      }
+    }
+    const char* vr = reinterpret_cast<const char*>(vs + (n & 1) * Hp);
+    const int nanv = nanrow[n & 1];
+    float na = 0.f, qa = 0.f;
+    int nsl = nslot;
+    asm volatile("" : "+s"(nsl));
+    // Slots in groups of ZG, their gates in phases (states, arguments,
+    // exponentials, reciprocals), then the sums.
+#pragma unroll
+    for (int q = 0; q < RCP; q += ZG) {
+      if (q < nsl) {
+        float z[ZG];
+#pragma unroll
+        for (int i = 0; i < ZG; i += 2) {
+          // opaque, or the compiler keeps every unpacked offset across the loop
+          asm volatile("" : "+v"(ix[(q + i) / 2]));
+          z[i] = *reinterpret_cast<const float*>(vr + slot_offset(ix, q + i));
+          z[i + 1] = *reinterpret_cast<const float*>(vr + slot_offset(ix, q + i + 1));
+        }
+#pragma unroll
+        for (int i = 0; i < ZG; ++i)
+          z[i] = fmaf(preg[q + i].x, z[i], preg[q + i].y);
+#pragma unroll
+        for (int i = 0; i < ZG; ++i)
+          z[i] = 1.0f + __builtin_amdgcn_exp2f(z[i]);
+#pragma unroll
+        for (int i = 0; i < ZG; ++i)
+          z[i] = __builtin_amdgcn_rcpf(z[i]);
+#pragma unroll
+        for (int i = 0; i < ZG; ++i) {
+          na = fmaf(z[i], preg[q + i].z, na);
+          qa = fmaf(z[i], preg[q + i].w, qa);
+        }
+      }
+    }
+    na = lane_group_sum<LPC>(na);
+    qa = lane_group_sum<LPC>(qa);
+    float den = CG + (qa + sdr) + k.eps;
+    if (nanv != 0) den = __builtin_nanf("");
+    const float num = C * v + GL + (na + snr);
+    const float rden = __builtin_amdgcn_rcpf(den);
+    const float vnew = col ? num * rden : 0.f;
+    const unsigned tag = (unsigned)(n + 1);
+    unsigned long long* slot = xbase + (long long)(tag & 1) * Hp;
+    if (lead) {
+      // Publish first: the partners wait on it, the other stores on nothing.
+      if (n + 1 < N) xch_put(slot + c, vnew, tag);
+      vs[(tag & 1) * Hp + c] = vnew;
+      if (vnew != vnew) nanrow[tag & 1] = 1;
+      if (k.vsave != nullptr) {
+        const long long e = (n * k.B + b0) * Hp;
+        (k.vsave + e)[c] = v;
+        (k.densave + e)[c] = rden;
+      }
+      if (u == U - 1 && col) (k.out + ((long long)b0 * T + t) * H)[c] = vnew;
+    }
+    v = vnew;
+    if (n + 1 < N) {
+      if (k.spin <= 0) {
+        gave_up = 1;  // a budget of 0: give up at the first wait
+      } else if (gth) {
+        unsigned long long w = xch_get(slot + gj);
+        const long long t0 = wall_clock64();
+        bool ok = true;
+        while ((unsigned)(w >> 32) != tag) {
+          if (wall_clock64() - t0 > k.spin) {
+            ok = false;
+            break;
+          }
+          w = xch_get(slot + gj);
+        }
+        if (ok) {
+          const float s = __uint_as_float((unsigned)w);
+          vs[(tag & 1) * Hp + gj] = s;
+          if (s != s) nanrow[tag & 1] = 1;
+        } else {
+          gave_up = 1;
+        }
+      }
+      lds_barrier();
+      if (gave_up) {
+        if (lead && col) k.hfin[(long long)b0 * H + c] = __builtin_nanf("");
+        if (tid == 0) __hip_atomic_store(k.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return;
+      }
+    }
+    if (++u == U) {
+      u = 0;
+      ++t;
+    }
+  }
+  if (lead) {
+    if (col) k.hfin[(long long)b0 * H + c] = v;
+    if (k.vsave != nullptr) k.vsave[(N * k.B + b0) * Hp + c] = v;
   }
 }
 
@@ -5321,6 +5560,33 @@ hipError_t fwd_cl_by_rcp(const Plan& p, const FwdCK& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Register-resident clusters: every member of a cluster on one XCD (its
+// exchange words and saved rows then go through one L2). cluster_coords deals
+// whole rounds of eight clusters, so the grid is padded to them; the plan
+// keeps the padded grid at one workgroup per CU, and the members past the
+// last cluster leave at once.
+template <int NB>
+hipError_t launch_reg_fwd(const Plan& p, FwdCK a, hipStream_t s) {
+  const RegCluster& g = p.rf;
+  const int rounds = (g.NCL + 7) / 8 * 8;
+  a.xcd_local = g.xcd ? 1 : 0;
+  const dim3 grid((g.xcd ? rounds : g.NCL) * g.CP), block(1024);
+  const size_t lds = (size_t)reg_fwd_lds(g, p.Hp);
+  if constexpr (NB == 1) {
+    if (g.RC > (g.JW == 64 ? 20 : 16)) return hipErrorInvalidConfiguration;
+    if (g.JW == 64 && g.RC <= 16)
+      LTC_LAUNCH((ode_fwd_own_kernel<16, 16>), grid, block, lds, s, a);
+    else if (g.JW == 64)
+      LTC_LAUNCH((ode_fwd_own_kernel<16, 20>), grid, block, lds, s, a);
+    else
+      LTC_LAUNCH((ode_fwd_own_kernel<32, 16>), grid, block, lds, s, a);
+  } else if (g.JW == 64)
+    LTC_LAUNCH((ode_fwd_cl2_kernel<(NB > 1 ? NB : 2), 64, true>), grid, block, lds, s, a);
+  else
+    LTC_LAUNCH((ode_fwd_cl2_kernel<(NB > 1 ? NB : 2), 32, true>), grid, block, lds, s, a);
+  return hipGetLastError();
+}
+
 template <int NB>
 hipError_t bwd_cl_by_rcp(const Plan& p, const BwdCK& a, hipStream_t s) {
   const dim3 grid(p.NCLB * p.CPB), block(p.JWB * p.KSB);
@@ -5475,12 +5741,32 @@ hipError_t launch_sens_fwd_ln(const Plan& p, const float* x, Strides3 xs, const 
 hipError_t launch_ode_fwd(const Plan& p, const Prepped& pp, const float* sn, const float* sd,
                           const float* state0, float eps, float* out, float* hfin,
                           float* vsave, float* densave, const ClusterBuf& cb, hipStream_t s) {
+  if (p.rf.CP > 0) {
+    if (pp.cF == nullptr || pp.cFi == nullptr || pp.cFn == nullptr) return hipErrorInvalidValue;
+    const RegCluster& g = p.rf;
+    FwdCK a{pp.recF, pp.neuron, sn, sd, state0, out, hfin, vsave, densave, cb.xch, cb.status,
+            cb.spin, p.B, p.T, p.H, p.Hp, p.U, g.KS, g.RC, g.CP, 0, eps,
+            pp.cF, pp.cFi, pp.cFn, 0, g.NCL};
+    for (int l = 0; l < g.L; ++l) {
+      hipError_t e = clear_cluster(p, cb, false, s, l == 0);
+      if (e != hipSuccess) return e;
+      a.R0 = l * g.NCL * g.NB;
+      switch (g.NB) {
+        case 8: e = launch_reg_fwd<8>(p, a, s); break;
+        case 4: e = launch_reg_fwd<4>(p, a, s); break;
+        case 2: e = launch_reg_fwd<2>(p, a, s); break;
+        default: e = launch_reg_fwd<1>(p, a, s); break;
+      }
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   if (p.CP > 0) {
     // Register-resident operands (RC = 16) read no image from L2 in the loop.
     const int xl = (p.RC == 16 && p.NCL % 8 == 0) ? 1 : 0;
     FwdCK a{pp.recF, pp.neuron, sn, sd, state0, out, hfin, vsave, densave, cb.xch, cb.status,
             cb.spin, p.B, p.T, p.H, p.Hp, p.U, p.KS, p.RC, p.CP, xl, eps,
-            pp.cF, pp.cFi, pp.cFn, 0};
+            pp.cF, pp.cFi, pp.cFn, 0, p.NCL};
     if (cmp_fwd(p) && (pp.cF == nullptr || pp.cFi == nullptr || pp.cFn == nullptr))
       return hipErrorInvalidValue;
     // One launch per NCL * NB rows (more than one only at Hp > 1024); the

@@ -62,6 +62,17 @@ enum KernelId : int {
   K_COUNT
 };
 
+// Cluster geometry of the register-resident compacted kernels beyond the
+// Hp = 256 forms: CP members of JW columns (CP * JW = Hp) advance NB rows in
+// two groups; each thread holds up to RC = Hp / KS compacted synapses. L
+// launches per call, each taking the next NCL * NB rows.
+// With xcd set every member of a cluster runs on one XCD (the grid, padded to
+// whole rounds of eight clusters, still holds at most one workgroup per CU).
+struct RegCluster {
+  int CP, JW, KS, RC, NB, NCL, L;
+  bool xcd;
+};
+
 // Shapes and launch choices shared by every kernel of one call.
 struct Plan {
   int B, T, D, H, U;
@@ -85,6 +96,9 @@ struct Plan {
   // form covers a row) as many as take the B rows NCL * NB at a time, each
   // launch holding at most one workgroup per CU. Forward and chain.
   int LCH, LCHB;
+  // Register-resident clusters (plan_reg_clusters): when rf.CP > 0 the forward
+  // ODE kernel runs in this geometry instead of the one above.
+  RegCluster rf;
 };
 
 // Derived, zero-padded parameter images built once per call by the prep kernel.
@@ -308,7 +322,13 @@ inline void fill_add(FillList& fl, float* dst, const float* src, long long n) {
 // device) and clears it when `clear` is set. Returns the HIP status.
 hipError_t device_fault(int* value, bool clear);
 // Exchange words of one cluster launch (forward / chain).
-inline long long cluster_words(const Plan& p) { return 2LL * p.NCL * p.CP * p.NB * 64; }
+inline long long cluster_words(const Plan& p) {
+  if (p.rf.CP > 0) return 2LL * p.rf.NCL * p.rf.CP * p.rf.NB * p.rf.JW;
+  return 2LL * p.NCL * p.CP * p.NB * 64;
+}
+// Whether the call's ODE kernel runs as clusters (its waits can give up).
+inline bool fwd_clusters(const Plan& p) { return p.rf.CP > 0 || p.CP > 0; }
+inline bool bwd_clusters(const Plan& p) { return p.CP > 0; }
 inline long long cluster_words_bwd(const Plan& p) {
   return 2LL * p.NCLB * p.CPB * p.NBB * p.JWB;
 }
@@ -406,7 +426,11 @@ inline long long row_bwd_words(const Plan& p) {
     return (long long)p.B * p.T * p.U * 256 + (row128_sens_fused(p) ? (long long)p.B * p.T * 384 : 0) + 1;
   return 0;
 }
+// Whether the forward launch reads a compacted image: the plan's own forms
+// (cmp_fwd) or the register-resident clusters.
+inline bool fwd_image_cmp(const Plan& p) { return p.rf.CP > 0 || cmp_fwd(p); }
 inline int cmp_chunks_fwd(const Plan& p) {
+  if (p.rf.CP > 0) return p.rf.KS;
   return (row_kernels(p) || row_wave128_fwd(p)) ? 4 : (p.CP > 0 ? kCmpChunks : p.KS);
 }
 inline int cmp_chunks_bwd(const Plan& p) {
@@ -425,6 +449,14 @@ inline long long cluster_bwd_lds(const Plan& p) {
 inline long long cluster_fwd_lds(const Plan& p) {
   return (long long)p.NB * p.Hp * 4 + (long long)p.KS * p.NB * 64 * 8 +
          (cmp_fwd(p) ? cmp_index_lds(64 * p.KS) + balance_lds(64 * p.KS) : 0);
+}
+// The same for a register-resident cluster of 1024-thread members (the two-group
+// form's layout): state rows [Hp][NB], the partials of both groups, the slot
+// table and the balanced lane order's scratch.
+inline long long reg_fwd_lds(const RegCluster& g, int hp) {
+  if (g.NB == 1) return 2LL * hp * 4;  // the wave-owned form: the state by parity
+  return (long long)g.NB * hp * 4 + (long long)g.KS * g.NB * g.JW * 8 + cmp_index_lds(1024) +
+         balance_lds(1024);
 }
 // Dynamic LDS of the single-workgroup forward: state rows and the KS
 // partials, or the wave-owned single-row forward's state and staged sums.

@@ -75,7 +75,9 @@ class CApi:
                    "NRC", "ode_workgroups", "fuse", "KSB", "RCB",
                    "threads_bwd", "CP", "NCL", "CPB", "NBB", "ode_workgroups_bwd",
                    "cmp_fwd", "cmp_bwd", "module_sens_in_prep", "module_row_bwd_fused",
-                   "module_row128_rec_fused", "launches_fwd", "launches_bwd", "sens_full_list")
+                   "module_row128_rec_fused", "launches_fwd", "launches_bwd", "sens_full_list",
+                   "reg_fwd_members", "reg_fwd_cols", "reg_fwd_rows", "reg_fwd_launches",
+                   "reg_fwd_lds")
 
     def __init__(self, path: str = LIB_PATH):
         self.path = path

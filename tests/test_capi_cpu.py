@@ -453,3 +453,23 @@ def test_two_group_cluster_plans(capi, B, nb, nbb):
     lds = ((nbb + 2) * Hp * 8 + ks * nbb * jw * 4 + pf * nbb * Hp + thr * 16 * 4
            + thr * 4 + (thr // 64) * 17 * 4)
     assert p["lds_bwd"] == lds <= 159 * 1024
+
+
+@pytest.mark.parametrize("H", [129, 192, 256, 257, 320, 384, 448, 500, 512])
+@pytest.mark.parametrize("B", [1, 16, 64, 65, 128, 257, 700, 4096])
+def test_register_resident_cluster_plan(capi, B, H):
+    """Forward members of 64 or 32 columns whose 1024 threads hold every synapse
+    of a dense column (20 or 16 each), one workgroup per CU and launch."""
+    p = capi.plan(B, 4, 8, H, 6)
+    if p["reg_fwd_members"] == 0:
+        assert p["Hp"] == 256 and p["cmp_fwd"] == 1  # the plan's own form holds them
+        return
+    cp, jw, nb, L = (p["reg_fwd_members"], p["reg_fwd_cols"], p["reg_fwd_rows"],
+                     p["reg_fwd_launches"])
+    assert cp * jw == p["Hp"] and nb in (1, 2, 4, 8)
+    per_thread = p["Hp"] * jw // 1024
+    assert per_thread <= (20 if nb == 1 and jw == 64 else 16)
+    slots = 256 // cp
+    assert L == -(-B // (nb * min(slots, -(-B // nb))))
+    assert L == 1 or nb == 8
+    assert p["reg_fwd_lds"] <= 159 * 1024

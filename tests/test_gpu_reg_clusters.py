@@ -1,0 +1,103 @@
+"""The register-resident clusters (128 < H <= 512) against the float64 oracle.
+
+Every rows-per-cluster form at the edges of its range: one row per cluster up
+to the last batch that leaves every row a cluster, the two-group form from the
+next row on, and the batches that take a second launch; padded and full
+columns; recurrent masks with a column that has no synapse, one that has every
+synapse and one whose only synapse sits in the last row. The kernels skip
+zero-weight synapses but treat a NaN state as the dense kernels they replaced:
+it makes every neuron of its row NaN from the next unfold on.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import ltc_cuda
+from _gpu_common import (_native, boundary, gpu_forward, oracle_forward)  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+# (B, T, D, H, rows per cluster, launches)
+FWD = [
+    (1, 3, 8, 129, 1, 1),     # Hp = 192: 64-column members, padded columns
+    (85, 2, 5, 192, 1, 1),    # 85 clusters of 3 members: the last batch of one row each
+    (86, 2, 5, 192, 2, 1),
+    (683, 1, 5, 192, 8, 2),   # 680 rows per launch: three rows in the second
+    (260, 1, 4, 256, 8, 1),   # Hp = 256 beyond four rows per cluster
+    (515, 1, 4, 250, 8, 2),
+    (3, 2, 70, 257, 1, 1),    # Hp = 320: 20 synapses per lane at full density
+    (52, 2, 5, 320, 4, 1),    # 10 members of 32 columns, 13 clusters
+    (21, 2, 5, 380, 1, 1),
+    (22, 2, 5, 384, 2, 1),
+    (5, 2, 5, 448, 1, 1),
+    (16, 1, 5, 512, 1, 1),
+    (17, 1, 5, 500, 2, 1),
+    (129, 1, 5, 512, 8, 2),
+]
+
+
+def _edge_masks(args):
+    """Recurrent columns with no synapse, every synapse, and one in the last row."""
+    w_pos, w_erev = args[2], args[3]
+    H = w_pos.shape[0]
+    w_pos[:, 0] = 0.0
+    w_erev[:, 0] = 0.0
+    g = torch.Generator().manual_seed(H)
+    w_pos[:, H // 2] = torch.rand(H, generator=g) + 0.1
+    w_erev[:, H // 2] = w_pos[:, H // 2]
+    w_pos[:, H - 1] = 0.0
+    w_erev[:, H - 1] = 0.0
+    w_pos[H - 1, H - 1] = 0.7
+    w_erev[H - 1, H - 1] = -0.7
+    return args
+
+
+@pytest.mark.parametrize("shape", FWD, ids=lambda s: "B%dT%dD%dH%d" % s[:4])
+def test_forward_matches_oracle(shape):
+    B, T, D, H, rows, launches = shape
+    p = ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)
+    assert p["reg_fwd_members"] * p["reg_fwd_cols"] == p["Hp"], p
+    assert (p["reg_fwd_rows"], p["reg_fwd_launches"]) == (rows, launches), p
+    args = _edge_masks(boundary(B, T, D, H, seed=B + H))
+    _, (out, h) = gpu_forward(args)
+    ref_out, ref_h = oracle_forward(args)
+    err = (out.cpu().double() - ref_out).abs().max().item()
+    print(f"{shape}: max|out err| = {err:.2e}", flush=True)
+    # float32 sums of up to H terms over T*U unfolds of a contraction: errors of
+    # single roundings (6e-8 of values below 1), not the 1e-3 bar
+    assert err <= 5e-6
+    assert (h.cpu().double() - ref_h).abs().max().item() <= 5e-6
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 8, 129), (90, 1, 4, 192), (2, 1, 4, 300),
+                                   (60, 1, 4, 320), (300, 1, 4, 256)],
+                         ids=lambda s: "B%dT%dD%dH%d" % s)
+@pytest.mark.parametrize("U", [1, 2, 3])
+def test_nan_state_reaches_its_whole_row(shape, U):
+    """After one unfold every neuron of the row is NaN, and no other row is."""
+    B, T, D, H = shape
+    assert ltc_cuda._cuda_module.capi.plan(B, T, D, H, U)["reg_fwd_members"] > 0
+    args = boundary(B, T, D, H, seed=13)
+    h0 = args[1].clone()
+    h0[B - 1, 7] = float("nan")
+    _, res = gpu_forward([args[0], h0] + args[2:], U=U)
+    out = res[0].cpu()
+    assert torch.isnan(out[B - 1]).all()
+    assert torch.isfinite(out[:B - 1]).all()
+
+
+def test_nan_sum_spreads_one_unfold_later():
+    """A NaN input at a neuron's sensory synapse makes that neuron NaN in the
+    first unfold and its whole row NaN in the second, as a dense kernel does."""
+    B, T, D, H = 60, 1, 6, 320
+    args = boundary(B, T, D, H, seed=3)
+    x = args[0].clone()
+    x[2, 0, 1] = float("nan")
+    connected = args[9][1] != 0  # sensory_w_pos[d = 1]
+    _, res = gpu_forward([x] + args[1:], U=1)
+    assert torch.equal(torch.isnan(res[0].cpu()[2, 0]), connected)
+    _, res = gpu_forward([x] + args[1:], U=2)
+    assert torch.isnan(res[0].cpu()[2, 0]).all()
+    assert torch.isfinite(res[0].cpu()[3]).all()
