@@ -96,7 +96,8 @@ void plan_fused_chain(ltc::Plan& p, int ncu) {
     if (ltc::cluster_chain_lds(nb, p.Hp, 16, 32, p.Hp == 256) +
             (p.Hp == 256 ? ltc::cmp_index_lds(512) + ltc::cmp_pad_lds(p.Hp) + ltc::balance_lds(512)
                          : 0) >
-        chain_lds_limit())
+            chain_lds_limit() ||
+        ltc::partial_tile_lds(p.Hp) > chain_lds_limit())
       continue;
     p.CPB = cp;
     p.JWB = 32;
@@ -196,6 +197,15 @@ bool plan_cluster(ltc::Plan& p, int ncu) {
   return false;
 }
 
+// Clusters of a launch, launches of a call, and whether each cluster's members
+// fit one XCD.
+void reg_cluster_counts(ltc::RegCluster& g, int B, int ncu) {
+  const int need = (B + g.NB - 1) / g.NB, slots = ncu / g.CP;
+  g.NCL = need < slots ? need : slots;
+  g.L = (B + g.NCL * g.NB - 1) / (g.NCL * g.NB);
+  g.xcd = (g.NCL + 7) / 8 * 8 * g.CP <= ncu;
+}
+
 // Register-resident clusters for 128 < Hp <= 512 where the plan above has no
 // register-resident form: a forward member's 1024 threads hold the compacted
 // synapses of 64 columns or 32, at most 20 or 16 each at any mask density, so
@@ -203,9 +213,7 @@ bool plan_cluster(ltc::Plan& p, int ncu) {
 // row per cluster (ode_fwd_own_kernel); else the fewest rows per cluster of
 // the two-group form that take the batch in one launch of at most one
 // workgroup per CU, and past eight rows as many launches as the batch needs.
-void plan_reg_clusters(ltc::Plan& p, int ncu) {
-  p.rf = ltc::RegCluster{};
-  if (p.Hp <= 128 || p.Hp > 512 || p.B < 1) return;
+void plan_reg_forward(ltc::Plan& p, int ncu) {
   if (p.CP > 0 && p.Hp == 256 && p.KS == 16 && p.RC == 16) return;
   ltc::RegCluster g{};
   auto geom = [&](int jw) {
@@ -225,11 +233,37 @@ void plan_reg_clusters(ltc::Plan& p, int ncu) {
       if ((p.B + nb - 1) / nb <= slots) break;
     }
   }
-  const int need = (p.B + g.NB - 1) / g.NB, slots = ncu / g.CP;
-  g.NCL = need < slots ? need : slots;
-  g.L = (p.B + g.NCL * g.NB - 1) / (g.NCL * g.NB);
-  g.xcd = (g.NCL + 7) / 8 * 8 * g.CP <= ncu;
+  reg_cluster_counts(g, p.B, ncu);
   if (ltc::reg_fwd_lds(g, p.Hp) <= chain_lds_limit()) p.rf = g;
+}
+
+// The chain: members of 32 columns and 512 threads, whose registers hold the
+// operands and the four gradient sums of up to reg_chain_slots synapses per
+// thread: every one of a dense column up to Hp = 256, beyond that the synapses
+// of half-dense masks. The column counts are known on the device
+// only, so at those sizes a second launch, of the kernel that streams dense
+// operands, follows and exactly one of the two runs past its first check.
+void plan_reg_chain(ltc::Plan& p, int ncu) {
+  if (p.CP > 0 && p.Hp == 256 && p.FUSE) return;
+  ltc::RegCluster g{};
+  g.JW = 32;
+  g.CP = p.Hp / 32;
+  g.KS = 16;
+  g.RC = p.Hp / 16;
+  const int slots = ncu / g.CP;
+  if (slots < 1) return;
+  for (int nb : {2, 4, 8}) {
+    g.NB = nb;
+    if ((p.B + nb - 1) / nb <= slots) break;
+  }
+  reg_cluster_counts(g, p.B, ncu);
+  if (ltc::reg_bwd_lds(g, p.Hp) <= chain_lds_limit()) p.rb = g;
+}
+
+void plan_reg_clusters(ltc::Plan& p, int ncu) {
+  if (p.Hp <= 128 || p.Hp > 512 || p.B < 1) return;
+  plan_reg_forward(p, ncu);
+  plan_reg_chain(p, ncu);
 }
 
 // ---------------------------------------------------------------------------
@@ -418,10 +452,11 @@ void carve_cmp(const ltc::Plan& p, Carver& c, ltc::Prepped& pp, bool fwd, bool b
     pp.cFi = c.take<int>(n);
     pp.cFn = c.take<int>(p.Hp);
   }
-  if (bwd && ltc::cmp_bwd(p)) {
+  if (bwd && ltc::bwd_image_cmp(p)) {
     pp.cB = c.take<float4>(n);
     pp.cBi = c.take<int>(n);
     pp.cBn = c.take<int>(p.Hp);
+    pp.cBmark = p.rb.CP > 0 && p.rb.RC > ltc::reg_chain_slots(p.rb.RC) ? 1 : 0;
   }
 }
 
@@ -492,13 +527,13 @@ BwdWs carve_bwd(const ltc::Plan& p, Carver& c, bool images = true) {
     // the forward's as well: the per-step backward recomputes a forward unfold
     carve_cmp(p, c, w.pp, true, true);
   }
-  w.absave = p.FUSE ? nullptr : c.take<float2>(p.N * p.Hp);
+  w.absave = ltc::chain_fused(p) ? nullptr : c.take<float2>(p.N * p.Hp);
   w.dsn = c.take<float>((long long)p.B * p.T * p.Hp);
   w.dsd = c.take<float>((long long)p.B * p.T * p.Hp);
   w.npart = c.take<float>((long long)p.B * 3 * p.Hp);
   // recurrent partials: NCH chunks, or one per batch row (Hp = 128 chain with
   // recurrent-gradient companions)
-  const long long nch = ltc::row128_rec_fused(p) && p.B > p.NCH ? p.B : p.NCH;
+  const long long nch = ltc::row128_rec_fused(p) && p.B > p.NCH ? p.B : ltc::rec_parts(p);
   w.rpart = c.take<float>(nch * 4 * p.Hp * p.Hp);
   // sensory partials: NRC row chunks, or one per batch row (fused row backward,
   // or the sensory companions of the Hp = 128 chain)
@@ -959,7 +994,7 @@ int ltc_full_backward(const float* x, long long sxb, long long sxt, long long sx
                                w.dsn, w.dsd, w.npart, grad_state, w.rpart, w.cb, s);
   });
   if (e != hipSuccess) return hip_fail("ODE backward launch", e);
-  if (!p.FUSE) {
+  if (!ltc::chain_fused(p)) {
     e = timed(ltc::K_REC_GRAD, s,
               [&] { return ltc::launch_rec_grad(p, w.pp, vsave, w.absave, w.rpart, s); });
     if (e != hipSuccess) return hip_fail("recurrent gradient launch", e);
@@ -968,11 +1003,13 @@ int ltc_full_backward(const float* x, long long sxb, long long sxt, long long sx
     return ltc::launch_sens_bwd(p, x, xs, w.pp, w.dsn, w.dsd, w.spart, w.dxpart, s);
   });
   if (e != hipSuccess) return hip_fail("sensory backward launch", e);
+  ltc::Plan pf = p;
+  pf.NCH = ltc::rec_parts(p);
   e = timed(ltc::K_FINALIZE, s, [&] {
-    return ltc::launch_finalize(p, rp, w.rpart, w.spart, w.dxpart, w.npart, w.ps, go, s);
+    return ltc::launch_finalize(pf, rp, w.rpart, w.spart, w.dxpart, w.npart, w.ps, go, s);
   });
   if (e != hipSuccess) return hip_fail("finalize launch", e);
-  if (p.CP > 0) {
+  if (ltc::bwd_clusters(p)) {
     ltc::FillList fl = poison_list(w.cb);
     ltc::fill_add(fl, grad_x, nullptr, (long long)B * T * D);
     ltc::fill_add(fl, grad_state, nullptr, (long long)B * H);
@@ -1220,6 +1257,7 @@ int ltc_module_backward(const float* x, long long sxb, long long sxt, long long 
   // At Hp = 128 (one row per workgroup) the recurrent-gradient sums are formed
   // inside the chain launch by companion workgroups: one partial per row.
   ltc::Plan pf = p;
+  pf.NCH = ltc::rec_parts(p);
   const int* status = nullptr;
   const bool sens_comp = ltc::row128_sens_fused(p);
   if (ltc::row128_rec_fused(p)) {
@@ -1244,7 +1282,7 @@ int ltc_module_backward(const float* x, long long sxb, long long sxt, long long 
                                  s);
     });
     if (e != hipSuccess) return hip_fail("ODE backward launch", e);
-    if (!p.FUSE) {
+    if (!ltc::chain_fused(p)) {
       e = timed(ltc::K_REC_GRAD, s,
                 [&] { return ltc::launch_rec_grad(p, wb.pp, vsave, wb.absave, wb.rpart, s); });
       if (e != hipSuccess) return hip_fail("recurrent gradient launch", e);
@@ -1267,7 +1305,7 @@ int ltc_module_backward(const float* x, long long sxb, long long sxt, long long 
                                      status, grad_state);
   });
   if (e != hipSuccess) return hip_fail("finalize launch", e);
-  if (p.CP > 0) {
+  if (ltc::bwd_clusters(p)) {
     ltc::FillList fl = poison_list(wb.cb);
     ltc::fill_add(fl, grad_x, nullptr, (long long)B * T * D);
     ltc::fill_add(fl, grad_state, nullptr, (long long)B * H);
@@ -1607,7 +1645,7 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
                                w.b.dsn, w.b.dsd, w.b.npart, grad_v, w.b.rpart, w.b.cb, s);
   });
   if (e != hipSuccess) return hip_fail("ODE backward launch", e);
-  if (!p.FUSE) {
+  if (!ltc::chain_fused(p)) {
     e = timed(ltc::K_REC_GRAD, s,
               [&] { return ltc::launch_rec_grad(p, w.b.pp, vsave, w.b.absave, w.b.rpart, s); });
     if (e != hipSuccess) return hip_fail("recurrent gradient launch", e);
@@ -1615,8 +1653,10 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
   e = ltc::launch_copy_rows(w.b.dsn, p.Hp, grad_w_num_sensory, H, B, H, s);
   if (e == hipSuccess) e = ltc::launch_copy_rows(w.b.dsd, p.Hp, grad_w_den_sensory, H, B, H, s);
   if (e != hipSuccess) return hip_fail("copy launch", e);
+  ltc::Plan pf = p;
+  pf.NCH = ltc::rec_parts(p);
   e = timed(ltc::K_FINALIZE, s, [&] {
-    return ltc::launch_finalize(p, rp, w.b.rpart, nullptr, nullptr, w.b.npart, w.b.ps, go, s,
+    return ltc::launch_finalize(pf, rp, w.b.rpart, nullptr, nullptr, w.b.npart, w.b.ps, go, s,
                                 ltc::kFinRec);
   });
   if (e != hipSuccess) return hip_fail("finalize launch", e);
@@ -1655,7 +1695,8 @@ int ltc_launch_plan(int B, int T, int D, int H, int ode_unfolds, long long* out,
       ltc::cmp_fwd(p) ? 1 : 0, ltc::cmp_bwd(p) ? 1 : 0, ltc::prep_sens_fused(p) ? 1 : 0,
       ltc::row_bwd_fused(p) ? 1 : 0, ltc::row128_rec_fused(p) ? 1 : 0, p.LCH, p.LCHB,
       ltc::sens_full_list(p) ? 1 : 0,
-      p.rf.CP, p.rf.JW, p.rf.NB, p.rf.L, p.rf.CP > 0 ? ltc::reg_fwd_lds(p.rf, p.Hp) : 0};
+      p.rf.CP, p.rf.JW, p.rf.NB, p.rf.L, p.rf.CP > 0 ? ltc::reg_fwd_lds(p.rf, p.Hp) : 0,
+      p.rb.CP, p.rb.NB, p.rb.L, p.rb.CP > 0 ? ltc::reg_bwd_lds(p.rb, p.Hp) : 0};
   const int m = n < LTC_PLAN_FIELDS ? n : LTC_PLAN_FIELDS;
   for (int i = 0; i < m; ++i) out[i] = v[i];
   return m;

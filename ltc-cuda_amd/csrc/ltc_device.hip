@@ -26,6 +26,7 @@
 //    (t,k,b) by separate kernels into partial buffers that a finalize kernel
 //    sums in a fixed order. No atomics anywhere, so every result is bitwise
 //    reproducible run to run.
+#include <algorithm>
 #include <type_traits>
 
 #include "ltc_internal.h"
@@ -125,43 +126,47 @@ __device__ __forceinline__ int wave_max(int v) {
 // to thread r puts lanes of nearly equal counts in each wave, so waves run
 // few padding slots, and the long waves and the short ones spread over the
 // SIMDs (the workgroups of a CU place each wave index on different SIMDs).
-// n: the count of this thread's own lane (lane = tid); returns the lane this
-// thread evaluates. Every thread of the workgroup must call it (it holds two
-// workgroup barriers). LDS: perm [nthr] ints, wcnt [nthr / 64][17] ints.
+// n: the count of this thread's own lane (lane = tid), at most MAXC; returns
+// the lane this thread evaluates. Every thread of the workgroup must call it
+// (it holds workgroup barriers). LDS: perm [nthr] ints, wcnt [nthr / 64][MAXC
+// + 1] ints.
+template <int MAXC = 16>
 __device__ __forceinline__ int balanced_lane(int n, int tid, int nthr, int* perm, int* wcnt) {
+  constexpr int NC = MAXC + 1;
+  static_assert(NC <= 64, "one count per lane of wave 0");
   const int lane = tid & 63, w = tid >> 6, nw = nthr >> 6;
   const unsigned long long below = (1ull << lane) - 1ull;
   int local = 0;
 #pragma unroll
-  for (int v = 0; v <= 16; ++v) {
+  for (int v = 0; v <= MAXC; ++v) {
     const unsigned long long m = __ballot(n == v);
     if (n == v) local = __popcll(m & below);
-    if (lane == 0) wcnt[w * 17 + v] = __popcll(m);
+    if (lane == 0) wcnt[w * NC + v] = __popcll(m);
   }
   __syncthreads();
-  // wave 0, lane v < 17: start[w][v] = (lanes of any wave with count > v)
+  // wave 0, lane v <= MAXC: start[w][v] = (lanes of any wave with count > v)
   // + (lanes of count v in waves before w), written over wcnt in place
   if (w == 0) {
     int tot = 0;
-    if (lane <= 16)
-      for (int x = 0; x < nw; ++x) tot += wcnt[x * 17 + lane];
+    if (lane <= MAXC)
+      for (int x = 0; x < nw; ++x) tot += wcnt[x * NC + lane];
     int above = 0;
 #pragma unroll
-    for (int v = 1; v <= 16; ++v) {
+    for (int v = 1; v <= MAXC; ++v) {
       const int t = __shfl(tot, v, 64);
       if (v > lane) above += t;
     }
-    if (lane <= 16) {
+    if (lane <= MAXC) {
       int run = above;
       for (int x = 0; x < nw; ++x) {
-        const int c = wcnt[x * 17 + lane];
-        wcnt[x * 17 + lane] = run;
+        const int c = wcnt[x * NC + lane];
+        wcnt[x * NC + lane] = run;
         run += c;
       }
     }
   }
   __syncthreads();
-  perm[wcnt[w * 17 + n] + local] = tid;
+  perm[wcnt[w * NC + n] + local] = tid;
   __syncthreads();
   return perm[tid];
 }
@@ -313,6 +318,12 @@ __device__ __forceinline__ void compact_column(int col, int nrows, int stride, i
   if (lane == 0) ccnt[col] = n;
 }
 
+// Marks chain column `col` when any lane of its wave met an entry whose w cannot
+// be factored out of wE (Prepped::cBmark).
+__device__ __forceinline__ void mark_irregular(const Prepped& pp, int col, int lane, bool bad) {
+  if (pp.cBmark != 0 && __any(bad) && lane == 0) pp.cBn[col] |= kChainIrregular;
+}
+
 // Compacted columns a prep launch builds: Hp forward columns when cF is set,
 // then Hp chain columns when the chain image is built and cB is set.
 __host__ __device__ inline int cmp_columns(const Prepped& pp, int Hp, int Dp, bool fwd, bool bwd,
@@ -385,6 +396,7 @@ __global__ __launch_bounds__(256) void prep_kernel(RawParams rp, Prepped pp, int
         // the parameter gradients); the unfused one (bwd == 2, folded
         // operands) only those that add to dL/dv.
         const int i = col;
+        bool bad = false;
         compact_column(i, Hp, Hp, nchb, lane, pp.cB, pp.cBi, pp.cBn, [&](int j, float4& v, bool& act) {
           if (i < H && j < H) {
             operand(i, j, v);
@@ -393,9 +405,11 @@ __global__ __launch_bounds__(256) void prep_kernel(RawParams rp, Prepped pp, int
               act = v.z != 0.f || v.w != 0.f;
             } else {
               act = true;
+              bad |= !(fabsf(v.z) <= 1e18f * fabsf(v.w));
             }
           }
         });
+        mark_irregular(pp, i, lane, bad);
         return;
       }
       col -= Hp;
@@ -3407,6 +3421,7 @@ __global__ __launch_bounds__(FS ? kPrepSensThreads : 256) void prep_leaf_kernel(
         // nonzero; the unfused one (recb == 2, folded operands) those that
         // add to dL/dv.
         const int i = col;
+        bool bad = false;
         compact_column(i, Hp, Hp, nchb, lane, pp.cB, pp.cBi, pp.cBn, [&](int j, float4& v, bool& act) {
           if (i < H && j < H) {
             if (recb == 2) {
@@ -3416,9 +3431,11 @@ __global__ __launch_bounds__(FS ? kPrepSensThreads : 256) void prep_leaf_kernel(
             } else if (lp.mask[(long long)i * H + j] != 0.f) {
               operand(i, j, v);
               act = true;
+              bad |= !(fabsf(v.z) <= 1e18f * fabsf(v.w));
             }
           }
         });
+        mark_irregular(pp, i, lane, bad);
         return;
       }
       col -= Hp;
@@ -4530,16 +4547,21 @@ __device__ __forceinline__ void chain_fused_stream(__amdgpu_buffer_rsrc_t rs, in
                                                    int srow0, int jrow0, int Hp,
                                                    const float2* ab, const float* vi,
                                                    float* acc, float4 (&gacc)[RCS]) {
-  static_assert(RCS % 8 == 0, "rows come in groups of eight");
+  static_assert(RCS % 4 == 0, "rows come in groups of four");
   const int rowb = Hp * 16;
   const int sb = srow0 * rowb;
+  // opaque: with 24 or 28 rows the compiler forms every alpha/beta address
+  // once, outside the unfold loop, and spills them
+  if constexpr (RCS < 32) asm volatile("" : "+v"(jrow0));
   float4 pa[4], pb[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) pa[q] = image_load(rs, lane_bytes, sb + q * rowb);
 #pragma unroll
   for (int rr = 0; rr < RCS; rr += 8) {
+    if (rr + 4 < RCS) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) pb[q] = image_load(rs, lane_bytes, sb + (rr + 4 + q) * rowb);
+      for (int q = 0; q < 4; ++q) pb[q] = image_load(rs, lane_bytes, sb + (rr + 4 + q) * rowb);
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -4553,11 +4575,13 @@ __device__ __forceinline__ void chain_fused_stream(__amdgpu_buffer_rsrc_t rs, in
       for (int q = 0; q < 4; ++q) pa[q] = image_load(rs, lane_bytes, sb + (rr + 8 + q) * rowb);
     }
     __builtin_amdgcn_sched_barrier(0);
+    if (rr + 4 < RCS) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      bwd_synapse<NB, true>(pb[q], ab, Hp, jrow0 + rr + 4 + q, vi, acc, gacc[rr + 4 + q]);
-      asm volatile("" : "+v"(gacc[rr + 4 + q].x), "+v"(gacc[rr + 4 + q].y),
-                   "+v"(gacc[rr + 4 + q].z), "+v"(gacc[rr + 4 + q].w));
+      for (int q = 0; q < 4; ++q) {
+        bwd_synapse<NB, true>(pb[q], ab, Hp, jrow0 + rr + 4 + q, vi, acc, gacc[rr + 4 + q]);
+        asm volatile("" : "+v"(gacc[rr + 4 + q].x), "+v"(gacc[rr + 4 + q].y),
+                     "+v"(gacc[rr + 4 + q].z), "+v"(gacc[rr + 4 + q].w));
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -4582,6 +4606,19 @@ __device__ __forceinline__ void rows_to_lds_fixed(const float* slice, int b0, in
           static_cast<const void*>(slice + (long long)b0 * HP + 4LL * u),
           (__attribute__((address_space(3))) void*)(dst + 4 * u0), 16, 0, 0);
   }
+}
+
+// rows_to_lds_fixed for a runtime row length.
+template <int NB, int NT>
+__device__ __forceinline__ void rows_to_lds(const float* slice, int b0, int B, int Hp, float* dst,
+                                            int tid) {
+  const int units = min(NB, B - b0) * (Hp / 4), lane = tid & 63;
+  const float* src = slice + (long long)b0 * Hp;
+  for (int u0 = tid & ~63; u0 < units; u0 += NT)
+    if (u0 + lane < units)
+      __builtin_amdgcn_global_load_lds(
+          static_cast<const void*>(src + 4 * (u0 + lane)),
+          (__attribute__((address_space(3))) void*)(dst + 4 * u0), 16, 0, 0);
 }
 
 // Waits for this wave's outstanding global loads (and stores), including
@@ -4612,12 +4649,25 @@ struct BwdCK {
   const int* cidx;
   const int* ccnt;
   int R0;  // first batch row of this launch (launches take NCL * NB rows each)
+  int NCL; // register-resident clusters: clusters of this launch (the grid may hold more)
+  // Fused streamed kernel behind the register-resident one: it runs only when
+  // a column count exceeds maxcnt (too many synapses for the registers, or
+  // kChainIrregular), and the other only when none does. 0: always run.
+  int maxcnt;
 };
+
+// Whether every column of the chain image has at most `maxcnt` entries: the
+// same answer in every workgroup. Holds a workgroup barrier.
+__device__ __forceinline__ bool chain_counts_fit(const int* ccnt, int Hp, int maxcnt) {
+  int over = 0;
+  for (int j = threadIdx.x; j < Hp; j += blockDim.x) over |= ccnt[j] > maxcnt;
+  return __syncthreads_or(over) == 0;
+}
 
 // One compacted chain synapse for every row of the tile: alpha/beta of its
 // row come from the [Hp][NB] float2 layout at byte offset `off` (one 8*NB
 // byte read per lane), the rest as bwd_synapse<NB, true>.
-template <int NB>
+template <int NB, bool ZP = false>
 __device__ __forceinline__ void bwd_synapse_cmp(const float4 p, const float2* ab, int off,
                                                 const float* vi, float* acc, float4& gacc) {
   float2 c[NB];
@@ -4634,14 +4684,15 @@ __device__ __forceinline__ void bwd_synapse_cmp(const float4 p, const float2* ab
   }
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const float a = gate(fmaf(p.x, vi[b], p.y));
+    const float zp = fmaf(p.x, vi[b], p.y);
+    const float a = gate(zp);
     const float a2 = fmaf(-a, a, a);
     const float dl = fmaf(c[b].x, p.z, c[b].y * p.w) * a2;
     acc[b] = fmaf(dl, p.x, acc[b]);
     gacc.x = fmaf(c[b].x, a, gacc.x);
     gacc.y = fmaf(c[b].y, a, gacc.y);
     gacc.z += dl;
-    gacc.w = fmaf(dl, vi[b], gacc.w);
+    gacc.w = fmaf(dl, ZP ? zp : vi[b], gacc.w);
   }
 }
 
@@ -4650,7 +4701,7 @@ __device__ __forceinline__ void bwd_synapse_cmp(const float4 p, const float2* ab
 // and the last two gradient sums (of dL/darg and dL/darg v_i) come out
 // divided by w, which the caller multiplies back once at the end. One
 // multiply per synapse-row fewer.
-template <int NB>
+template <int NB, bool ZP = false>
 __device__ __forceinline__ void bwd_synapse_cmpe(const float4 p, const float2* ab, int off,
                                                  const float* vi, float* acc, float4& gacc) {
   float2 c[NB];
@@ -4667,15 +4718,50 @@ __device__ __forceinline__ void bwd_synapse_cmpe(const float4 p, const float2* a
   }
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const float a = gate(fmaf(p.x, vi[b], p.y));
+    const float zp = fmaf(p.x, vi[b], p.y);
+    const float a = gate(zp);
     const float a2 = fmaf(-a, a, a);
     const float dl = fmaf(c[b].x, p.z, c[b].y) * a2;
     acc[b] = fmaf(dl, p.w, acc[b]);
     gacc.x = fmaf(c[b].x, a, gacc.x);
     gacc.y = fmaf(c[b].y, a, gacc.y);
     gacc.z += dl;
-    gacc.w = fmaf(dl, vi[b], gacc.w);
+    gacc.w = fmaf(dl, ZP ? zp : vi[b], gacc.w);
   }
+}
+
+// Recurrent-gradient partial planes of a fused chain member with 32 columns
+// and 512 threads, through LDS: put(tile, stride, plane) places this thread's
+// sums of a plane at tile[column * stride + j], and each of the member's 32
+// rows i leaves as one coalesced run of Hp floats, to out[plane][i][j]. Written
+// from the registers, each 4-byte piece goes to a cache line of its own: the
+// 64 MB of an Hp = 512 chain took about 80 us a launch, 20 us this way. Places
+// without a synapse carry whatever LDS held; nothing reads them. `add`: a
+// later launch of the call adds to the cluster's partial.
+template <class Put>
+__device__ __forceinline__ void store_partials32(float* tile, float* out, int Hp, bool add,
+                                                 Put&& put) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, stride = Hp + 1;
+  const long long HH = (long long)Hp * Hp;
+  for (int pl = 0; pl < 4; ++pl) {
+    __syncthreads();  // the LDS is free (chain buffers or the previous plane)
+    put(tile, stride, pl);
+    __syncthreads();
+    for (int i = w; i < 32; i += 8) {
+      float* row = out + pl * HH + (long long)i * Hp;
+      for (int j = lane; j < Hp; j += 64) {
+        float v = tile[i * stride + j];
+        if (add) v += row[j];
+        row[j] = v;
+      }
+    }
+  }
+}
+
+// Whether alpha or beta is infinite or NaN.
+__device__ __forceinline__ bool not_finite(float al, float be) {
+  const float z = fmaf(al, 0.f, be * 0.f);
+  return z != z;
 }
 
 // Cluster chain: member p forms dL/dv_i for its JW columns i (reduction over
@@ -4740,6 +4826,9 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
   const long long BHp = (long long)B * Hp;
   const float C = k.neuron[c];
   if (T == 0) return;
+  if constexpr (RCS > 0) {
+    if (k.maxcnt > 0 && (cl >= k.NCL || chain_counts_fit(k.ccnt, Hp, k.maxcnt))) return;
+  }
 
   float4 preg[RCP > 0 ? RCP : 1];
   int nmine = 0, nslot = 0;  // CMP: this lane's entries, slots the wave runs
@@ -5024,32 +5113,29 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
   }
   if constexpr (FUSE) {
     // This cluster's share of the recurrent parameter gradients for synapses
-    // (i = sc, j = r0 + rr), layout [cluster][4][i][j] as rec_grad_kernel's.
-    const long long HH = (long long)Hp * Hp;
-    if constexpr (CMP) {
-      float* out = k.rpart + (long long)(k.R0 / NB + cl) * 4 * HH + (long long)sc * Hp;
+    // (i = sc, j = r0 + rr or the slot's row), layout [cluster][4][i][j] as
+    // rec_grad_kernel's.
+    store_partials32(reinterpret_cast<float*>(lds4),
+                     k.rpart + (long long)cl * 4 * Hp * Hp + (long long)p * JW * Hp, Hp, k.R0 > 0,
+                     [&](float* tile, int stride, int pl) {
 #pragma unroll
-      for (int rr = 0; rr < NACC; ++rr) {
-        if (rr < nmine) {
-          const int j = k.cidx[(long long)(sks * RCP + rr) * Hp + sc];
-          out[j] = gacc[rr].x;
-          out[HH + j] = gacc[rr].y;
-          out[2 * HH + j] = gacc[rr].z;
-          out[3 * HH + j] = gacc[rr].w;
-        }
-      }
-    } else {
-      float* out = k.rpart + (long long)(k.R0 / NB + cl) * 4 * HH + (long long)c * Hp + r0;
-#pragma unroll
-      for (int rr = 0; rr < NACC; ++rr) {
-        out[rr] = gacc[rr].x;
-        out[HH + rr] = gacc[rr].y;
-        out[2 * HH + rr] = gacc[rr].z;
-        out[3 * HH + rr] = gacc[rr].w;
-      }
-    }
+                       for (int rr = 0; rr < NACC; ++rr) {
+                         const float4 v = gacc[rr];
+                         const float x = pl == 0 ? v.x : (pl == 1 ? v.y : (pl == 2 ? v.z : v.w));
+                         if constexpr (CMP) {
+                           if (rr < nmine)
+                             tile[so * stride + k.cidx[(long long)(sks * RCP + rr) * Hp + sc]] = x;
+                         } else {
+                           tile[o * stride + r0 + rr] = x;
+                         }
+                       }
+                     });
   }
 }
+
+// Smallest |x| = |sigma| log2(e) of a register-resident chain slot: below it
+// every gate of bounded states is 1/2 to the last bit.
+constexpr float kMinSlope = 1e-20f;
 
 // The compacted fused cluster chain (register-resident operands, Hp = 256,
 // 32-column members of 512 threads) with its NB >= 2 rows in two groups of
@@ -5066,15 +5152,34 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
 // sums of each synapse take the rows in the same order as the one-group
 // kernel; a slot's operands are (x, y, E, w x), w factored out of dL/darg
 // (bwd_synapse_cmpe), and its alpha/beta row offset stays in a register.
-template <int NB>
+//
+// REG: the register-resident clusters beyond that form: 12 or 16 slots cover
+// Hp = 192 or 256, 16 slots Hp = 320 ... 448 and 20 Hp = 512 while no column
+// has more than 16 * RCP entries (half-dense masks; a second launch, of
+// ode_bwd_cl_kernel, covers the rest). FACT factors w out as above, which needs w != 0 wherever wE is
+// (kChainIrregular otherwise); without it the operands stay (x, y, wE, w).
+// REG's fourth sum is that of dl * zp, zp = x v + y the gate's argument, not of
+// dl * v: the sigma gradient is sum dl (v - mu), and summed as sum dl v less mu
+// sum dl its terms cancel only after hundreds of rounded additions (B64 T32
+// H192: error against float64 2.2e-6, 1.3e-6 with rec_grad_kernel's shorter
+// sums). A slope x below kMinSlope is raised to it so that sum dl v can be
+// taken out again at the end.
+// REG keeps the dense kernels' treatment of a non-finite alpha or beta: the
+// synapses left out have weight zero, and zero times it is NaN, so dL/dv of
+// every neuron of that row that has such a synapse becomes NaN. A row flag by
+// unfold parity carries it, as the forward's does a NaN state.
+template <int NB, int RCP = 16, bool FACT = true, bool REG = false>
 __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   static_assert(NB == 2 || NB == 4 || NB == 8, "two groups of rows");
-  constexpr int JW = 32, RCP = 16, HB = NB / 2, PER = NB * JW, PERG = HB * JW;
+  constexpr int JW = 32, HB = NB / 2, PER = NB * JW, PERG = HB * JW;
   constexpr int ABS = NB + 2;  // padded alpha/beta rows, as in ode_bwd_cl_kernel
-  constexpr int HPC = 16 * RCP;  // Hp = 256
-  constexpr int XW = 2;          // gather words per thread and group: (CP-1)*PERG <= 2*512
+  constexpr int HPC = 16 * RCP;  // Hp, without REG
+  // gather words per thread and group: (CP - 1) * PERG <= XW * 512
+  // (CP = 8 without REG, at most 8 without FACT, 16 with both)
+  constexpr int XW = !REG ? 2 : (FACT ? NB / 2 : (NB == 8 ? 2 : 1));
   extern __shared__ float4 lds4[];
   __shared__ int gave_up;
+  __shared__ int badrow[2][NB];  // REG: alpha/beta of that unfold parity not finite
   const int Hp = k.Hp, H = k.H, KS = k.KS, B = k.B, T = k.T, U = k.U, CP = k.CP;
   float2* ab = reinterpret_cast<float2*>(lds4);                  // [Hp][ABS]
   float* red = reinterpret_cast<float*>(ab + ABS * Hp);         // [2][KS][HB][JW]
@@ -5083,6 +5188,9 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   // [4][threads] int4 of the compacted kernels' slot table, of which this
   // kernel only uses the space after it (balanced_lane's scratch)
   int4* slot_tab = reinterpret_cast<int4*>(pv + 3 * NB * Hp);
+  // REG: balanced_lane's scratch directly
+  int* perm = REG ? reinterpret_cast<int*>(slot_tab)
+                  : reinterpret_cast<int*>(slot_tab + (RCP / 4) * 512);
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int ks = tid / JW, o = tid % JW;
   int p, cl;
@@ -5096,6 +5204,14 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   const long long BHp = (long long)B * Hp;
   const float C = k.neuron[c];
   if (T == 0) return;
+  if constexpr (REG) {
+    if (cl >= k.NCL) return;  // grid padded to whole rounds of the XCDs
+    if (k.maxcnt > 0 && !chain_counts_fit(k.ccnt, Hp, k.maxcnt)) return;
+    if (tid < 2 * NB) badrow[tid / NB][tid % NB] = 0;  // before balanced_lane's barriers
+  }
+  const int RC = REG ? k.RC : RCP;  // slots of a chunk
+  if ((CP - 1) * PERG > XW * 512) return;  // the host's geometry keeps to it
+  const int cntc = REG ? k.ccnt[c] : 0;
   auto pden_at = [&](long long m) { return pden + (m & 1) * NB * Hp; };
   auto pv_at = [&](long long m) { return pv + (m % 3) * NB * Hp; };
   // v slot r (an unfold index mod 3, kept by the loop instead of divided)
@@ -5104,12 +5220,17 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   auto mod3_prev = [](int r) { return r == 0 ? 2 : r - 1; };
 
   float4 preg[RCP];
-  int ix[RCP];  // slot row offsets, in registers
+  // The gathered words' LDS operands are read when the words are requested,
+  // except where 20 slots leave no registers for them (spilled to scratch
+  // memory, their reloads wait for every load in flight).
+  constexpr bool EARLY = RCP <= 16;
+  // slot row offsets, in registers; with 20 slots two to a register
+  constexpr bool PACK = RCP > 16;
+  unsigned ix[PACK ? RCP / 2 : RCP];
   int nmine, nslot, sks, so;
   {
-    int* perm = reinterpret_cast<int*>(slot_tab + (RCP / 4) * nthr);
     const int cnt0 = k.ccnt[c];
-    const int lane_id = balanced_lane(cnt0 > ks ? (cnt0 - 1 - ks) / kCmpChunks + 1 : 0, tid,
+    const int lane_id = balanced_lane<RCP <= 16 ? 16 : RCP>(cnt0 > ks ? (cnt0 - 1 - ks) / kCmpChunks + 1 : 0, tid,
                                       nthr, perm, perm + nthr);
     sks = lane_id / JW;
     so = lane_id - sks * JW;
@@ -5118,12 +5239,20 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
     nslot = wave_max(nmine);
 #pragma unroll
     for (int rr = 0; rr < RCP; ++rr) {
-      const long long a = (long long)(sks * RCP + rr) * Hp + p * JW + so;
+      const long long a = (long long)(sks * RC + rr) * Hp + p * JW + so;
+      const float4 q = k.cimg[a];
       // image operands (x, y, w E, w) -> (x, y, E, w x); an entry with
       // w = 0 (a padding slot) contributes nothing either way
-      const float4 q = k.cimg[a];
-      preg[rr] = make_float4(q.x, q.y, q.w != 0.f ? q.z / q.w : 0.f, q.w * q.x);
-      ix[rr] = k.cidx[a] * ABS * 8;
+      preg[rr] = FACT ? make_float4(q.x, q.y, q.w != 0.f ? q.z / q.w : 0.f, q.w * q.x) : q;
+      if (REG && fabsf(q.x) < kMinSlope) {  // the gate is 1/2 either way
+        preg[rr].x = kMinSlope;
+        preg[rr].y = 0.f;
+      }
+      const unsigned of = (unsigned)(k.cidx[a] * ABS * 8);
+      if constexpr (PACK)
+        ix[rr >> 1] = (rr & 1) ? (ix[rr >> 1] | (of << 16)) : of;
+      else
+        ix[rr] = of;
     }
   }
   const int sc = p * JW + so;
@@ -5134,7 +5263,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
 
   // Owner state, as in ode_bwd_cl_kernel.
   float g = 0.f, gdir = 0.f, accA = 0.f, accB = 0.f, pC = 0.f, pGv = 0.f, pA = 0.f;
-  auto own_ab = [&](float den, float vk, float vk1) {
+  auto own_ab = [&](float den, float vk, float vk1, int par) {
     float al = 0.f, be = 0.f;
     gdir = 0.f;
     if (live && c < H) {
@@ -5148,13 +5277,20 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
       gdir = al * C;
     }
     ab[c * ABS + bo] = make_float2(al, be);
+    if (REG && not_finite(al, be)) badrow[par][bo] = 1;
   };
   auto gout_at = [&](int b, int t, int col) {
     return k.gout[(long long)(b0 + b) * k.gs.b + (long long)t * k.gs.t + (long long)col * k.gs.c];
   };
+  auto stage = [&](const float* slice, float* dst) {
+    if constexpr (REG)
+      rows_to_lds<NB, 512>(slice, b0, B, Hp, dst, tid);
+    else
+      rows_to_lds_fixed<NB, HPC, 512>(slice, b0, B, dst, tid);
+  };
   auto prefetch = [&](long long m) {  // 1/den of unfold m, v of slot m
-    rows_to_lds_fixed<NB, HPC, 512>(k.densave + m * BHp, b0, B, pden_at(m), tid);
-    rows_to_lds_fixed<NB, HPC, 512>(k.vsave + m * BHp, b0, B, pv_at(m), tid);
+    stage(k.densave + m * BHp, pden_at(m));
+    stage(k.vsave + m * BHp, pv_at(m));
   };
 
   const long long n_last = (long long)T * U - 1;
@@ -5171,7 +5307,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
       vk = k.vsave[e];
       vk1 = k.vsave[e + BHp];
     }
-    own_ab(den, vk, vk1);
+    own_ab(den, vk, vk1, (int)(n_last & 1));
   }
   for (int e = tid; e < (CP - 1) * PER; e += nthr) {
     const int q = e / PER, r = e - q * PER, b = r / JW;
@@ -5186,20 +5322,24 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
       be = -gg * k.vsave[ee + BHp] * rden;
     }
     ab[col * ABS + b] = make_float2(al, be);
+    if (REG && not_finite(al, be)) badrow[n_last & 1][b] = 1;
   }
   // The prefetched rows the first three phases read: v of slots n_last and
   // n_last - 1, 1/den of unfold n_last - 1.
-  rows_to_lds_fixed<NB, HPC, 512>(k.vsave + n_last * BHp, b0, B, pv_at(n_last), tid);
+  stage(k.vsave + n_last * BHp, pv_at(n_last));
   if (n_last > 0) prefetch(n_last - 1);
   wait_vm();
   lds_barrier();
 
-  // This thread's gather words (x < XW): partner member, row of the group, column.
-  int gm[XW], gr[XW], gcl[XW];
+  // This thread's gather words (x < XW): partner member, row of the group,
+  // column. 512 is a multiple of PERG, so they share row and column in it.
+  static_assert(512 % PERG == 0, "a thread's words share row and column");
+  const int gr = tid % PERG / JW, gc = tid % JW;
+  int gcl[XW];
   bool gth[XW];
 #pragma unroll
   for (int x = 0; x < XW; ++x) {
-    const int e = tid + x * nthr;
+    const int e = tid + x * 512;
     // With two or more rows per group the word count (CP - 1) * PERG is a
     // multiple of 64, so a wave gathers all its words or none: a scalar
     // branch instead of a lane mask.
@@ -5207,11 +5347,13 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
       gth[x] = __builtin_amdgcn_readfirstlane(e) < (CP - 1) * PERG;
     else
       gth[x] = e < (CP - 1) * PERG;
-    const int q = e / PERG, r = e - q * PERG;
-    gm[x] = q + (q >= p ? 1 : 0);
-    gr[x] = r / JW;
-    gcl[x] = gm[x] * JW + (r - gr[x] * JW);
+    const int q = e / PERG;
+    gcl[x] = (q + (q >= p ? 1 : 0)) * JW + gc;
   }
+  // word of column gcl[x] in a slot, for the rows of group g
+  auto gword = [&](int x, int g) {
+    return (unsigned)((gcl[x] - gc) * NB + (g * HB + gr) * JW + gc);
+  };
   bool pend = false;  // owners: their group's finish is due
   long long pn = 0;
   int pn3 = 0, pt = 0, pu = 0;  // pn mod 3, its step and unfold within the step
@@ -5229,6 +5371,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
         const float* rg = red + og * KS * HB * JW;
         const float s = ks_sum_wide(rg + (bo - og * HB) * JW + o, HB * JW, KS);
         g = c < H ? fmaf(kNegLn2, s, gdir) : 0.f;
+        if (REG && badrow[pn & 1][bo] != 0 && cntc < H && c < H) g = __builtin_nanf("");
         if (pn > 0) {
           g += gnext;
           const unsigned tag = (unsigned)pn;
@@ -5277,18 +5420,18 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
 #pragma unroll
           for (int x = 0; x < XW; ++x)
             if (need && gth[x])
-              w[x] = xch_get(gslot + gm[x] * PER + (gg * HB + gr[x]) * JW + (gcl[x] - gm[x] * JW));
+              w[x] = xch_get(gslot + gword(x, gg));
 #pragma unroll
           for (int x = 0; x < XW; ++x) {
             rdn[x] = rvk[x] = 0.f;
-            if (need && gth[x]) {
-              const int e = (gg * HB + gr[x]) * Hp + gcl[x];
+            if (EARLY && need && gth[x]) {
+              const int e = (gg * HB + gr) * Hp + gcl[x];
               rdn[x] = dn[e];
               rvk[x] = vk1[e];
             }
           }
           // the owners' own entry likewise
-          if (own_next) {
+          if (EARLY && own_next) {
             odn = pden_at(pn - 1)[bo * Hp + c];
             ovk = pv_slot(mod3_prev(pn3))[bo * Hp + c];
             ovk1 = pv_slot(pn3)[bo * Hp + c];
@@ -5297,20 +5440,31 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
           // word loads
           if (gi == 1 && n >= 2) {
             // 1/den of unfold n - 2, v of slot n - 2 (n - 2 = n + 1 mod 3)
-            rows_to_lds_fixed<NB, HPC, 512>(k.densave + (n - 2) * BHp, b0, B, pden_at(n), tid);
-            rows_to_lds_fixed<NB, HPC, 512>(k.vsave + (n - 2) * BHp, b0, B,
-                                            pv_slot(mod3_next(n3)), tid);
+            stage(k.densave + (n - 2) * BHp, pden_at(n));
+            stage(k.vsave + (n - 2) * BHp, pv_slot(mod3_next(n3)));
           }
         }
         if (4 * q < nsl) {
-          const int off[4] = {ix[4 * q], ix[4 * q + 1], ix[4 * q + 2], ix[4 * q + 3]};
+          int off[4];
+          if constexpr (PACK) {
+            // opaque, or the compiler keeps every unpacked offset across the loop
+            asm volatile("" : "+v"(ix[2 * q]), "+v"(ix[2 * q + 1]));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) off[i] = slot_offset(ix, 4 * q + i);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) off[i] = (int)ix[4 * q + i];
+          }
 #pragma unroll
           for (int h = 0; h < 4; h += 2) {
             if (4 * q + h < nsl) {
 #pragma unroll
               for (int i = 0; i < 2; ++i) {
                 const int rr = 4 * q + h + i;
-                bwd_synapse_cmpe<HB>(preg[rr], ab + gi * HB, off[h + i], cvi, acc, gacc[rr]);
+                if constexpr (FACT)
+                  bwd_synapse_cmpe<HB, REG>(preg[rr], ab + gi * HB, off[h + i], cvi, acc, gacc[rr]);
+                else
+                  bwd_synapse_cmp<HB, REG>(preg[rr], ab + gi * HB, off[h + i], cvi, acc, gacc[rr]);
                 asm volatile("" : "+v"(gacc[rr].x), "+v"(gacc[rr].y), "+v"(gacc[rr].z),
                              "+v"(gacc[rr].w));
               }
@@ -5332,8 +5486,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
           if (!gth[x]) continue;
           const long long t0 = wall_clock64();
           bool ok = true;
-          unsigned long long* wa =
-              gslot + gm[x] * PER + (gg * HB + gr[x]) * JW + (gcl[x] - gm[x] * JW);
+          unsigned long long* wa = gslot + gword(x, gg);
           while ((unsigned)(w[x] >> 32) != (unsigned)gtag) {
             if (wall_clock64() - t0 > k.spin) {
               ok = false;
@@ -5345,18 +5498,27 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
             gave_up = 1;
             continue;
           }
-          const int b = gg * HB + gr[x], col = gcl[x];
+          const int b = gg * HB + gr, col = gcl[x];
           float al = 0.f, be = 0.f;
           if (b0 + b < B && col < H) {
             const float gv = __uint_as_float((unsigned)w[x]);
-            const float rden = rdn[x];
+            const int e = b * Hp + col;
+            const float rden = EARLY ? rdn[x] : dn[e];
             al = gv * rden;
-            be = -gv * rvk[x] * rden;
+            be = -gv * (EARLY ? rvk[x] : vk1[e]) * rden;
           }
           ab[col * ABS + b] = make_float2(al, be);
+          if (REG && not_finite(al, be)) badrow[am & 1][b] = 1;
         }
       }
-      if (own_next) own_ab(odn, ovk, ovk1);
+      if (own_next) {
+        if constexpr (!EARLY) {
+          odn = pden_at(pn - 1)[bo * Hp + c];
+          ovk = pv_slot(mod3_prev(pn3))[bo * Hp + c];
+          ovk1 = pv_slot(pn3)[bo * Hp + c];
+        }
+        own_ab(odn, ovk, ovk1, (int)((pn - 1) & 1));
+      }
       // the prefetch issued in the previous (group 1) phase, visible to
       // every wave after this barrier
       if (gi == 0) wait_vm();
@@ -5386,6 +5548,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
     const float* rg = red + og * KS * HB * JW;
     const float s = ks_sum_wide(rg + (bo - og * HB) * JW + o, HB * JW, KS);
     g = c < H ? fmaf(kNegLn2, s, gdir) : 0.f;
+    if (REG && badrow[0][bo] != 0 && cntc < H && c < H) g = __builtin_nanf("");
     if (live) {
       const long long e = ((long long)(b0 + bo) * T) * Hp + c;
       k.dsn[e] = accA;
@@ -5400,26 +5563,44 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
     np[2 * Hp] = pA;
   }
   // This cluster's share of the recurrent parameter gradients, layout
-  // [cluster][4][i][j], as ode_bwd_cl_kernel writes it.
-  const long long HH = (long long)Hp * Hp;
-  float* out = k.rpart + (long long)(k.R0 / NB + cl) * 4 * HH + (long long)sc * Hp;
-  // The image entries are indexed again from a copy of sks the compiler
-  // cannot match with the preload's, so that it does not keep the preload's
-  // addresses (or every w) live across the loop.
+  // [cluster][4][i][j], as ode_bwd_cl_kernel writes it. The image entries are
+  // indexed again from a copy of sks the compiler cannot match with the
+  // preload's, so that it does not keep the preload's addresses (or every w)
+  // live across the loop.
   int sks_end = sks;
   asm volatile("" : "+v"(sks_end));
+  // REG: sum dl*v from sum dl*(x*v + y)
+  if constexpr (REG) {
 #pragma unroll
-  for (int rr = 0; rr < RCP; ++rr) {
-    if (rr < nmine) {
-      const long long a = (long long)(sks_end * RCP + rr) * Hp + sc;
-      const int j = k.cidx[a];
-      const float w = k.cimg[a].w;  // the factor the last two sums left out
-      out[j] = gacc[rr].x;
-      out[HH + j] = gacc[rr].y;
-      out[2 * HH + j] = gacc[rr].z * w;
-      out[3 * HH + j] = gacc[rr].w * w;
+    for (int rr = 0; rr < RCP; ++rr)
+      gacc[rr].w = (gacc[rr].w - preg[rr].y * gacc[rr].z) / preg[rr].x;
+  }
+  if constexpr (FACT) {
+#pragma unroll
+    for (int rr = 0; rr < RCP; ++rr) {
+      if (rr < nmine) {
+        const float w = k.cimg[(long long)(sks_end * RC + rr) * Hp + sc].w;
+        gacc[rr].z *= w;  // the factor the last two sums left out
+        gacc[rr].w *= w;
+      }
     }
   }
+  int jx[RCP];
+#pragma unroll
+  for (int rr = 0; rr < RCP; ++rr)
+    jx[rr] = rr < nmine ? k.cidx[(long long)(sks_end * RC + rr) * Hp + sc] : 0;
+  store_partials32(reinterpret_cast<float*>(lds4),
+                   k.rpart + (long long)cl * 4 * Hp * Hp + (long long)p * JW * Hp, Hp,
+                   REG && k.R0 > 0, [&](float* tile, int stride, int pl) {
+#pragma unroll
+                     for (int rr = 0; rr < RCP; ++rr) {
+                       if (rr < nmine) {
+                         const float4 v = gacc[rr];
+                         tile[so * stride + jx[rr]] =
+                             pl == 0 ? v.x : (pl == 1 ? v.y : (pl == 2 ? v.z : v.w));
+                       }
+                     }
+                   });
 }
 
 // Clears the cluster exchange words (tag 0) and the status word before a
@@ -5588,6 +5769,40 @@ hipError_t launch_reg_fwd(const Plan& p, FwdCK a, hipStream_t s) {
 }
 
 template <int NB>
+hipError_t launch_reg_bwd(const Plan& p, BwdCK a, hipStream_t s) {
+  const RegCluster& g = p.rb;
+  const int rounds = (g.NCL + 7) / 8 * 8;
+  const dim3 grid((g.xcd ? rounds : g.NCL) * g.CP), block(512);
+  const size_t lds = (size_t)reg_bwd_lds(g, p.Hp);
+  if (g.RC == 12 || g.RC == 16) {
+    if (g.RC == 12)
+      LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 12, false, true>), grid, block, lds, s, a);
+    else
+      LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 16, false, true>), grid, block, lds, s, a);
+    return hipGetLastError();
+  }
+  // The kernel over at most reg_chain_slots synapses a thread, then the one
+  // that streams them all: one of the two leaves at its first check.
+  a.maxcnt = 16 * reg_chain_slots(g.RC);
+  if (reg_chain_slots(g.RC) == 16)
+    LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 16, true, true>), grid, block, lds, s, a);
+  else
+    LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 20, true, true>), grid, block, lds, s, a);
+  const size_t lds2 = (size_t)std::max(cluster_chain_lds(NB, p.Hp, 16, 32, false),
+                                       partial_tile_lds(p.Hp));
+  a.xcd_local = 0;  // streamed operands: members spread over the XCDs (cluster_coords)
+  const dim3 grid2(g.NCL * g.CP);
+  switch (g.RC) {
+    case 20: LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, 20>), grid2, block, lds2, s, a); break;
+    case 24: LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, 24>), grid2, block, lds2, s, a); break;
+    case 28: LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, 28>), grid2, block, lds2, s, a); break;
+    case 32: LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, 32>), grid2, block, lds2, s, a); break;
+    default: return hipErrorInvalidConfiguration;
+  }
+  return hipGetLastError();
+}
+
+template <int NB>
 hipError_t bwd_cl_by_rcp(const Plan& p, const BwdCK& a, hipStream_t s) {
   const dim3 grid(p.NCLB * p.CPB), block(p.JWB * p.KSB);
   const size_t lds = bwd_cl_lds_bytes(p);
@@ -5623,7 +5838,7 @@ hipError_t launch_prep(const Plan& p, const RawParams& rp, const Prepped& pp, bo
   const bool rec = (segs & kPrepRec) != 0;
   const int ncmp = (cmp_columns(pp, p.Hp, p.Dp, rec, rec && bwd, (segs & kPrepSens) != 0) + 3) / 4;
   LTC_LAUNCH(prep_kernel, dim3((unsigned)(nflat + ncmp)), dim3(256), 0, s, rp, pp, p.H,
-                     p.D, p.Hp, p.Dp, bwd ? (p.FUSE ? 1 : 2) : 0, segs, nflat, cmp_chunks_fwd(p),
+                     p.D, p.Hp, p.Dp, bwd ? (chain_fused(p) ? 1 : 2) : 0, segs, nflat, cmp_chunks_fwd(p),
                      cmp_chunks_bwd(p));
   return hipGetLastError();
 }
@@ -5803,13 +6018,32 @@ hipError_t launch_ode_bwd(const Plan& p, const Prepped& pp, const float* vsave,
                           const float* ghfin, float2* absave, float* dsn, float* dsd,
                           float* npart, float* gstate, float* rpart, const ClusterBuf& cb,
                           hipStream_t s) {
+  if (p.rb.CP > 0) {
+    if (pp.cB == nullptr || pp.cBi == nullptr || pp.cBn == nullptr) return hipErrorInvalidValue;
+    const RegCluster& g = p.rb;
+    BwdCK a{pp.recB, pp.neuron, vsave, densave, gout, gs, ghfin, absave, dsn, dsd, npart,
+            gstate, rpart, cb.xch, cb.status, cb.spin, p.B, p.T, p.H, p.Hp, p.U, g.KS, g.RC,
+            g.CP, g.xcd ? 1 : 0, pp.cB, pp.cBi, pp.cBn, 0, g.NCL, 0};
+    for (int l = 0; l < g.L; ++l) {
+      hipError_t e = clear_cluster(p, cb, true, s, l == 0);
+      if (e != hipSuccess) return e;
+      a.R0 = l * g.NCL * g.NB;
+      switch (g.NB) {
+        case 8: e = launch_reg_bwd<8>(p, a, s); break;
+        case 4: e = launch_reg_bwd<4>(p, a, s); break;
+        default: e = launch_reg_bwd<2>(p, a, s); break;
+      }
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   if (p.CP > 0) {
     // The register-resident fused chain (Hp = 256) prefetches saved rows that
     // every member of a cluster reads: keep a cluster on one XCD.
     const int xl = (chain_prefetches(p) && p.NCLB % 8 == 0) ? 1 : 0;
     BwdCK a{pp.recB, pp.neuron, vsave, densave, gout, gs, ghfin, absave, dsn, dsd, npart,
             gstate, rpart, cb.xch, cb.status, cb.spin, p.B, p.T, p.H, p.Hp, p.U, p.KSB, p.RCB,
-            p.CPB, xl, pp.cB, pp.cBi, pp.cBn, 0};
+            p.CPB, xl, pp.cB, pp.cBi, pp.cBn, 0, p.NCLB, 0};
     if (cmp_bwd(p) && (pp.cB == nullptr || pp.cBi == nullptr || pp.cBn == nullptr))
       return hipErrorInvalidValue;
     for (int l = 0; l < p.LCHB; ++l) {
@@ -5943,7 +6177,7 @@ struct Partials {
 
 hipError_t presum(const Plan& p, const float* rpart, const float* npart, const PresumBuf& ps,
                   hipStream_t s, Partials& out) {
-  out = Partials{rpart, p.NCH, npart, p.B};
+  out = Partials{rpart, p.NCH, npart, p.B};  // p.NCH: the partials written (rec_parts)
   auto pass = [&](const float* src, int M, long long N, float* dst) {
     const int parts = presum_parts(M);
     const int rpb = (M + parts - 1) / parts;
@@ -6004,7 +6238,7 @@ hipError_t launch_prep_leaf(const Plan& p, const LeafParams& lp, const Prepped& 
   const int sensf = (images & kLeafFwdImages) && !fs && pp.sF == nullptr ? 1 : 0;
 #define LTC_PREPL(C, F)                                                                           \
   LTC_LAUNCH((prep_leaf_kernel<C, F>), dim3(nprep + ncmp + nln), dim3(threads), 0, s, lp, pp, \
-                     p.H, p.D, p.Hp, p.Dp, bwd ? (p.FUSE ? 1 : 2) : 0, sensf, bwd ? 1 : 0, nprep, \
+                     p.H, p.D, p.Hp, p.Dp, bwd ? (chain_fused(p) ? 1 : 2) : 0, sensf, bwd ? 1 : 0, nprep, \
                      ncmp, cmp_chunks_fwd(p), cmp_chunks_bwd(p), lb, p.T, BT, clear_words,       \
                      nclear, sn, sd)
   if (fs) {

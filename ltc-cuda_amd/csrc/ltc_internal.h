@@ -97,8 +97,9 @@ struct Plan {
   // launch holding at most one workgroup per CU. Forward and chain.
   int LCH, LCHB;
   // Register-resident clusters (plan_reg_clusters): when rf.CP > 0 the forward
-  // ODE kernel runs in this geometry instead of the one above.
-  RegCluster rf;
+  // ODE kernel runs in this geometry instead of the one above, when rb.CP > 0
+  // the chain does (fused, one gradient partial per cluster).
+  RegCluster rf, rb;
 };
 
 // Derived, zero-padded parameter images built once per call by the prep kernel.
@@ -143,7 +144,13 @@ struct Prepped {
   // 1: the same image as one list per neuron over all of D instead
   // ([slot][Hp] operands and input indices, [Hp] counts; sens_full_list)
   int sFfull;
+  // 1: mark chain columns whose w cannot be factored out of wE
+  // (kChainIrregular in the column's count)
+  int cBmark;
 };
+// Set in a chain column's count when an entry's |wE| exceeds 1e18 |w| (w = 0
+// with wE nonzero among them): the chain that factors w out cannot take it.
+constexpr int kChainIrregular = 1 << 30;
 // Chunks (and slots per chunk) of a compacted image column at Hp = 256.
 constexpr int kCmpChunks = 16;
 // LDS of the compacted kernels' slot table: one int per slot per thread.
@@ -328,8 +335,13 @@ inline long long cluster_words(const Plan& p) {
 }
 // Whether the call's ODE kernel runs as clusters (its waits can give up).
 inline bool fwd_clusters(const Plan& p) { return p.rf.CP > 0 || p.CP > 0; }
-inline bool bwd_clusters(const Plan& p) { return p.CP > 0; }
+inline bool bwd_clusters(const Plan& p) { return p.rb.CP > 0 || p.CP > 0; }
+// Whether the chain forms the recurrent parameter-gradient sums itself, and
+// how many partials of them the backward's finalize sums.
+inline bool chain_fused(const Plan& p) { return p.rb.CP > 0 || p.FUSE; }
+inline int rec_parts(const Plan& p) { return p.rb.CP > 0 ? p.rb.NCL : p.NCH; }
 inline long long cluster_words_bwd(const Plan& p) {
+  if (p.rb.CP > 0) return 2LL * p.rb.NCL * p.rb.CP * p.rb.NB * p.rb.JW;
   return 2LL * p.NCLB * p.CPB * p.NBB * p.JWB;
 }
 // Rows of slack after the [Hp][Hp] operand images that the cluster kernels'
@@ -429,20 +441,26 @@ inline long long row_bwd_words(const Plan& p) {
 // Whether the forward launch reads a compacted image: the plan's own forms
 // (cmp_fwd) or the register-resident clusters.
 inline bool fwd_image_cmp(const Plan& p) { return p.rf.CP > 0 || cmp_fwd(p); }
+inline bool bwd_image_cmp(const Plan& p) { return p.rb.CP > 0 || cmp_bwd(p); }
 inline int cmp_chunks_fwd(const Plan& p) {
   if (p.rf.CP > 0) return p.rf.KS;
   return (row_kernels(p) || row_wave128_fwd(p)) ? 4 : (p.CP > 0 ? kCmpChunks : p.KS);
 }
 inline int cmp_chunks_bwd(const Plan& p) {
+  if (p.rb.CP > 0) return p.rb.KS;
   return row_kernels(p) ? 8 : (row_wave128_bwd(p) ? 4 : (p.CP > 0 ? kCmpChunks : p.KSB));
 }
+// LDS tile of a fused chain member's gradient partials: 32 padded rows.
+inline long long partial_tile_lds(int hp) { return 32LL * (hp + 1) * 4; }
 // Dynamic LDS of a cluster chain member (cluster_chain_lds) plus, with the
 // compacted image, its slot table.
 inline long long cluster_bwd_lds(const Plan& p) {
-  return cluster_chain_lds(p.NBB, p.Hp, p.KSB, p.JWB, chain_prefetches(p)) +
-         (cmp_bwd(p) ? cmp_index_lds(p.JWB * p.KSB) + cmp_pad_lds(p.Hp) +
-                           balance_lds(p.JWB * p.KSB)
-                     : 0);
+  const long long n = cluster_chain_lds(p.NBB, p.Hp, p.KSB, p.JWB, chain_prefetches(p)) +
+                      (cmp_bwd(p) ? cmp_index_lds(p.JWB * p.KSB) + cmp_pad_lds(p.Hp) +
+                                        balance_lds(p.JWB * p.KSB)
+                                  : 0);
+  // the fused forms' gradient partials leave through an LDS tile
+  return p.FUSE && n < partial_tile_lds(p.Hp) ? partial_tile_lds(p.Hp) : n;
 }
 // Dynamic LDS of a cluster forward member: state rows [NB][Hp], the KS
 // partials [KS][NB][64] float2, and with the compacted image the slot table.
@@ -457,6 +475,19 @@ inline long long reg_fwd_lds(const RegCluster& g, int hp) {
   if (g.NB == 1) return 2LL * hp * 4;  // the wave-owned form: the state by parity
   return (long long)g.NB * hp * 4 + (long long)g.KS * g.NB * g.JW * 8 + cmp_index_lds(1024) +
          balance_lds(1024);
+}
+// A register-resident chain member of 512 threads: alpha/beta rows padded by
+// two pairs, the partials of both groups, 1/den of two unfolds and v of three
+// slots, and the balanced lane order's scratch (counts up to kRegChainSlots).
+constexpr int kRegChainSlots = 20;
+// Synapses a chain thread of Hp / 16 = rc holds in registers: all of them up
+// to 16 (Hp <= 256); beyond, enough for half-dense masks (at Hp = 512 the
+// fullest of 512 columns has about 290 entries, 19 a thread; at 448, 256).
+inline int reg_chain_slots(int rc) { return rc <= 16 ? rc : (rc <= 28 ? 16 : 20); }
+inline long long reg_bwd_lds(const RegCluster& g, int hp) {
+  const long long n = (g.NB + 2LL) * hp * 8 + (long long)g.KS * g.NB * g.JW * 4 +
+                      chain_pf_bytes(g.NB) * g.NB * hp + 512 * 4 + 8 * (kRegChainSlots + 1) * 4;
+  return n > partial_tile_lds(hp) ? n : partial_tile_lds(hp);
 }
 // Dynamic LDS of the single-workgroup forward: state rows and the KS
 // partials, or the wave-owned single-row forward's state and staged sums.

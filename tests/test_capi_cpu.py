@@ -461,6 +461,15 @@ def test_register_resident_cluster_plan(capi, B, H):
     """Forward members of 64 or 32 columns whose 1024 threads hold every synapse
     of a dense column (20 or 16 each), one workgroup per CU and launch."""
     p = capi.plan(B, 4, 8, H, 6)
+    if p["reg_bwd_members"]:
+        # the chain: 32 columns a member, in a launch per slots * rows batch rows
+        cp, nb = p["reg_bwd_members"], p["reg_bwd_rows"]
+        assert cp * 32 == p["Hp"] and nb in (2, 4, 8) and p["reg_bwd_lds"] <= 159 * 1024
+        assert p["reg_bwd_launches"] == -(-B // (nb * min(256 // cp, -(-B // nb))))
+        # a second gather word per 512 threads' worth, at most four
+        assert (cp - 1) * nb * 16 <= 512 * (nb // 2 if p["Hp"] > 256 else (2 if nb == 8 else 1))
+    else:
+        assert p["Hp"] == 256 and p["fuse"] == 1
     if p["reg_fwd_members"] == 0:
         assert p["Hp"] == 256 and p["cmp_fwd"] == 1  # the plan's own form holds them
         return

@@ -15,7 +15,9 @@ import pytest
 import torch
 
 import ltc_cuda
-from _gpu_common import (_native, boundary, gpu_forward, oracle_forward)  # noqa: F401
+from _gpu_common import (DEV, _native, _oracle_module_grads, _perturbed_module,  # noqa: F401
+                         assert_grads_close, boundary, gpu_backward, gpu_forward,
+                         oracle_forward, oracle_grads)
 
 pytestmark = pytest.mark.gpu
 
@@ -101,3 +103,92 @@ def test_nan_sum_spreads_one_unfold_later():
     _, res = gpu_forward([x] + args[1:], U=2)
     assert torch.isnan(res[0].cpu()[2, 0]).all()
     assert torch.isfinite(res[0].cpu()[3]).all()
+
+
+# (B, T, D, H, density, rows per cluster, launches): the chain, which needs
+# 16 (H <= 448) or 20 synapses per thread and past that runs the kernel that
+# streams dense operands
+BWD = [
+    (1, 3, 8, 129, 0.5, 2, 1),
+    (85, 2, 5, 192, 0.5, 4, 1),
+    (337, 1, 5, 192, 1.0, 8, 2),   # 336 rows per launch; 12 synapses each when dense
+    (257, 1, 4, 256, 0.5, 8, 2),   # one row in the second launch
+    (3, 2, 70, 257, 0.5, 2, 1),
+    (101, 1, 5, 320, 0.5, 8, 1),   # 4 gather words per thread
+    (30, 2, 5, 320, 1.0, 2, 1),    # streamed
+    (43, 2, 5, 384, 0.5, 4, 1),    # 21 clusters of 12 members hold 42 rows at two each
+    (22, 1, 5, 384, 1.0, 2, 1),
+    (150, 1, 5, 448, 1.0, 8, 2),
+    (37, 1, 5, 448, 0.5, 4, 1),
+    (129, 1, 5, 512, 0.5, 8, 2),
+    (40, 1, 5, 500, 1.0, 4, 1),
+]
+
+
+@pytest.mark.parametrize("shape", BWD, ids=lambda s: "B%dT%dD%dH%dp%g" % s[:5])
+def test_module_backward_matches_oracle(shape):
+    B, T, D, H, density, rows, launches = shape
+    p = ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)
+    assert p["reg_bwd_members"] * 32 == p["Hp"], p
+    assert (p["reg_bwd_rows"], p["reg_bwd_launches"]) == (rows, launches), p
+    m = _perturbed_module(D, H, seed=B + H, sparsity=density).to(DEV)
+    with torch.no_grad():  # a neuron whose only outgoing synapse ends at the last one
+        m.sparsity_mask[2] = 0.0
+        m.sparsity_mask[2, H - 1] = 1.0
+    g = torch.Generator().manual_seed(17)
+    x = torch.randn(B, T, D, generator=g)
+    h0 = torch.randn(B, H, generator=g) * 0.2
+    G = torch.randn(B, T, H, generator=g)
+    Gh = torch.randn(B, H, generator=g)
+    xg = x.to(DEV).requires_grad_(True)
+    hg = h0.to(DEV).requires_grad_(True)
+    out, (h, _) = m(xg, (hg, hg))
+    ((out * G.to(DEV)).sum() + (h * Gh.to(DEV)).sum()).backward()
+    r_out, r_h, r_g, r_gx, r_gh = _oracle_module_grads(m, x, h0, G, Gh)
+    # float32 sums over U*T*B instances in fixed order: relative 2-norm errors
+    # of a few 1e-6; 2e-5 leaves the room the weight gradients' cancelling
+    # terms need
+    for name, a, b in ([("x", xg.grad, r_gx), ("h0", hg.grad, r_gh)]
+                       + [(n, q.grad, r_g[n]) for n, q in m.named_parameters()]):
+        err = ((a.cpu().double() - b).norm() / b.norm()).item()
+        assert err <= 2e-5, f"{name}: {err:.1e}"
+
+
+@pytest.mark.parametrize("shape", [(5, 2, 6, 192), (300, 1, 4, 256), (40, 1, 4, 320),
+                                   (20, 2, 4, 500)], ids=lambda s: "B%dT%dD%dH%d" % s)
+def test_boundary_backward_with_unequal_zero_weights(shape):
+    """w_pos = 0 where w_erev is not (and the other way round): the factor the
+    register form takes out of them does not exist there."""
+    B, T, D, H = shape
+    assert ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)["reg_bwd_members"] > 0
+    args = boundary(B, T, D, H, seed=5)
+    g = torch.Generator().manual_seed(6)
+    pick = torch.rand(H, H, generator=g)
+    args[2] = torch.where(pick < 0.1, torch.zeros(()), args[2])
+    args[3] = torch.where(pick > 0.9, torch.zeros(()), args[3])
+    dev_args, (out, h, saved) = gpu_forward(args, save=True)
+    g_out = torch.randn(B, T, H, generator=g)
+    g_h = torch.randn(B, H, generator=g)
+    got = gpu_backward(dev_args, saved, g_out.to(DEV), g_h.to(DEV))
+    ref = oracle_grads(args, g_out, g_h)
+    assert_grads_close(got, ref, f"{shape}")
+
+
+@pytest.mark.parametrize("shape", [(6, 1, 4, 192), (60, 1, 4, 384)],
+                         ids=lambda s: "B%dT%dD%dH%d" % s)
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_non_finite_gradient_reaches_its_whole_row(shape, value):
+    """Zero weight times a non-finite dL/dout is NaN: dL/dh0 of that row has no
+    finite entry, and every other row is untouched."""
+    B, T, D, H = shape
+    m = _perturbed_module(D, H, seed=4).to(DEV)
+    x = torch.randn(B, T, D, generator=torch.Generator().manual_seed(1)).to(DEV)
+    h0 = torch.zeros(B, H, device=DEV, requires_grad=True)
+    out, _ = m(x, (h0, h0))
+    G = torch.ones(B, T, H, device=DEV)
+    clean, = torch.autograd.grad(out, h0, G, retain_graph=True)
+    G[3, 0, 11] = value
+    dirty, = torch.autograd.grad(out, h0, G)
+    assert not torch.isfinite(dirty[3]).any()
+    keep = [b for b in range(B) if b != 3]
+    assert torch.equal(dirty[keep], clean[keep])
