@@ -1284,7 +1284,7 @@ int ltc_module_backward(const float* x, long long sxb, long long sxt, long long 
     if (e != hipSuccess) return hip_fail("ODE backward launch", e);
     if (!ltc::chain_fused(p)) {
       e = timed(ltc::K_REC_GRAD, s,
-                [&] { return ltc::launch_rec_grad(p, wb.pp, vsave, wb.absave, wb.rpart, s); });
+                [&] { return ltc::launch_rec_grad(p, wb.pp, vsave, wb.absave, wb.rpart, s, lp.mask); });
       if (e != hipSuccess) return hip_fail("recurrent gradient launch", e);
     }
   }

@@ -2539,26 +2539,131 @@ __global__ __launch_bounds__(512) void ode_bwd_row_fused_kernel(BwdK k, RowCompa
 }
 
 // ---------------------------------------------------------------------------
-// Recurrent parameter gradients, reduced over n = (t,k,b).
-// grid (Hp/64, Hp/32, NCH), block 256: lane -> j, wave w -> 8 presynaptic i.
+// Recurrent parameter gradients, reduced over n = (t,k,b), of the synapses that
+// have any: those with a nonzero mask entry on the module path, every real one
+// on the boundary. grid (Hp/64, Hp/32, NCH), block 256, a tile of 32
+// presynaptic i x 64 postsynaptic j. Nothing is reduced over i or j here, so
+// a thread can take any synapse: the block lists its tile's synapses in row
+// order and thread t takes entries t, t + 256, ... (at most 6), and a wave
+// runs as many slots as it has entries: half the work at half-dense masks,
+// and nothing for the padding of H to Hp. Neighbouring threads mostly share i
+// and have neighbouring j, so their LDS reads of v_i and alpha/beta_j stay
+// broadcasts and nearly conflict-free. Nearly full tiles take every synapse
+// (rec_grad_dense). VALU-bound (B128 T25 H100 half-dense: 128 us with every
+// synapse of the padded tile evaluated, 88 us this way).
 // Per synapse and n:  a = gate, a2 = a(1-a), h = alpha*WE + beta*WP,
 //   sWE += alpha*a, sWP += beta*a, sD += h*a2, sDv += h*a2*v_i
-// and the finalize kernel forms dM = -S*sD and dS = sDv - M*sD.
+// and the finalize kernel forms dM = -S*sD and dS = sDv - M*sD. Partials of
+// synapses not listed stay unwritten; the finalize does not read them.
 // ---------------------------------------------------------------------------
 constexpr int RG_NT = 32;
+// Entries up to which a tile of 2048 goes by its list: six slots a thread cost
+// about what the dense form's eight do.
+constexpr int kRecListMax = 1536;
 
 struct RecGK {
   const float4* recF;
   const float* vsave;
   const float2* absave;
+  const float* mask;  // (H,H), or null: every real synapse
   float* rpart;
-  int Hp;
+  int H, Hp;
   long long N, nper;
 };
 
-__global__ __launch_bounds__(256) void rec_grad_kernel(RecGK k) {
-  __shared__ __align__(16) float vsh[RG_NT][32];
-  __shared__ __align__(16) float2 absh[RG_NT][64];
+template <int NS>
+__device__ __forceinline__ void rec_grad_rows(const RecGK& k, const unsigned short* list, int total,
+                                              float (*vsh)[32], float2 (*absh)[64]) {
+  const int Hp = k.Hp, tid = threadIdx.x;
+  const int jb = blockIdx.x * 64, ib = blockIdx.y * 32;
+  float4 p[NS];
+  int lv[NS], lab[NS];  // LDS positions of the entry's v_i and alpha/beta_j
+  float sWE[NS], sWP[NS], sD[NS], sDv[NS];
+#pragma unroll
+  for (int q = 0; q < NS; ++q) {
+    sWE[q] = sWP[q] = sD[q] = sDv[q] = 0.f;
+    const int e = tid + 256 * q;
+    const int c = e < total ? list[e] : 0, i = c >> 6, j = c & 63;
+    lv[q] = i;
+    lab[q] = j;
+    p[q] = e < total ? k.recF[(ib + i) * Hp + jb + j] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  const long long nb = (long long)blockIdx.z * k.nper;
+  const long long ne = min(k.N, nb + k.nper);
+  // A chunk's v_i and alpha/beta rows are loaded into registers one chunk
+  // ahead, so the loads travel while the previous chunk is evaluated.
+  constexpr int NV = RG_NT * 32 / 256, NA = RG_NT * 64 / 256;
+  float nv[NV];
+  float2 nab[NA];
+  // Element (n0 + 8q + tid / 32, ib + tid % 32) of v and (n0 + 4q + tid / 64, jb
+  // + tid % 64) of alpha/beta: wave-uniform bases and one 32-bit lane offset
+  // each, so that no address is held per element.
+  const unsigned voff = (unsigned)((tid >> 5) * Hp + (tid & 31));
+  const unsigned aoff = (unsigned)((tid >> 6) * Hp + (tid & 63));
+  auto fetch = [&](long long n0) {
+    const int left = (int)min((long long)RG_NT, ne - n0);
+    const float* vb = k.vsave + n0 * Hp + ib;
+    const float2* ab = k.absave + n0 * Hp + jb;
+#pragma unroll
+    for (int q = 0; q < NV; ++q)
+      nv[q] = q * 8 + (tid >> 5) < left ? (vb + q * 8 * Hp)[voff] : 0.f;
+#pragma unroll
+    for (int q = 0; q < NA; ++q)
+      nab[q] = q * 4 + (tid >> 6) < left ? (ab + q * 4 * Hp)[aoff] : make_float2(0.f, 0.f);
+  };
+  if (nb < ne) fetch(nb);
+#pragma unroll 1
+  for (long long n0 = nb; n0 < ne; n0 += RG_NT) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q) vsh[q * 8 + (tid >> 5)][tid & 31] = nv[q];
+#pragma unroll
+    for (int q = 0; q < NA; ++q) absh[q * 4 + (tid >> 6)][tid & 63] = nab[q];
+    __syncthreads();
+    if (n0 + RG_NT < ne) fetch(n0 + RG_NT);
+    // UN instances at a time at constant LDS offsets; those past the chunk
+    // hold alpha = beta = 0 and add zero. (With 2 or 1 of them and three waves
+    // a SIMD instead of two: 88 -> 98 us.)
+    constexpr int UN = 4;
+    const int cnt = (int)min((long long)RG_NT, ne - n0);
+#pragma unroll 1
+    for (int nn = 0; nn < cnt; nn += UN) {
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+#pragma unroll
+        for (int q = 0; q < NS; ++q) {
+          const float v = (&vsh[nn][0])[u * 32 + lv[q]];
+          const float2 c = (&absh[nn][0])[u * 64 + lab[q]];
+          const float a = gate(fmaf(p[q].x, v, p[q].y));
+          const float a2 = fmaf(-a, a, a);
+          sWE[q] = fmaf(c.x, a, sWE[q]);
+          sWP[q] = fmaf(c.y, a, sWP[q]);
+          const float dl = fmaf(c.x, p[q].z, c.y * p[q].w) * a2;
+          sD[q] += dl;
+          sDv[q] = fmaf(dl, v, sDv[q]);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  const long long HH = (long long)Hp * Hp;
+  float* out = k.rpart + (long long)blockIdx.z * 4 * HH;
+#pragma unroll
+  for (int q = 0; q < NS; ++q) {
+    if (tid + 256 * q < total) {
+      float* o = out + (ib + lv[q]) * Hp + jb + lab[q];
+      o[0] = sWE[q];
+      o[HH] = sWP[q];
+      o[2 * HH] = sD[q];
+      o[3 * HH] = sDv[q];
+    }
+  }
+}
+
+// Every synapse of the tile: lane -> j, wave w -> 8 presynaptic i, whose v come
+// as two 16-byte LDS reads and share one alpha/beta read. The better form of a
+// nearly full tile (B128 T25 H128 dense: 129 us, 152 us by the list).
+__device__ __forceinline__ void rec_grad_dense(const RecGK& k, float (*vsh)[32],
+                                               float2 (*absh)[64]) {
   const int Hp = k.Hp;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int jb = blockIdx.x * 64, ib = blockIdx.y * 32;
@@ -2633,6 +2738,58 @@ __global__ __launch_bounds__(256) void rec_grad_kernel(RecGK k) {
     out[HH + e] = sWP[ii];
     out[2 * HH + e] = sD[ii];
     out[3 * HH + e] = sDv[ii];
+  }
+}
+
+__global__ __launch_bounds__(256) void rec_grad_kernel(RecGK k) {
+  __shared__ __align__(16) float vsh[RG_NT][32];
+  __shared__ __align__(16) float2 absh[RG_NT][64];
+  __shared__ unsigned short list[32 * 64];
+  __shared__ int wtot[4];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, H = k.H;
+  // This thread's eight synapses of the tile: row i, columns j0 ... j0 + 7.
+  const int i = tid >> 3, j0 = (tid & 7) * 8;
+  const int gi = blockIdx.y * 32 + i, gj = blockIdx.x * 64 + j0;
+  unsigned m = 0;
+  if (gi < H) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (gj + q < H && (k.mask == nullptr || k.mask[(long long)gi * H + gj + q] != 0.f))
+        m |= 1u << q;
+  }
+  const int mine = __popc(m);
+  int incl = mine;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int up = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += up;
+  }
+  if (lane == 63) wtot[w] = incl;
+  __syncthreads();
+  int at = incl - mine, total = 0;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    if (x < w) at += wtot[x];
+    total += wtot[x];
+  }
+  if (total > kRecListMax) {  // uniform over the block
+    rec_grad_dense(k, vsh, absh);
+    return;
+  }
+  while (m != 0) {
+    const int q = __builtin_ctz(m);
+    m &= m - 1;
+    list[at++] = (unsigned short)((i << 6) | (j0 + q));
+  }
+  __syncthreads();
+  // slots of this wave: its first entry is 64 w
+  const int ns = __builtin_amdgcn_readfirstlane(total > 64 * w ? (total - 64 * w + 255) / 256 : 0);
+  switch (ns) {
+#define LTC_RG(N) \
+  case N: rec_grad_rows<N>(k, list, total, vsh, absh); break;
+    LTC_RG(2) LTC_RG(3) LTC_RG(4) LTC_RG(5) LTC_RG(6)
+    default: rec_grad_rows<1>(k, list, total, vsh, absh); break;
+#undef LTC_RG
   }
 }
 
@@ -6145,9 +6302,9 @@ hipError_t launch_ode_bwd_row_fused(const Plan& p, const Prepped& pp, const floa
 }
 
 hipError_t launch_rec_grad(const Plan& p, const Prepped& pp, const float* vsave,
-                           const float2* absave, float* rpart, hipStream_t s) {
+                           const float2* absave, float* rpart, hipStream_t s, const float* mask) {
   const long long nper = (p.N + p.NCH - 1) / p.NCH;
-  RecGK a{pp.recF, vsave, absave, rpart, p.Hp, p.N, nper};
+  RecGK a{pp.recF, vsave, absave, mask, rpart, p.H, p.Hp, p.N, nper};
   LTC_LAUNCH(rec_grad_kernel, dim3(p.Hp / 64, p.Hp / 32, p.NCH), dim3(256), 0, s, a);
   return hipGetLastError();
 }

@@ -554,8 +554,11 @@ hipError_t launch_ode_bwd(const Plan& p, const Prepped& pp, const float* vsave,
                           const float* ghfin, float2* absave, float* dsn, float* dsd,
                           float* npart, float* gstate, float* rpart, const ClusterBuf& cb,
                           hipStream_t s);
+// mask (the module path's recurrent mask, (H,H)): skip the masked synapses,
+// whose partials stay unwritten.
 hipError_t launch_rec_grad(const Plan& p, const Prepped& pp, const float* vsave,
-                           const float2* absave, float* rpart, hipStream_t s);
+                           const float2* absave, float* rpart, hipStream_t s,
+                           const float* mask = nullptr);
 // smask (the module path's sensory mask, (D,H)): skip the masked synapses
 // (sens_bwd_cmp_kernel), whose partials stay unwritten.
 hipError_t launch_sens_bwd(const Plan& p, const float* x, Strides3 xs, const Prepped& pp,
