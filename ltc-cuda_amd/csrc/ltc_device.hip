@@ -4530,7 +4530,9 @@ __device__ __forceinline__ float lane_group_sum(float v) {
 // state rows, so an unfold has one barrier. Members are as wide as the
 // registers allow (an exchange costs more the more members take part: Hp =
 // 320, 1.9-2.2 us an unfold with 5 members of 64 columns, 2.5 with 10, 3.6
-// with 20). NaN states and waits as in ode_fwd_cl2_kernel.
+// with 20). B8 T100 H320 in 600 sequential unfolds: 2392 -> 1312 us a call
+// against the streamed cluster form. NaN states and waits as in
+// ode_fwd_cl2_kernel.
 template <int LPC, int RCP>
 __global__ __launch_bounds__(1024) void ode_fwd_own_kernel(FwdCK k) {
   constexpr int NT = 1024, CW = 64 / LPC, JW = NT / LPC, ZG = 4;
@@ -5271,7 +5273,24 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
   if constexpr (FUSE) {
     // This cluster's share of the recurrent parameter gradients for synapses
     // (i = sc, j = r0 + rr or the slot's row), layout [cluster][4][i][j] as
-    // rec_grad_kernel's.
+    // rec_grad_kernel's. The compacted form writes its slots directly: half
+    // the entries, and at Hp = 256 the tile costs more than it saves (B8 T2
+    // chain 43 -> 48 us). Hp = 256 is one launch, so nothing is added to.
+    if constexpr (CMP) {
+      const long long HH = (long long)Hp * Hp;
+      float* out = k.rpart + (long long)cl * 4 * HH + (long long)sc * Hp;
+#pragma unroll
+      for (int rr = 0; rr < NACC; ++rr) {
+        if (rr < nmine) {
+          const int j = k.cidx[(long long)(sks * RCP + rr) * Hp + sc];
+          out[j] = gacc[rr].x;
+          out[HH + j] = gacc[rr].y;
+          out[2 * HH + j] = gacc[rr].z;
+          out[3 * HH + j] = gacc[rr].w;
+        }
+      }
+      return;
+    }
     store_partials32(reinterpret_cast<float*>(lds4),
                      k.rpart + (long long)cl * 4 * Hp * Hp + (long long)p * JW * Hp, Hp, k.R0 > 0,
                      [&](float* tile, int stride, int pl) {
@@ -5279,12 +5298,7 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
                        for (int rr = 0; rr < NACC; ++rr) {
                          const float4 v = gacc[rr];
                          const float x = pl == 0 ? v.x : (pl == 1 ? v.y : (pl == 2 ? v.z : v.w));
-                         if constexpr (CMP) {
-                           if (rr < nmine)
-                             tile[so * stride + k.cidx[(long long)(sks * RCP + rr) * Hp + sc]] = x;
-                         } else {
-                           tile[o * stride + r0 + rr] = x;
-                         }
+                         tile[o * stride + r0 + rr] = x;
                        }
                      });
   }
@@ -5313,8 +5327,14 @@ constexpr float kMinSlope = 1e-20f;
 // REG: the register-resident clusters beyond that form: 12 or 16 slots cover
 // Hp = 192 or 256, 16 slots Hp = 320 ... 448 and 20 Hp = 512 while no column
 // has more than 16 * RCP entries (half-dense masks; a second launch, of
-// ode_bwd_cl_kernel, covers the rest). FACT factors w out as above, which needs w != 0 wherever wE is
-// (kChainIrregular otherwise); without it the operands stay (x, y, wE, w).
+// ode_bwd_cl_kernel, covers the rest). Bound by the slot loops at two waves per
+// SIMD and the exchange of up to 16 members: B64 T32 H192 554 us (chain 996
+// and rec_grad 205 before), H512 1104 us (1868). Partials are written slot by
+// slot: through store_partials32's tile, whole planes of which half is padding,
+// B64 T32 H512 took 1124 instead of 1111 us and B256 T4 H512, whose two
+// launches add, 676 instead of 640. FACT factors w out as above, which needs
+// w != 0 wherever wE is (kChainIrregular otherwise); without it the operands
+// stay (x, y, wE, w).
 // REG's fourth sum is that of dl * zp, zp = x v + y the gate's argument, not of
 // dl * v: the sigma gradient is sum dl (v - mu), and summed as sum dl v less mu
 // sum dl its terms cancel only after hundreds of rounded additions (B64 T32
@@ -5732,32 +5752,27 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
     for (int rr = 0; rr < RCP; ++rr)
       gacc[rr].w = (gacc[rr].w - preg[rr].y * gacc[rr].z) / preg[rr].x;
   }
-  if constexpr (FACT) {
+  const long long HH = (long long)Hp * Hp;
+  float* out = k.rpart + (long long)cl * 4 * HH + (long long)sc * Hp;
 #pragma unroll
-    for (int rr = 0; rr < RCP; ++rr) {
-      if (rr < nmine) {
-        const float w = k.cimg[(long long)(sks_end * RC + rr) * Hp + sc].w;
-        gacc[rr].z *= w;  // the factor the last two sums left out
-        gacc[rr].w *= w;
+  for (int rr = 0; rr < RCP; ++rr) {
+    if (rr < nmine) {
+      const long long a = (long long)(sks_end * RC + rr) * Hp + sc;
+      const int j = k.cidx[a];
+      const float w = FACT ? k.cimg[a].w : 1.f;  // the factor the last two sums left out
+      float4 s = make_float4(gacc[rr].x, gacc[rr].y, gacc[rr].z * w, gacc[rr].w * w);
+      if (REG && k.R0 > 0) {  // a later launch of the call adds to the cluster's partial
+        s.x += out[j];
+        s.y += out[HH + j];
+        s.z += out[2 * HH + j];
+        s.w += out[3 * HH + j];
       }
+      out[j] = s.x;
+      out[HH + j] = s.y;
+      out[2 * HH + j] = s.z;
+      out[3 * HH + j] = s.w;
     }
   }
-  int jx[RCP];
-#pragma unroll
-  for (int rr = 0; rr < RCP; ++rr)
-    jx[rr] = rr < nmine ? k.cidx[(long long)(sks_end * RC + rr) * Hp + sc] : 0;
-  store_partials32(reinterpret_cast<float*>(lds4),
-                   k.rpart + (long long)cl * 4 * Hp * Hp + (long long)p * JW * Hp, Hp,
-                   REG && k.R0 > 0, [&](float* tile, int stride, int pl) {
-#pragma unroll
-                     for (int rr = 0; rr < RCP; ++rr) {
-                       if (rr < nmine) {
-                         const float4 v = gacc[rr];
-                         tile[so * stride + jx[rr]] =
-                             pl == 0 ? v.x : (pl == 1 ? v.y : (pl == 2 ? v.z : v.w));
-                       }
-                     }
-                   });
 }
 
 // Clears the cluster exchange words (tag 0) and the status word before a
