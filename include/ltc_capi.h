@@ -333,7 +333,7 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
 int ltc_launch_plan(int B, int T, int D, int H, int ode_unfolds, long long* out, int n);
 
 /*
- * Cluster give-up. For H > 192 the ODE kernels run as clusters of workgroups
+ * Cluster give-up. For H > 128 the ODE kernels run as clusters of workgroups
  * that exchange values every unfold and must all be resident at once (the
  * plan asks for at most one workgroup per CU). Each wait is bounded; when a
  * member runs out of its budget (another kernel held the CUs its partners

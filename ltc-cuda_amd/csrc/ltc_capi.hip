@@ -51,7 +51,8 @@ int device_cus() {
   return cache[dev];
 }
 
-// Cluster path (H > 192): CP = Hp/64 workgroups share NB rows, one 64-column
+// Cluster path of the base plan (H > 192; the register-resident clusters of
+// plan_reg_clusters replace its launches for 128 < H <= 512): CP = Hp/64 workgroups share NB rows, one 64-column
 // slice each, so every operand serves NB rows while up to one workgroup per
 // CU runs. The whole grid must be resident at once (members wait on each
 // other), so it is used only when NCL * CP <= CUs, with at most 1024 threads
@@ -213,6 +214,14 @@ void reg_cluster_counts(ltc::RegCluster& g, int B, int ncu) {
 // row per cluster (ode_fwd_own_kernel); else the fewest rows per cluster of
 // the two-group form that take the batch in one launch of at most one
 // workgroup per CU, and past eight rows as many launches as the batch needs.
+// Against the streamed kernels of the base plan (ode_fwd, us): B64 T32 H192
+// 929 -> 387, B64 T32 H512 1153 -> 618, every synapse unmasked B128 T32 H512
+// 1732 -> 1661; B1 T100 H320 3.9 -> 2.1 us an unfold. The line at 320 for one
+// row: 64-column members hold up to 20 slots per lane without spilling, and
+// fewer members exchange faster (H320 2.2 us an unfold with 5, 2.5 with 10);
+// with several rows a thread holds 16, so 32 columns beyond Hp = 256. At
+// Hp = 128 and below the single-workgroup forms keep every operand already,
+// and past 512 no member's registers hold its columns.
 void plan_reg_forward(ltc::Plan& p, int ncu) {
   if (p.CP > 0 && p.Hp == 256 && p.KS == 16 && p.RC == 16) return;
   ltc::RegCluster g{};
@@ -242,7 +251,10 @@ void plan_reg_forward(ltc::Plan& p, int ncu) {
 // thread: every one of a dense column up to Hp = 256, beyond that the synapses
 // of half-dense masks. The column counts are known on the device
 // only, so at those sizes a second launch, of the kernel that streams dense
-// operands, follows and exactly one of the two runs past its first check.
+// operands, follows and exactly one of the two runs past its first check
+// (about 3 us for the other). Against the base plan (us): B64 T32 H192 chain
+// and rec_grad 1201 -> 554, B64 T32 H512 chain 1868 -> 1104; every synapse
+// unmasked, B128 T32 H512 3241 -> 3238 (the streaming kernel either way).
 void plan_reg_chain(ltc::Plan& p, int ncu) {
   if (p.CP > 0 && p.Hp == 256 && p.FUSE) return;
   ltc::RegCluster g{};

@@ -4266,7 +4266,9 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl_kernel(FwdCK k) {
 // synapses that the image leaves out have weight zero, and 0 * NaN is NaN, so
 // a NaN in a row's state v^n makes every neuron of that row NaN at v^{n+1}.
 // Each state value is tested when it is written to LDS, and a row flag by
-// unfold parity carries the result to the owners.
+// unfold parity carries the result to the owners. With NF, bound by issue and
+// the phases' exchange: B64 T32 H192 387 us (929 in the streamed single-workgroup
+// form it replaced), B64 T32 H512 618 us (1153, streamed clusters).
 template <int NB, int JW = kClW, bool NF = false>
 __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
   static_assert(NB == 2 || NB == 4 || NB == 8, "two groups of rows");

@@ -740,7 +740,7 @@ def require_kernels():
 def device_status(clear: bool = True) -> None:
     """Raise RuntimeError if a launch on the current device gave up waiting
     for its partner workgroups since the last check: a cluster launch
-    (H > 192), or the companion workgroups of a module backward with one batch
+    (H > 128), or the companion workgroups of a module backward with one batch
     row per workgroup (the sensory and LayerNorm companions at H <= 64, the
     recurrent-gradient and sensory companions at 64 < H <= 128). The outputs
     of that call were set to NaN. Synchronises the device."""
