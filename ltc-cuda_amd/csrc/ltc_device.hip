@@ -288,21 +288,36 @@ __device__ __forceinline__ void stream_rows(__amdgpu_buffer_rsrc_t rs, int lane_
 // active rows their entry numbers in ascending row order. With nch chunks,
 // entry e goes to chunk e % nch, slot e / nch, so a dense column gives every
 // chunk the rows ks, ks + nch, ... and all lanes of a chunk the same row per
-// slot. Slots past the column's count get zero operands and row 0. The image
-// has nrows rows (slots of all chunks) of `stride` columns.
+// slot. The image has nrows rows (slots of all chunks) of `stride` columns.
+// The kernels evaluate slots past a column's count too (a wave runs as many as
+// its fullest lane), with a weight of zero, so such a slot's gate must not be
+// NaN where the column's own gates are not: it repeats the row, slope and
+// offset of the column's first entry. (With zero operands an infinite state of
+// row 0 gave 0 * inf = NaN in every column.) In a column without entries it
+// takes row 0 with a slope so small that every finite state's gate is 1/2,
+// and an infinite state's 0 or 1.
 // ---------------------------------------------------------------------------
+constexpr float kMinSlope = 1e-20f;
+
 template <class Op>
 __device__ __forceinline__ void compact_column(int col, int nrows, int stride, int nch, int lane,
                                                float4* cimg, int* cidx, int* ccnt, Op op) {
   const int sc = nrows / nch;
   auto at = [&](int e) { return (long long)((e % nch) * sc + e / nch) * stride + col; };
-  int n = 0;
+  int n = 0, pad_row = 0;
+  float4 pad = make_float4(kMinSlope, 0.f, 0.f, 0.f);
   for (int r0 = 0; r0 < nrows; r0 += 64) {
     const int r = r0 + lane;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     bool act = false;
     op(r, v, act);
     const unsigned long long m = __ballot(act);
+    if (n == 0 && m != 0) {  // wave-uniform
+      const int l = __ffsll(m) - 1;
+      pad_row = r0 + l;
+      pad.x = __shfl(v.x, l, 64);
+      pad.y = __shfl(v.y, l, 64);
+    }
     if (act) {
       const long long a = at(n + __popcll(m & ((1ULL << lane) - 1ULL)));
       cimg[a] = v;
@@ -312,8 +327,8 @@ __device__ __forceinline__ void compact_column(int col, int nrows, int stride, i
   }
   for (int e = n + lane; e < nrows; e += 64) {
     const long long a = at(e);
-    cimg[a] = make_float4(0.f, 0.f, 0.f, 0.f);
-    cidx[a] = 0;
+    cimg[a] = pad;
+    cidx[a] = pad_row;
   }
   if (lane == 0) ccnt[col] = n;
 }
@@ -609,8 +624,8 @@ __global__ __launch_bounds__(256) void sens_fwd_kernel(const float* __restrict__
 // the chunk; sFn: [chunk][Hp] counts), so a wave runs as many slots as its
 // fullest neuron has entries in the chunk instead of 64, and each lane reads
 // its slot's input at its own LDS address. With DS = 4 the four waves take
-// quarters of each chunk's slots. Slots past a count hold zero operands
-// (input 0) and add zero.
+// quarters of each chunk's slots. Slots past a count hold zero weights and
+// add zero.
 // ---------------------------------------------------------------------------
 // LN (DS = 1, D <= 64): x is the raw input, and each wave applies the
 // module's LayerNorm + affine to its rows of the staged chunk in place, with
@@ -4561,7 +4576,8 @@ __global__ __launch_bounds__(1024) void ode_fwd_own_kernel(FwdCK k) {
   unsigned ix[RCP / 2];
 #pragma unroll
   for (int rr = 0; rr < RCP; ++rr) {
-    preg[rr] = make_float4(0.f, 0.f, 0.f, 0.f);
+    // slots past the image's RC but within the last group of ZG
+    preg[rr] = make_float4(kMinSlope, 0.f, 0.f, 0.f);
     unsigned o = 0;
     if (rr < RC) {
       const int a = (ck * RC + rr) * Hp + c;
@@ -5305,10 +5321,6 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
                      });
   }
 }
-
-// Smallest |x| = |sigma| log2(e) of a register-resident chain slot: below it
-// every gate of bounded states is 1/2 to the last bit.
-constexpr float kMinSlope = 1e-20f;
 
 // The compacted fused cluster chain (register-resident operands, Hp = 256,
 // 32-column members of 512 threads) with its NB >= 2 rows in two groups of

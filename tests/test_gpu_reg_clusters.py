@@ -90,6 +90,29 @@ def test_nan_state_reaches_its_whole_row(shape, U):
     assert torch.isfinite(out[:B - 1]).all()
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 8, 192), (90, 1, 4, 192), (1, 1, 4, 300),
+                                   (60, 1, 4, 320), (5, 1, 4, 448), (300, 1, 4, 256)],
+                         ids=lambda s: "B%dT%dD%dH%d" % s)
+@pytest.mark.parametrize("i", [0, 7])
+def test_infinite_state_saturates_its_gates(shape, i):
+    """An infinite v_i makes the gates of its synapses 0 or 1, whatever slot holds
+    them or pads a column: every other neuron stays finite and equals the oracle."""
+    B, T, D, H = shape
+    assert ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)["reg_fwd_members"] > 0
+    args = _edge_masks(boundary(B, T, D, H, seed=14))
+    h0 = args[1].clone()
+    h0[0, i] = float("inf")
+    h0[B - 1, i] = -float("inf")
+    _, (out, h) = gpu_forward([args[0], h0] + args[2:])
+    ref_out, ref_h = oracle_forward([args[0], h0] + args[2:])
+    keep = [j for j in range(H) if j != i]
+    for got, ref in ((out, ref_out), (h, ref_h)):
+        got = got.cpu().double()[..., keep]
+        assert torch.isfinite(ref[..., keep]).all()
+        # the bound of test_forward_matches_oracle
+        assert (got - ref[..., keep]).abs().max().item() <= 5e-6
+
+
 def test_nan_sum_spreads_one_unfold_later():
     """A NaN input at a neuron's sensory synapse makes that neuron NaN in the
     first unfold and its whole row NaN in the second, as a dense kernel does."""
