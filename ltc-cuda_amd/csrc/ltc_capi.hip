@@ -463,11 +463,13 @@ void carve_cmp(const ltc::Plan& p, Carver& c, ltc::Prepped& pp, bool fwd, bool b
     pp.cF = c.take<float4>(n);
     pp.cFi = c.take<int>(n);
     pp.cFn = c.take<int>(p.Hp);
+    pp.cFdense = p.rf.CP > 0 ? 1 : 0;
   }
   if (bwd && ltc::bwd_image_cmp(p)) {
     pp.cB = c.take<float4>(n);
     pp.cBi = c.take<int>(n);
     pp.cBn = c.take<int>(p.Hp);
+    pp.cBdense = p.rb.CP > 0 ? 1 : 0;
     pp.cBmark = p.rb.CP > 0 && p.rb.RC > ltc::reg_chain_slots(p.rb.RC) ? 1 : 0;
   }
 }

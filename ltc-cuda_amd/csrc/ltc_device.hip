@@ -333,6 +333,14 @@ __device__ __forceinline__ void compact_column(int col, int nrows, int stride, i
   if (lane == 0) ccnt[col] = n;
 }
 
+// Whether a synapse of zero weight has to stay in an image that keeps the dense
+// kernels' results (Prepped::cFdense, cBdense): its gate can be NaN at a state
+// that is not, and 0 * NaN is NaN. With a finite slope other than zero and a
+// finite offset it cannot (an infinite state saturates it).
+__device__ __forceinline__ bool gate_can_be_nan(const float4& v) {
+  return !(fabsf(v.x) < __builtin_inff() && fabsf(v.y) < __builtin_inff()) || v.x == 0.f;
+}
+
 // Marks chain column `col` when any lane of its wave met an entry whose w cannot
 // be factored out of wE (Prepped::cBmark).
 __device__ __forceinline__ void mark_irregular(const Prepped& pp, int col, int lane, bool bad) {
@@ -398,7 +406,7 @@ __global__ __launch_bounds__(256) void prep_kernel(RawParams rp, Prepped pp, int
         compact_column(j, Hp, Hp, nchf, lane, pp.cF, pp.cFi, pp.cFn, [&](int i, float4& v, bool& act) {
           if (i < H && j < H) {
             operand(i, j, v);
-            act = v.z != 0.f || v.w != 0.f;
+            act = v.z != 0.f || v.w != 0.f || (pp.cFdense && gate_can_be_nan(v));
           }
         });
         return;
@@ -3580,7 +3588,7 @@ __global__ __launch_bounds__(FS ? kPrepSensThreads : 256) void prep_leaf_kernel(
         compact_column(j, Hp, Hp, nchf, lane, pp.cF, pp.cFi, pp.cFn, [&](int i, float4& v, bool& act) {
           if (i < H && j < H) {
             operand(i, j, v);
-            act = v.z != 0.f || v.w != 0.f;
+            act = v.z != 0.f || v.w != 0.f || (pp.cFdense && gate_can_be_nan(v));
           }
         });
         return;
@@ -3590,8 +3598,9 @@ __global__ __launch_bounds__(FS ? kPrepSensThreads : 256) void prep_leaf_kernel(
     if (recb && pp.cB != nullptr) {
       if (col < Hp) {
         // The fused chain (recb == 1) keeps the synapses whose mask entry is
-        // nonzero; the unfused one (recb == 2, folded operands) those that
-        // add to dL/dv.
+        // nonzero (with cBdense also masked ones that are NaN all the same);
+        // the unfused one (recb == 2, folded operands) those that add to
+        // dL/dv.
         const int i = col;
         bool bad = false;
         compact_column(i, Hp, Hp, nchb, lane, pp.cB, pp.cBi, pp.cBn, [&](int j, float4& v, bool& act) {
@@ -3600,10 +3609,11 @@ __global__ __launch_bounds__(FS ? kPrepSensThreads : 256) void prep_leaf_kernel(
               operand(i, j, v);
               v = make_float4(v.x, v.y, v.x * v.z, v.x * v.w);
               act = v.z != 0.f || v.w != 0.f;
-            } else if (lp.mask[(long long)i * H + j] != 0.f) {
-              operand(i, j, v);
-              act = true;
-              bad |= !(fabsf(v.z) <= 1e18f * fabsf(v.w));
+            } else {
+              act = lp.mask[(long long)i * H + j] != 0.f;
+              if (act || pp.cBdense) operand(i, j, v);
+              if (pp.cBdense) act |= v.z != 0.f || v.w != 0.f || gate_can_be_nan(v);
+              if (act) bad |= !(fabsf(v.z) <= 1e18f * fabsf(v.w));
             }
           }
         });

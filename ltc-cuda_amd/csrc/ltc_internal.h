@@ -148,6 +148,10 @@ struct Prepped {
   // 1: mark chain columns whose w cannot be factored out of wE
   // (kChainIrregular in the column's count)
   int cBmark;
+  // 1: the image's kernels replace dense ones and keep their results for
+  // non-finite operands: zero-weight synapses whose gate can be NaN at a state
+  // that is not stay in the columns (a NaN state the kernels handle themselves)
+  int cFdense, cBdense;
 };
 // Set in a chain column's count when an entry's |wE| exceeds 1e18 |w| (w = 0
 // with wE nonzero among them): the chain that factors w out cannot take it.

@@ -113,6 +113,35 @@ def test_infinite_state_saturates_its_gates(shape, i):
         assert (got - ref[..., keep]).abs().max().item() <= 5e-6
 
 
+@pytest.mark.parametrize("shape", [(2, 1, 4, 192), (90, 1, 4, 192), (2, 1, 4, 320),
+                                   (60, 1, 4, 320), (300, 1, 4, 256)],
+                         ids=lambda s: "B%dT%dD%dH%d" % s)
+@pytest.mark.parametrize("leaf,value", [("mu", float("nan")), ("sigma", float("nan")),
+                                        ("mu", float("inf"))])
+def test_non_finite_operand_at_a_masked_synapse(shape, leaf, value):
+    """Masked or not, a synapse with a NaN gate makes its neuron NaN (0 * NaN), and
+    one with an infinite argument does not (0 * 0 or 0 * 1): the output and
+    dL/dh0 are finite exactly where the oracle has them so."""
+    B, T, D, H = shape
+    m = _perturbed_module(D, H, seed=6).to(DEV)
+    m.ode_unfolds = 1
+    p = ltc_cuda._cuda_module.capi.plan(B, T, D, H, 1)
+    assert p["reg_fwd_members"] > 0
+    with torch.no_grad():
+        m.sparsity_mask[5, 9] = m.sparsity_mask[H - 1, H - 1] = 0.0
+        getattr(m, leaf)[5, 9] = value
+        getattr(m, leaf)[H - 1, H - 1] = -value
+    g = torch.Generator().manual_seed(2)
+    x = torch.randn(B, T, D, generator=g)
+    h0 = torch.randn(B, H, generator=g) * 0.2
+    hg = h0.to(DEV).requires_grad_(True)
+    out, (h, _) = m(x.to(DEV), (hg, hg))
+    out.sum().backward()
+    r_out, _, _, _, r_gh = _oracle_module_grads(m, x, h0, torch.ones(B, T, H), torch.zeros(B, H))
+    assert torch.equal(torch.isfinite(out.cpu()), torch.isfinite(r_out))
+    assert torch.equal(torch.isfinite(hg.grad.cpu()), torch.isfinite(r_gh))
+
+
 def test_nan_sum_spreads_one_unfold_later():
     """A NaN input at a neuron's sensory synapse makes that neuron NaN in the
     first unfold and its whole row NaN in the second, as a dense kernel does."""
