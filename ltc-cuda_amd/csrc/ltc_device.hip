@@ -5364,7 +5364,10 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
 // sum dl its terms cancel only after hundreds of rounded additions (B64 T32
 // H192: error against float64 2.2e-6, 1.3e-6 with rec_grad_kernel's shorter
 // sums). A slope x below kMinSlope is raised to it so that sum dl v can be
-// taken out again at the end.
+// taken out again at the end, unless the offset y counts beside it: then
+// |mu| = |y / x| > 1e12, and sum dl v, nothing beside mu sum dl, is left out.
+// (A gate argument past the float range, |sigma (v - mu)| > 2e38, makes that
+// synapse's sigma gradient NaN.)
 // REG keeps the dense kernels' treatment of a non-finite alpha or beta: the
 // synapses left out have weight zero, and zero times it is NaN, so dL/dv of
 // every neuron of that row that has such a synapse becomes NaN. A row flag by
@@ -5445,7 +5448,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
       // image operands (x, y, w E, w) -> (x, y, E, w x); an entry with
       // w = 0 (a padding slot) contributes nothing either way
       preg[rr] = FACT ? make_float4(q.x, q.y, q.w != 0.f ? q.z / q.w : 0.f, q.w * q.x) : q;
-      if (REG && fabsf(q.x) < kMinSlope) {  // the gate is 1/2 either way
+      if (REG && fabsf(q.x) < kMinSlope && fabsf(q.y) < 1e-8f) {  // the gate is 1/2 either way
         preg[rr].x = kMinSlope;
         preg[rr].y = 0.f;
       }
@@ -5774,7 +5777,9 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   if constexpr (REG) {
 #pragma unroll
     for (int rr = 0; rr < RCP; ++rr)
-      gacc[rr].w = (gacc[rr].w - preg[rr].y * gacc[rr].z) / preg[rr].x;
+      gacc[rr].w = fabsf(preg[rr].x) < kMinSlope
+                       ? 0.f
+                       : (gacc[rr].w - preg[rr].y * gacc[rr].z) / preg[rr].x;
   }
   const long long HH = (long long)Hp * Hp;
   float* out = k.rpart + (long long)cl * 4 * HH + (long long)sc * Hp;

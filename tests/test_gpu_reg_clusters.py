@@ -244,3 +244,29 @@ def test_non_finite_gradient_reaches_its_whole_row(shape, value):
     assert not torch.isfinite(dirty[3]).any()
     keep = [b for b in range(B) if b != 3]
     assert torch.equal(dirty[keep], clean[keep])
+
+
+@pytest.mark.parametrize("shape", [(5, 2, 6, 192), (40, 1, 4, 320)], ids=lambda s: "B%dT%dD%dH%d" % s)
+@pytest.mark.parametrize("sigma,mu", [(0.0, 0.5), (1e-22, 0.5), (1e-22, 1e22), (-1e-21, 2e21),
+                                      (1e-15, 1e15)])
+def test_gradients_at_a_vanishing_slope(shape, sigma, mu):
+    """A slope too small to tell the states apart: the gate is 1/2, or that of the
+    offset alone when |mu| is as large as the slope is small."""
+    B, T, D, H = shape
+    m = _perturbed_module(D, H, seed=8).to(DEV)
+    with torch.no_grad():
+        m.sparsity_mask[3, 4] = 1.0
+        m.sigma[3, 4], m.mu[3, 4] = sigma, mu
+    g = torch.Generator().manual_seed(9)
+    x = torch.randn(B, T, D, generator=g)
+    h0 = torch.randn(B, H, generator=g) * 0.2
+    G = torch.randn(B, T, H, generator=g)
+    hg = h0.to(DEV)
+    out, _ = m(x.to(DEV), (hg, hg))
+    (out * G.to(DEV)).sum().backward()
+    _, _, r_g, _, _ = _oracle_module_grads(m, x, h0, G, torch.zeros(B, H))
+    for n in ("w", "erev", "mu", "sigma"):
+        got = dict(m.named_parameters())[n].grad[3, 4].item()
+        ref = r_g[n][3, 4].item()
+        # a float32 sum of a few hundred terms whose signs differ
+        assert abs(got - ref) <= 1e-4 * abs(ref) + 1e-30, (n, got, ref)
