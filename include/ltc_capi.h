@@ -322,14 +322,14 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
  * operands): workgroups per cluster (0: not used, and the forward runs in the
  * geometry above), columns per workgroup, rows per cluster, launches per call
  * and LDS bytes per workgroup. They keep the state's NaN treatment of the
- * geometry they replace (cmp_fwd above); then four of the register-resident
+ * geometry they replace (cmp_fwd above); then five of the register-resident
  * chain (members of 32 columns, parameter gradients fused): workgroups per
- * cluster (0: not used), rows per cluster, launches per call and LDS bytes per
- * workgroup. Returns the number of values
- * written, or -1 for invalid sizes. The plan depends on the current device's
- * CU count.
+ * cluster (0: not used), rows per cluster, launches per call, LDS bytes per
+ * workgroup, and unfolds between the moves of its gradient sums out of the
+ * registers (0: none). Returns the number of values written, or -1 for invalid
+ * sizes. The plan depends on the current device's CU count.
  */
-#define LTC_PLAN_FIELDS 37
+#define LTC_PLAN_FIELDS 38
 int ltc_launch_plan(int B, int T, int D, int H, int ode_unfolds, long long* out, int n);
 
 /*

@@ -4,6 +4,7 @@
 // stream. Allocates no device memory.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <string>
@@ -198,6 +199,17 @@ bool plan_cluster(ltc::Plan& p, int ncu) {
   return false;
 }
 
+// Chunks of rec_grad_kernel's sums over the N unfold instances: about 1024
+// workgroups, at least 32 instances each, at most 64 partials per synapse.
+long long rec_grad_chunks(const ltc::Plan& p) {
+  const long long bpc = (long long)(p.Hp / 64) * (p.Hp / 32);
+  long long nch = (1024 + bpc - 1) / bpc;
+  if (nch > 64) nch = 64;
+  const long long cap = (p.N + 31) / 32;
+  if (nch > cap) nch = cap;
+  return nch < 1 ? 1 : nch;
+}
+
 // Clusters of a launch, launches of a call, and whether each cluster's members
 // fit one XCD.
 void reg_cluster_counts(ltc::RegCluster& g, int B, int ncu) {
@@ -246,6 +258,19 @@ void plan_reg_forward(ltc::Plan& p, int ncu) {
   if (ltc::reg_fwd_lds(g, p.Hp) <= chain_lds_limit()) p.rf = g;
 }
 
+// A gradient sum kept over a whole launch is T * U * NB rounded additions long,
+// however small the batch, and what one row adds keeps its sign for long: the
+// sums move out of the registers, and start again, after as many unfolds as
+// make a quarter of the terms of one of rec_grad_kernel's partials (rec_grad_
+// chunks; half at Hp = 512, whose chains kept whole sums before too), and at
+// least kRegSumTerms. Largest 2-norm error of the w, mu and erev gradients
+// against float64, rec_grad_kernel / never moved / moved, in units of 1e-7: B2
+// T100 H192 2.9 / 9.6 / 3.0, B64 T32 H192 3.5 / 5.5 / 3.2, B300 T16 H256 4.7 /
+// 7.4 / 4.3, B128 T8 H384 3.9 / 5.6 / 3.0. A move costs about 2 us a launch
+// (12 slots; 4 with 16 or 20): those four steps took 1.9, 1.7, 2.3 and 0%
+// longer for it.
+constexpr int kRegSumTerms = 48;
+
 // The chain: members of 32 columns and 512 threads, whose registers hold the
 // operands and the four gradient sums of up to reg_chain_slots synapses per
 // thread: every one of a dense column up to Hp = 256, beyond that the synapses
@@ -269,6 +294,10 @@ void plan_reg_chain(ltc::Plan& p, int ncu) {
     if ((p.B + nb - 1) / nb <= slots) break;
   }
   reg_cluster_counts(g, p.B, ncu);
+  const long long nch = (g.RC == 32 ? 2 : 4) * rec_grad_chunks(p);
+  const long long terms = std::max<long long>((p.N + nch - 1) / nch, kRegSumTerms);
+  const long long fl = (terms + g.NB - 1) / g.NB;
+  g.FL = fl < (long long)p.T * p.U ? (int)fl : 0;
   if (ltc::reg_bwd_lds(g, p.Hp) <= chain_lds_limit()) p.rb = g;
 }
 
@@ -368,19 +397,13 @@ ltc::Plan make_plan_uncached(int B, int T, int D, int H, int U, int ncu, bool re
   p.LCH = p.LCHB = 1;
   plan_cluster(p, ncu);
   if (reg) plan_reg_clusters(p, ncu);
-  // Recurrent parameter-gradient chunks: about 1024 workgroups, at least 32
-  // unfold instances each, at most 64 partials per synapse.
+  // Recurrent parameter-gradient partials.
   if (p.FUSE) {
     // One partial per chain workgroup, or per chain cluster.
     p.NCH = p.CP > 0 ? p.NCLB : (B + p.NB - 1) / p.NB;
     if (p.NCH < 1) p.NCH = 1;
   } else {
-    const long long bpc = (long long)(p.Hp / 64) * (p.Hp / 32);
-    long long nch = (1024 + bpc - 1) / bpc;
-    if (nch > 64) nch = 64;
-    const long long cap = (p.N + 31) / 32;
-    if (nch > cap) nch = cap;
-    if (nch < 1) nch = 1;
+    const long long nch = rec_grad_chunks(p);
     const long long nper = (p.N + nch - 1) / nch;
     p.NCH = (int)(nper > 0 ? (p.N + nper - 1) / nper : 1);
     if (p.NCH < 1) p.NCH = 1;
@@ -475,10 +498,11 @@ void carve_cmp(const ltc::Plan& p, Carver& c, ltc::Prepped& pp, bool fwd, bool b
 }
 
 ltc::ClusterBuf carve_cluster(const ltc::Plan& p, Carver& c, bool bwd) {
-  ltc::ClusterBuf cb{nullptr, nullptr, g_spin.load(std::memory_order_relaxed)};
+  ltc::ClusterBuf cb{nullptr, nullptr, g_spin.load(std::memory_order_relaxed), nullptr};
   if (bwd ? ltc::bwd_clusters(p) : ltc::fwd_clusters(p)) {
     cb.xch = c.take<unsigned long long>(bwd ? ltc::cluster_words_bwd(p) : ltc::cluster_words(p));
     cb.status = c.take<int>(1);
+    if (bwd && p.rb.FL > 0) cb.gsum = c.take<float4>((long long)ltc::reg_grid(p.rb) * p.rb.RC * 512);
   }
   return cb;
 }
@@ -1710,7 +1734,7 @@ int ltc_launch_plan(int B, int T, int D, int H, int ode_unfolds, long long* out,
       ltc::row_bwd_fused(p) ? 1 : 0, ltc::row128_rec_fused(p) ? 1 : 0, p.LCH, p.LCHB,
       ltc::sens_full_list(p) ? 1 : 0,
       p.rf.CP, p.rf.JW, p.rf.NB, p.rf.L, p.rf.CP > 0 ? ltc::reg_fwd_lds(p.rf, p.Hp) : 0,
-      p.rb.CP, p.rb.NB, p.rb.L, p.rb.CP > 0 ? ltc::reg_bwd_lds(p.rb, p.Hp) : 0};
+      p.rb.CP, p.rb.NB, p.rb.L, p.rb.CP > 0 ? ltc::reg_bwd_lds(p.rb, p.Hp) : 0, p.rb.FL};
   const int m = n < LTC_PLAN_FIELDS ? n : LTC_PLAN_FIELDS;
   for (int i = 0; i < m; ++i) out[i] = v[i];
   return m;

@@ -229,6 +229,12 @@ __device__ __forceinline__ float4 image_load(__amdgpu_buffer_rsrc_t r, int lane_
                                                                            row_bytes, 0));
 }
 
+__device__ __forceinline__ void image_store(__amdgpu_buffer_rsrc_t r, int lane_bytes,
+                                            int row_bytes, const float4& v) {
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, lane_bytes, row_bytes, 0);
+}
+
 // Streams operand rows [r0, r0 + RC) of one image column (RC a multiple of 8)
 // through a double buffer of four rows, calling f(operand, row) for each row.
 // r0 must be wave-uniform. The prefetch past the chunk reads the next chunk's
@@ -4841,7 +4847,50 @@ struct BwdCK {
   // a column count exceeds maxcnt (too many synapses for the registers, or
   // kChainIrregular), and the other only when none does. 0: always run.
   int maxcnt;
+  // Register-resident chain: the gradient sums move to gsum every `flush`
+  // unfolds (0: never; RegCluster::FL).
+  float4* gsum;
+  int flush;
 };
+
+// A chain thread's gradient sums and their place in gsum, [workgroup][slot][512
+// threads]. LEAVE: what was moved there before (`moved`) plus the
+// registers' sums stays there, and the registers start again; else the total
+// comes back into the registers. Through a buffer resource made here: with
+// ordinary addresses the compiler forms every slot's once, outside the unfold
+// loop, and spills them (20 slots: 18 -> 61 registers).
+template <bool LEAVE, int N>
+__device__ __forceinline__ void move_sums(float4 (&gacc)[N], float4* gsum, bool moved) {
+  int g = blockIdx.x;
+  asm volatile("" : "+s"(g));
+  const __amdgpu_buffer_rsrc_t r = image_rsrc(gsum + (long long)g * N * 512, N * 512LL * 16);
+  int lane_bytes = threadIdx.x * 16;
+  asm volatile("" : "+v"(lane_bytes));
+  constexpr int G = N <= 16 ? 4 : 2;
+#pragma unroll
+  for (int q = 0; q < N; q += G) {
+    if (moved) {
+      float4 s[G];
+#pragma unroll
+      for (int i = 0; i < G; ++i) s[i] = image_load(r, lane_bytes + i * 8192, 0);
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        float4& a = gacc[q + i];
+        a = make_float4(a.x + s[i].x, a.y + s[i].y, a.z + s[i].z, a.w + s[i].w);
+      }
+    }
+    if (LEAVE) {
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        image_store(r, lane_bytes + i * 8192, 0, gacc[q + i]);
+        gacc[q + i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+    }
+    lane_bytes += G * 8192;
+    asm volatile("" : "+v"(lane_bytes));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
 
 // Whether every column of the chain image has at most `maxcnt` entries: the
 // same answer in every workgroup. Holds a workgroup barrier.
@@ -4968,7 +5017,7 @@ __device__ __forceinline__ bool not_finite(float al, float be) {
 // come from an LDS table [4][threads] of int4. Each slot's gradient sums go
 // to its synapse's place in the partial; synapses without an entry are
 // never written.
-template <int NB, int JW, int RCP, bool FUSE, int RCS = 0>
+template <int NB, int JW, int RCP, bool FUSE, int RCS = 0, bool MOVE = false>
 __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) {
   static_assert(!FUSE || RCP > 0 || RCS > 0, "the fused chain needs a compile-time row count");
   static_assert(RCS == 0 || (FUSE && JW == 32 && RCP == 0), "streamed fusion: 32-column members");
@@ -5128,6 +5177,8 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
   for (int b = 0; b < NB; ++b)
     cvi[b] = b0 + b < B ? k.vsave[(n_last * B + b0 + b) * Hp + sc] : 0.f;
 
+  // MOVE: the gradient sums move every k.flush unfolds (move_sums)
+  int fl = k.flush;
   for (long long n = n_last; n >= 0; --n) {
     const int t = (int)(n / U), u = (int)(n - (long long)t * U);
     // PF: the saved values that unfold n-1's alpha/beta need, in flight
@@ -5290,6 +5341,15 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
       if (tid == 0) __hip_atomic_store(k.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return;
     }
+    if constexpr (MOVE) {
+      if (--fl == 0 && n > 0) {
+        move_sums<true>(gacc, k.gsum, n + k.flush <= n_last);
+        fl = k.flush;
+      }
+    }
+  }
+  if constexpr (MOVE) {
+    move_sums<false>(gacc, k.gsum, true);
   }
   if (live) {
     if (k.gstate != nullptr && c < H) k.gstate[(long long)(b0 + bo) * H + c] = g;
@@ -5372,7 +5432,7 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
 // synapses left out have weight zero, and zero times it is NaN, so dL/dv of
 // every neuron of that row that has such a synapse becomes NaN. A row flag by
 // unfold parity carries it, as the forward's does a NaN state.
-template <int NB, int RCP = 16, bool FACT = true, bool REG = false>
+template <int NB, int RCP = 16, bool FACT = true, bool REG = false, bool MOVE = false>
 __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   static_assert(NB == 2 || NB == 4 || NB == 8, "two groups of rows");
   constexpr int JW = 32, HB = NB / 2, PER = NB * JW, PERG = HB * JW;
@@ -5564,6 +5624,8 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   float gnext = 0.f;
   // step t, unfold u within it and n mod 3, stepped with n
   int t = T - 1, u = U - 1, n3 = (int)(n_last % 3);
+  // MOVE: the gradient sums move every k.flush unfolds (move_sums)
+  int fl = k.flush;
   for (long long n = n_last; n >= 0; --n) {
 #pragma unroll
     for (int gi = 0; gi < 2; ++gi) {
@@ -5741,6 +5803,12 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
         pend = true;
       }
     }
+    if constexpr (MOVE) {
+      if (--fl == 0 && n > 0) {
+        move_sums<true>(gacc, k.gsum, n + k.flush <= n_last);
+        fl = k.flush;
+      }
+    }
     n3 = mod3_prev(n3);
     if (--u < 0) {
       u = U - 1;
@@ -5775,6 +5843,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   asm volatile("" : "+v"(sks_end));
   // REG: sum dl*v from sum dl*(x*v + y)
   if constexpr (REG) {
+    if constexpr (MOVE) move_sums<false>(gacc, k.gsum, true);
 #pragma unroll
     for (int rr = 0; rr < RCP; ++rr)
       gacc[rr].w = fabsf(preg[rr].x) < kMinSlope
@@ -5950,9 +6019,8 @@ hipError_t fwd_cl_by_rcp(const Plan& p, const FwdCK& a, hipStream_t s) {
 template <int NB>
 hipError_t launch_reg_fwd(const Plan& p, FwdCK a, hipStream_t s) {
   const RegCluster& g = p.rf;
-  const int rounds = (g.NCL + 7) / 8 * 8;
   a.xcd_local = g.xcd ? 1 : 0;
-  const dim3 grid((g.xcd ? rounds : g.NCL) * g.CP), block(1024);
+  const dim3 grid(reg_grid(g)), block(1024);
   const size_t lds = (size_t)reg_fwd_lds(g, p.Hp);
   if constexpr (NB == 1) {
     if (g.RC > (g.JW == 64 ? 20 : 16)) return hipErrorInvalidConfiguration;
@@ -5969,38 +6037,45 @@ hipError_t launch_reg_fwd(const Plan& p, FwdCK a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int NB>
-hipError_t launch_reg_bwd(const Plan& p, BwdCK a, hipStream_t s) {
+template <int NB, bool MOVE>
+hipError_t launch_reg_bwd_mv(const Plan& p, BwdCK a, hipStream_t s) {
   const RegCluster& g = p.rb;
-  const int rounds = (g.NCL + 7) / 8 * 8;
-  const dim3 grid((g.xcd ? rounds : g.NCL) * g.CP), block(512);
+  const dim3 grid(reg_grid(g)), block(512);
   const size_t lds = (size_t)reg_bwd_lds(g, p.Hp);
   if (g.RC == 12 || g.RC == 16) {
     if (g.RC == 12)
-      LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 12, false, true>), grid, block, lds, s, a);
+      LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 12, false, true, MOVE>), grid, block, lds, s, a);
     else
-      LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 16, false, true>), grid, block, lds, s, a);
+      LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 16, false, true, MOVE>), grid, block, lds, s, a);
     return hipGetLastError();
   }
   // The kernel over at most reg_chain_slots synapses a thread, then the one
   // that streams them all: one of the two leaves at its first check.
   a.maxcnt = 16 * reg_chain_slots(g.RC);
   if (reg_chain_slots(g.RC) == 16)
-    LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 16, true, true>), grid, block, lds, s, a);
+    LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 16, true, true, MOVE>), grid, block, lds, s, a);
   else
-    LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 20, true, true>), grid, block, lds, s, a);
+    LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 20, true, true, MOVE>), grid, block, lds, s, a);
   const size_t lds2 = (size_t)std::max(cluster_chain_lds(NB, p.Hp, 16, 32, false),
                                        partial_tile_lds(p.Hp));
   a.xcd_local = 0;  // streamed operands: members spread over the XCDs (cluster_coords)
   const dim3 grid2(g.NCL * g.CP);
+#define LTC_STREAM(R) \
+  case R: LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, R, MOVE>), grid2, block, lds2, s, a); break
   switch (g.RC) {
-    case 20: LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, 20>), grid2, block, lds2, s, a); break;
-    case 24: LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, 24>), grid2, block, lds2, s, a); break;
-    case 28: LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, 28>), grid2, block, lds2, s, a); break;
-    case 32: LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, 32>), grid2, block, lds2, s, a); break;
+    LTC_STREAM(20);
+    LTC_STREAM(24);
+    LTC_STREAM(28);
+    LTC_STREAM(32);
     default: return hipErrorInvalidConfiguration;
   }
+#undef LTC_STREAM
   return hipGetLastError();
+}
+
+template <int NB>
+hipError_t launch_reg_bwd(const Plan& p, const BwdCK& a, hipStream_t s) {
+  return p.rb.FL > 0 ? launch_reg_bwd_mv<NB, true>(p, a, s) : launch_reg_bwd_mv<NB, false>(p, a, s);
 }
 
 template <int NB>
@@ -6224,7 +6299,8 @@ hipError_t launch_ode_bwd(const Plan& p, const Prepped& pp, const float* vsave,
     const RegCluster& g = p.rb;
     BwdCK a{pp.recB, pp.neuron, vsave, densave, gout, gs, ghfin, absave, dsn, dsd, npart,
             gstate, rpart, cb.xch, cb.status, cb.spin, p.B, p.T, p.H, p.Hp, p.U, g.KS, g.RC,
-            g.CP, g.xcd ? 1 : 0, pp.cB, pp.cBi, pp.cBn, 0, g.NCL, 0};
+            g.CP, g.xcd ? 1 : 0, pp.cB, pp.cBi, pp.cBn, 0, g.NCL, 0, cb.gsum, g.FL};
+    if (g.FL > 0 && cb.gsum == nullptr) return hipErrorInvalidValue;
     for (int l = 0; l < g.L; ++l) {
       hipError_t e = clear_cluster(p, cb, true, s, l == 0);
       if (e != hipSuccess) return e;
@@ -6244,7 +6320,7 @@ hipError_t launch_ode_bwd(const Plan& p, const Prepped& pp, const float* vsave,
     const int xl = (chain_prefetches(p) && p.NCLB % 8 == 0) ? 1 : 0;
     BwdCK a{pp.recB, pp.neuron, vsave, densave, gout, gs, ghfin, absave, dsn, dsd, npart,
             gstate, rpart, cb.xch, cb.status, cb.spin, p.B, p.T, p.H, p.Hp, p.U, p.KSB, p.RCB,
-            p.CPB, xl, pp.cB, pp.cBi, pp.cBn, 0, p.NCLB, 0};
+            p.CPB, xl, pp.cB, pp.cBi, pp.cBn, 0, p.NCLB, 0, nullptr, 0};
     if (cmp_bwd(p) && (pp.cB == nullptr || pp.cBi == nullptr || pp.cBn == nullptr))
       return hipErrorInvalidValue;
     for (int l = 0; l < p.LCHB; ++l) {

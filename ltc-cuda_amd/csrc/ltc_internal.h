@@ -68,10 +68,18 @@ enum KernelId : int {
 // launches per call, each taking the next NCL * NB rows.
 // With xcd set every member of a cluster runs on one XCD (the grid, padded to
 // whole rounds of eight clusters, still holds at most one workgroup per CU).
+// FL (chain): unfolds after which the gradient sums move from the registers to
+// ClusterBuf::gsum, 0 for never.
 struct RegCluster {
-  int CP, JW, KS, RC, NB, NCL, L;
+  int CP, JW, KS, RC, NB, NCL, L, FL;
   bool xcd;
 };
+
+// Workgroups of a register-resident launch: with every cluster on one XCD the
+// grid is padded to whole rounds of eight clusters.
+inline int reg_grid(const RegCluster& g) {
+  return (g.xcd ? (g.NCL + 7) / 8 * 8 : g.NCL) * g.CP;
+}
 
 // Shapes and launch choices shared by every kernel of one call.
 struct Plan {
@@ -298,10 +306,13 @@ hipError_t launch_sens_fwd_ln(const Plan& p, const float* x, Strides3 xs, const 
 // cluster member gave up waiting for its partners), plus the wait budget of
 // every exchange in ticks of the 100 MHz wall clock (<= 0: a member gives up
 // at its first wait, which the tests use to force the give-up path).
+// gsum: the register-resident chain's moved gradient sums, [workgroup][slot]
+// [512 threads], null unless the plan moves them (RegCluster::FL).
 struct ClusterBuf {
   unsigned long long* xch;
   int* status;
   long long spin;
+  float4* gsum;
 };
 // Default wait budget: 0.2 s.
 constexpr long long kDefaultSpinTicks = 20000000;

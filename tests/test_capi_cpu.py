@@ -482,3 +482,18 @@ def test_register_resident_cluster_plan(capi, B, H):
     assert L == -(-B // (nb * min(slots, -(-B // nb))))
     assert L == 1 or nb == 8
     assert p["reg_fwd_lds"] <= 159 * 1024
+
+
+@pytest.mark.parametrize("H", [192, 256, 320, 448, 512])
+@pytest.mark.parametrize("B,T", [(1, 1), (2, 100), (64, 32), (300, 16), (4096, 2)])
+def test_chain_sums_are_bounded(capi, B, T, H):
+    """A register sum of the chain takes at most as many terms as a partial of the
+    separate gradient pass would, or 48 and the rest of its last unfold."""
+    p = capi.plan(B, T, 8, H, 6)
+    if p["reg_bwd_members"] == 0:
+        return
+    nb, fl, n = p["reg_bwd_rows"], p["reg_bwd_move"], B * T * 6
+    terms = nb * (fl if fl else T * 6)
+    parts = max(1, min(64, -(-1024 // ((p["Hp"] // 64) * (p["Hp"] // 32))), -(-n // 32)))
+    assert terms <= max(48, -(-n // parts)) + nb
+    assert fl == 0 or 48 <= nb * fl and fl < T * 6

@@ -270,3 +270,29 @@ def test_gradients_at_a_vanishing_slope(shape, sigma, mu):
         ref = r_g[n][3, 4].item()
         # a float32 sum of a few hundred terms whose signs differ
         assert abs(got - ref) <= 1e-4 * abs(ref) + 1e-30, (n, got, ref)
+
+
+@pytest.mark.parametrize("shape", [(2, 100, 8, 192, 0.5), (2, 100, 8, 192, 1.0), (2, 100, 8, 320, 0.5),
+                                   (3, 60, 8, 320, 1.0), (1, 100, 8, 448, 0.5), (2, 60, 8, 512, 1.0)],
+                         ids=lambda s: "B%dT%dD%dH%dp%g" % s)
+def test_gradient_sums_of_long_sequences(shape):
+    """Hundreds of unfolds of a few rows: the recurrent sums move out of the
+    registers on the way, so their error is that of sums of some 50 terms and of
+    as many such sums (2.1 to 3.3e-7; 4.6 to 10e-7 in one sum each)."""
+    B, T, D, H, density = shape
+    p = ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)
+    assert 0 < p["reg_bwd_move"] < T * 6
+    m = _perturbed_module(D, H, seed=B + H, sparsity=density).to(DEV)
+    g = torch.Generator().manual_seed(21)
+    x = torch.randn(B, T, D, generator=g)
+    h0 = torch.randn(B, H, generator=g) * 0.2
+    G = torch.randn(B, T, H, generator=g)
+    hg = h0.to(DEV)
+    out, _ = m(x.to(DEV), (hg, hg))
+    (out * G.to(DEV)).sum().backward()
+    _, _, r_g, _, _ = _oracle_module_grads(m, x, h0, G, torch.zeros(B, H))
+    for n in ("w", "erev", "mu"):
+        q = dict(m.named_parameters())[n].grad.cpu().double()
+        err = ((q - r_g[n]).norm() / r_g[n].norm()).item()
+        print(f"{shape} {n}: {err:.2e}", flush=True)
+        assert err <= 4.3e-7, f"{n}: {err:.1e}"
