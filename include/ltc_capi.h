@@ -340,6 +340,10 @@ int ltc_launch_plan(int B, int T, int D, int H, int ode_unfolds, long long* out,
  * needed), the whole cluster leaves early, and the call then overwrites
  * every output it writes (out, h_final and saved for a forward; every
  * gradient for a backward) with NaN and raises a sticky per-device fault flag.
+ * For 128 < H <= 192, and for larger batches at 192 < H <= 512 (plan field CP
+ * = 0: the plan itself has no clusters), nothing is lost instead: kernels that
+ * wait on nobody are queued behind the clusters and make the results, and no
+ * flag is raised.
  * The module-path backward with one batch row per workgroup and B <= 64 also
  * runs companion workgroups that wait for the chain workgroups the same
  * bounded way, with the same outcome (every gradient, dL/dx and dL/dh0 NaN,

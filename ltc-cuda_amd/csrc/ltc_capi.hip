@@ -212,8 +212,8 @@ long long rec_grad_chunks(const ltc::Plan& p) {
 
 // Clusters of a launch, launches of a call, and whether each cluster's members
 // fit one XCD.
-void reg_cluster_counts(ltc::RegCluster& g, int B, int ncu) {
-  const int need = (B + g.NB - 1) / g.NB, slots = ncu / g.CP;
+void reg_cluster_counts(ltc::RegCluster& g, int B, int slots, int ncu) {
+  const int need = (B + g.NB - 1) / g.NB;
   g.NCL = need < slots ? need : slots;
   g.L = (B + g.NCL * g.NB - 1) / (g.NCL * g.NB);
   g.xcd = (g.NCL + 7) / 8 * 8 * g.CP <= ncu;
@@ -254,7 +254,7 @@ void plan_reg_forward(ltc::Plan& p, int ncu) {
       if ((p.B + nb - 1) / nb <= slots) break;
     }
   }
-  reg_cluster_counts(g, p.B, ncu);
+  reg_cluster_counts(g, p.B, ncu / g.CP, ncu);
   if (ltc::reg_fwd_lds(g, p.Hp) <= chain_lds_limit()) p.rf = g;
 }
 
@@ -287,13 +287,15 @@ void plan_reg_chain(ltc::Plan& p, int ncu) {
   g.CP = p.Hp / 32;
   g.KS = 16;
   g.RC = p.Hp / 16;
-  const int slots = ncu / g.CP;
+  // one gradient partial per cluster, at most the 64 that the finalize sums
+  // without a first pass
+  const int slots = std::min(ncu / g.CP, 64);
   if (slots < 1) return;
   for (int nb : {2, 4, 8}) {
     g.NB = nb;
     if ((p.B + nb - 1) / nb <= slots) break;
   }
-  reg_cluster_counts(g, p.B, ncu);
+  reg_cluster_counts(g, p.B, slots, ncu);
   const long long nch = (g.RC == 32 ? 2 : 4) * rec_grad_chunks(p);
   const long long terms = std::max<long long>((p.N + nch - 1) / nch, kRegSumTerms);
   const long long fl = (terms + g.NB - 1) / g.NB;
@@ -565,13 +567,14 @@ BwdWs carve_bwd(const ltc::Plan& p, Carver& c, bool images = true) {
     // the forward's as well: the per-step backward recomputes a forward unfold
     carve_cmp(p, c, w.pp, true, true);
   }
-  w.absave = ltc::chain_fused(p) ? nullptr : c.take<float2>(p.N * p.Hp);
+  w.absave = ltc::chain_fused(p) && !ltc::bwd_after(p) ? nullptr : c.take<float2>(p.N * p.Hp);
   w.dsn = c.take<float>((long long)p.B * p.T * p.Hp);
   w.dsd = c.take<float>((long long)p.B * p.T * p.Hp);
   w.npart = c.take<float>((long long)p.B * 3 * p.Hp);
   // recurrent partials: NCH chunks, or one per batch row (Hp = 128 chain with
   // recurrent-gradient companions)
-  const long long nch = ltc::row128_rec_fused(p) && p.B > p.NCH ? p.B : ltc::rec_parts(p);
+  long long nch = ltc::row128_rec_fused(p) && p.B > p.NCH ? p.B : ltc::rec_parts(p);
+  if (ltc::bwd_after(p) && p.NCH > nch) nch = p.NCH;
   w.rpart = c.take<float>(nch * 4 * p.Hp * p.Hp);
   // sensory partials: NRC row chunks, or one per batch row (fused row backward,
   // or the sensory companions of the Hp = 128 chain)
@@ -785,6 +788,56 @@ ltc::FillList poison_list(const ltc::ClusterBuf& cb) {
   return fl;
 }
 
+// The ODE forward of a call: the plan's launch, and behind register-resident
+// clusters the plan's own kernels where it has no clusters (fwd_after).
+hipError_t ode_forward(const ltc::Plan& p, const ltc::Prepped& pp, const float* sn,
+                       const float* sd, const float* state, float epsilon, float* out,
+                       float* h_final, float* vsave, float* densave, const ltc::ClusterBuf& cb,
+                       hipStream_t s) {
+  hipError_t e = ltc::launch_ode_fwd(p, pp, sn, sd, state, epsilon, out, h_final, vsave, densave,
+                                     cb, s);
+  if (e == hipSuccess && ltc::fwd_after(p))
+    e = ltc::launch_ode_fwd_after(ltc::own_plan(p), pp, sn, sd, state, epsilon, out, h_final,
+                                  vsave, densave, cb, cb.status, s);
+  return e;
+}
+
+// The chain of a backward and, when it does not form them itself, the recurrent
+// gradient sums; behind register-resident clusters the plan's own kernels where
+// it has no clusters (bwd_after). mask: launch_rec_grad's.
+int ode_backward(const ltc::Plan& p, const BwdWs& w, const float* vsave, const float* densave,
+                 const float* gout, ltc::Strides3 gs, const float* ghfin, float* gstate,
+                 const float* mask, hipStream_t s) {
+  hipError_t e = timed(ltc::K_ODE_BWD, s, [&] {
+    hipError_t r = ltc::launch_ode_bwd(p, w.pp, vsave, densave, gout, gs, ghfin, w.absave, w.dsn,
+                                       w.dsd, w.npart, gstate, w.rpart, w.cb, s);
+    if (r == hipSuccess && ltc::bwd_after(p))
+      r = ltc::launch_ode_bwd_after(ltc::own_plan(p), w.pp, vsave, densave, gout, gs, ghfin,
+                                    w.absave, w.dsn, w.dsd, w.npart, gstate, w.rpart, w.cb,
+                                    w.cb.status, s);
+    return r;
+  });
+  if (e != hipSuccess) return hip_fail("ODE backward launch", e);
+  if (!ltc::chain_fused(p) || ltc::bwd_after(p)) {
+    e = timed(ltc::K_REC_GRAD, s, [&] {
+      return ltc::launch_rec_grad(p, w.pp, vsave, w.absave, w.rpart, s, mask,
+                                  ltc::bwd_after(p) ? w.cb.status : nullptr);
+    });
+    if (e != hipSuccess) return hip_fail("recurrent gradient launch", e);
+  }
+  return LTC_OK;
+}
+
+// The recurrent partials of the finalize after ode_backward.
+ltc::RecParts rec_parts_after(const ltc::Plan& p, const BwdWs& w) {
+  return ltc::bwd_after(p) ? ltc::RecParts{w.cb.status, p.NCH} : ltc::RecParts{nullptr, 0};
+}
+
+// Whether a give-up ends in NaN outputs (poison_list): the clusters ran and
+// nothing runs behind them.
+bool fwd_poisons(const ltc::Plan& p) { return ltc::fwd_clusters(p) && !ltc::fwd_after(p); }
+bool bwd_poisons(const ltc::Plan& p) { return ltc::bwd_clusters(p) && !ltc::bwd_after(p); }
+
 // Device address of this device's scratch array (looked up on the first call
 // on each device, with that device current); nullptr after a failed lookup,
 // with the message set.
@@ -900,11 +953,11 @@ int full_forward(bool reg, const float* x, long long sxb, long long sxt, long lo
   e = timed(ltc::K_SENS_FWD, s, [&] { return ltc::launch_sens_fwd(p, x, xs, w.pp, w.sn, w.sd, s); });
   if (e != hipSuccess) return hip_fail("sensory forward launch", e);
   e = timed(ltc::K_ODE_FWD, s, [&] {
-    return ltc::launch_ode_fwd(p, w.pp, w.sn, w.sd, state, epsilon, out, h_final, vsave, densave,
+    return ode_forward(p, w.pp, w.sn, w.sd, state, epsilon, out, h_final, vsave, densave,
                                w.cb, s);
   });
   if (e != hipSuccess) return hip_fail("ODE forward launch", e);
-  if (ltc::fwd_clusters(p)) {
+  if (fwd_poisons(p)) {
     ltc::FillList fl = poison_list(w.cb);
     ltc::fill_add(fl, out, nullptr, (long long)B * T * H);
     ltc::fill_add(fl, h_final, nullptr, (long long)B * H);
@@ -1027,16 +1080,8 @@ int ltc_full_backward(const float* x, long long sxb, long long sxt, long long sx
   hipError_t e;
   e = timed(ltc::K_PREP, s, [&] { return ltc::launch_prep(p, rp, w.pp, true, s); });
   if (e != hipSuccess) return hip_fail("prep launch", e);
-  e = timed(ltc::K_ODE_BWD, s, [&] {
-    return ltc::launch_ode_bwd(p, w.pp, vsave, densave, grad_out, gs, grad_h_final, w.absave,
-                               w.dsn, w.dsd, w.npart, grad_state, w.rpart, w.cb, s);
-  });
-  if (e != hipSuccess) return hip_fail("ODE backward launch", e);
-  if (!ltc::chain_fused(p)) {
-    e = timed(ltc::K_REC_GRAD, s,
-              [&] { return ltc::launch_rec_grad(p, w.pp, vsave, w.absave, w.rpart, s); });
-    if (e != hipSuccess) return hip_fail("recurrent gradient launch", e);
-  }
+  rc = ode_backward(p, w, vsave, densave, grad_out, gs, grad_h_final, grad_state, nullptr, s);
+  if (rc != LTC_OK) return rc;
   e = timed(ltc::K_SENS_BWD, s, [&] {
     return ltc::launch_sens_bwd(p, x, xs, w.pp, w.dsn, w.dsd, w.spart, w.dxpart, s);
   });
@@ -1044,10 +1089,11 @@ int ltc_full_backward(const float* x, long long sxb, long long sxt, long long sx
   ltc::Plan pf = p;
   pf.NCH = ltc::rec_parts(p);
   e = timed(ltc::K_FINALIZE, s, [&] {
-    return ltc::launch_finalize(pf, rp, w.rpart, w.spart, w.dxpart, w.npart, w.ps, go, s);
+    return ltc::launch_finalize(pf, rp, w.rpart, w.spart, w.dxpart, w.npart, w.ps, go, s,
+                                ltc::kFinAll, rec_parts_after(p, w));
   });
   if (e != hipSuccess) return hip_fail("finalize launch", e);
-  if (ltc::bwd_clusters(p)) {
+  if (bwd_poisons(p)) {
     ltc::FillList fl = poison_list(w.cb);
     ltc::fill_add(fl, grad_x, nullptr, (long long)B * T * D);
     ltc::fill_add(fl, grad_state, nullptr, (long long)B * H);
@@ -1189,11 +1235,11 @@ int ltc_module_forward(const float* x, long long sxb, long long sxt, long long s
     if (e != hipSuccess) return hip_fail("sensory forward launch", e);
   }
   e = timed(ltc::K_ODE_FWD, s, [&] {
-    return ltc::launch_ode_fwd(p, pp, wfw.sn, wfw.sd, state, epsilon, out, h_final, vsave,
+    return ode_forward(p, pp, wfw.sn, wfw.sd, state, epsilon, out, h_final, vsave,
                                densave, wfw.cb, s);
   });
   if (e != hipSuccess) return hip_fail("ODE forward launch", e);
-  if (ltc::fwd_clusters(p)) {
+  if (fwd_poisons(p)) {
     ltc::FillList fl = poison_list(wfw.cb);
     ltc::fill_add(fl, out, nullptr, (long long)B * T * H);
     ltc::fill_add(fl, h_final, nullptr, (long long)B * H);
@@ -1314,17 +1360,8 @@ int ltc_module_backward(const float* x, long long sxb, long long sxt, long long 
     if (sens_comp) pf.NRC = p.B;
     status = reinterpret_cast<const int*>(words + ltc::row_bwd_words(p) - 1);
   } else {
-    e = timed(ltc::K_ODE_BWD, s, [&] {
-      return ltc::launch_ode_bwd(p, wb.pp, vsave, densave, grad_out, gs, grad_h_final,
-                                 wb.absave, wb.dsn, wb.dsd, wb.npart, grad_state, wb.rpart, wb.cb,
-                                 s);
-    });
-    if (e != hipSuccess) return hip_fail("ODE backward launch", e);
-    if (!ltc::chain_fused(p)) {
-      e = timed(ltc::K_REC_GRAD, s,
-                [&] { return ltc::launch_rec_grad(p, wb.pp, vsave, wb.absave, wb.rpart, s, lp.mask); });
-      if (e != hipSuccess) return hip_fail("recurrent gradient launch", e);
-    }
+    rc = ode_backward(p, wb, vsave, densave, grad_out, gs, grad_h_final, grad_state, lp.mask, s);
+    if (rc != LTC_OK) return rc;
   }
   if (!sens_comp) {
     e = timed(ltc::K_SENS_BWD, s, [&] {
@@ -1340,10 +1377,10 @@ int ltc_module_backward(const float* x, long long sxb, long long sxt, long long 
   }
   e = timed(ltc::K_FINALIZE, s, [&] {
     return ltc::launch_finalize_leaf(pf, lp, wb.rpart, wb.spart, wb.npart, lnpart, wb.ps, lg, s,
-                                     status, grad_state);
+                                     status, grad_state, rec_parts_after(p, wb));
   });
   if (e != hipSuccess) return hip_fail("finalize launch", e);
-  if (ltc::bwd_clusters(p)) {
+  if (bwd_poisons(p)) {
     ltc::FillList fl = poison_list(wb.cb);
     ltc::fill_add(fl, grad_x, nullptr, (long long)B * T * D);
     ltc::fill_add(fl, grad_state, nullptr, (long long)B * H);
@@ -1592,7 +1629,7 @@ int ltc_ode_unfold_fwd(const float* state, const float* w_pos, const float* w_er
   // T = 1: the kernel's (B,T,H) output and its final state are the same (B,H)
   // values, written by the same thread.
   e = timed(ltc::K_ODE_FWD, s, [&] {
-    return ltc::launch_ode_fwd(p, w.f.pp, w.f.sn, w.f.sd, state, epsilon, state_out, state_out,
+    return ode_forward(p, w.f.pp, w.f.sn, w.f.sd, state, epsilon, state_out, state_out,
                                vsave, densave, w.f.cb, s);
   });
   if (e != hipSuccess) return hip_fail("ODE forward launch", e);
@@ -1600,7 +1637,7 @@ int ltc_ode_unfold_fwd(const float* state, const float* w_pos, const float* w_er
     e = ltc::launch_copy_rows(vsave, p.Hp, v_buffer, H, (long long)ode_unfolds * B, H, s);
     if (e != hipSuccess) return hip_fail("copy launch", e);
   }
-  if (ltc::fwd_clusters(p)) {
+  if (fwd_poisons(p)) {
     ltc::FillList fl = poison_list(w.f.cb);
     ltc::fill_add(fl, state_out, nullptr, (long long)B * H);
     ltc::fill_add(fl, v_buffer, nullptr, save_intermediates ? (long long)ode_unfolds * B * H : 0);
@@ -1672,22 +1709,14 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
   // reference's backward kernels recompute each unfold from its saved
   // pre-state, csrc/ltc_kernels.cu:549-668).
   e = timed(ltc::K_ODE_FWD, s, [&] {
-    return ltc::launch_ode_fwd(p, w.b.pp, w.f.sn, w.f.sd, v_buffer, epsilon, w.hscr, w.hscr,
+    return ode_forward(p, w.b.pp, w.f.sn, w.f.sd, v_buffer, epsilon, w.hscr, w.hscr,
                                vsave, densave, w.f.cb, s);
   });
   if (e != hipSuccess) return hip_fail("ODE forward launch", e);
   // dL/dv^U enters as the output gradient of the single step.
   const ltc::Strides3 gs{H, 0, 1};
-  e = timed(ltc::K_ODE_BWD, s, [&] {
-    return ltc::launch_ode_bwd(p, w.b.pp, vsave, densave, grad_output, gs, nullptr, w.b.absave,
-                               w.b.dsn, w.b.dsd, w.b.npart, grad_v, w.b.rpart, w.b.cb, s);
-  });
-  if (e != hipSuccess) return hip_fail("ODE backward launch", e);
-  if (!ltc::chain_fused(p)) {
-    e = timed(ltc::K_REC_GRAD, s,
-              [&] { return ltc::launch_rec_grad(p, w.b.pp, vsave, w.b.absave, w.b.rpart, s); });
-    if (e != hipSuccess) return hip_fail("recurrent gradient launch", e);
-  }
+  rc = ode_backward(p, w.b, vsave, densave, grad_output, gs, nullptr, grad_v, nullptr, s);
+  if (rc != LTC_OK) return rc;
   e = ltc::launch_copy_rows(w.b.dsn, p.Hp, grad_w_num_sensory, H, B, H, s);
   if (e == hipSuccess) e = ltc::launch_copy_rows(w.b.dsd, p.Hp, grad_w_den_sensory, H, B, H, s);
   if (e != hipSuccess) return hip_fail("copy launch", e);
@@ -1695,14 +1724,14 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
   pf.NCH = ltc::rec_parts(p);
   e = timed(ltc::K_FINALIZE, s, [&] {
     return ltc::launch_finalize(pf, rp, w.b.rpart, nullptr, nullptr, w.b.npart, w.b.ps, go, s,
-                                ltc::kFinRec);
+                                ltc::kFinRec, rec_parts_after(p, w.b));
   });
   if (e != hipSuccess) return hip_fail("finalize launch", e);
   {
     // Either the recompute (forward) or the chain may have given up; both
     // status words gate the same fill.
     for (const ltc::ClusterBuf* cb : {&w.f.cb, &w.b.cb}) {
-      if (cb->status == nullptr) continue;  // no clusters in that launch
+      if (!(cb == &w.f.cb ? fwd_poisons(p) : bwd_poisons(p))) continue;
       ltc::FillList fl = poison_list(*cb);
       for (float* z : {grad_v, grad_w_num_sensory, grad_w_den_sensory})
         ltc::fill_add(fl, z, nullptr, (long long)B * H);

@@ -58,6 +58,13 @@ __device__ __forceinline__ unsigned long long xch_get(unsigned long long* w) {
   return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Whether a launch gated by a status word has to run: always without a word,
+// else when the word is set.
+__device__ __forceinline__ bool gate_open(const int* status) {
+  return status == nullptr ||
+         __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+
 // sigmoid(z) for zp = -z*log2(e). v_exp_f32 saturates to +inf for large zp
 // and rcp(inf) = 0, while exp2 of a large negative zp is 0 and rcp(1) = 1, so
 // both saturated limits are exact and a*(1-a) is 0 there (never inf/inf).
@@ -823,6 +830,7 @@ struct FwdK {
   const float4* cimg;
   const int* cidx;
   const int* ccnt;
+  const int* gate;  // AFTER: the status word of the clusters before this launch
 };
 
 template <int NB>
@@ -926,8 +934,12 @@ __device__ __forceinline__ void fwd_synapses_cmp(const float4* p, const float* v
 // around unused pairs), the state sits in LDS as [Hp][NB] so that a slot's NB
 // values are one read at a per-lane row, and the slot row offsets stay in
 // registers (no table read before a slot pair's state reads).
-template <int NB, int RCP>
+//
+// AFTER: behind register-resident clusters whose members gave up waiting, this
+// launch makes the call's results instead; otherwise it leaves at once.
+template <int NB, int RCP, bool AFTER = false>
 __global__ __launch_bounds__(ode_max_threads(NB)) void ode_fwd_kernel(FwdK k) {
+  if (AFTER && !gate_open(k.gate)) return;
   constexpr int MO = ode_owned_rows(NB);
   constexpr bool CMP = RCP > 0;
   extern __shared__ float4 lds4[];
@@ -1105,6 +1117,7 @@ struct BwdK {
   // dsd; the Hp = 128 chain with recurrent-gradient companions sends each
   // unfold's alpha/beta as [B][T*U][2][128] words instead of into absave.
   unsigned long long* rbw;
+  const int* gate;  // AFTER: the status word of the clusters before this launch
 };
 
 // The recurrent-gradient companions of the Hp = 128 chain: the forward image
@@ -1236,9 +1249,14 @@ __device__ __forceinline__ void bwd_load_gout(const BwdK& k, int t, int b0, int 
 // synapse). Thread (o, ks) holds the entries ks, ks + KS, ... of column o,
 // alpha/beta sit in LDS as [Hp][NB], and the slot row offsets come from an
 // LDS table [RCP/4][threads] of int4.
-template <int NB, int RCP, bool FUSE>
+//
+// AFTER: as in ode_fwd_kernel. The clusters' image is not folded: the operands
+// are folded here as they arrive.
+template <int NB, int RCP, bool FUSE, bool AFTER = false>
 __global__ __launch_bounds__(ode_max_threads(NB)) void ode_bwd_kernel(BwdK k) {
   static_assert(!FUSE || RCP > 0, "fused gradients need register-resident operands");
+  static_assert(!AFTER || RCP == 0, "the launch behind clusters streams its operands");
+  if (AFTER && !gate_open(k.gate)) return;
   constexpr int MO = ode_owned_rows(NB);
   constexpr bool CMP = !FUSE && RCP > 0;
   extern __shared__ float4 lds4[];
@@ -1357,7 +1375,8 @@ __global__ __launch_bounds__(ode_max_threads(NB)) void ode_bwd_kernel(BwdK k) {
         }
       } else {
         // Streamed (folded) operands, double-buffered four at a time.
-        stream_rows(rsB, o * 16, r0, RC, Hp, [&](const float4 p, int r) {
+        stream_rows(rsB, o * 16, r0, RC, Hp, [&](float4 p, int r) {
+          if (AFTER) p = make_float4(p.x, p.y, p.x * p.z, p.x * p.w);
           bwd_synapse_folded<NB>(p, ab, Hp, r, cvi, acc);
         });
       }
@@ -2598,6 +2617,7 @@ struct RecGK {
   float* rpart;
   int H, Hp;
   long long N, nper;
+  const int* gate;  // behind clusters: run only when their status word is set
 };
 
 template <int NS>
@@ -2771,6 +2791,7 @@ __device__ __forceinline__ void rec_grad_dense(const RecGK& k, float (*vsh)[32],
 }
 
 __global__ __launch_bounds__(256) void rec_grad_kernel(RecGK k) {
+  if (!gate_open(k.gate)) return;
   __shared__ __align__(16) float vsh[RG_NT][32];
   __shared__ __align__(16) float2 absh[RG_NT][64];
   __shared__ unsigned short list[32 * 64];
@@ -3239,7 +3260,13 @@ struct FinK {
   GradOut g;
   int B, D, H, Hp, Dp, NCH, NRC, HB, BT;  // B, NCH: counts of neuron / recurrent partials
   long long base, count;
+  RecParts rec;
 };
+
+// Recurrent partials the finalize sums: those of the launch that ran.
+__device__ __forceinline__ int rec_count(const RecParts& r, int nch) {
+  return r.status != nullptr && gate_open(r.status) ? r.nch : nch;
+}
 
 // Sum of n strided partials with 8 loads in flight per round.
 __device__ __forceinline__ float sum_partials(const float* p, long long stride, int n) {
@@ -3304,7 +3331,7 @@ __global__ __launch_bounds__(256) void finalize_kernel(FinK k) {
     const long long HH = (long long)Hp * Hp;
     const float* src = k.rpart + (long long)i * Hp + j;
     float sp[4];
-    sum_partials_planes<4>(src, HH, 4 * HH, k.NCH, sp);
+    sum_partials_planes<4>(src, HH, 4 * HH, rec_count(k.rec, k.NCH), sp);
     const float s0 = sp[0], s1 = sp[1], s2 = sp[2], s3 = sp[3];
     k.g.w_erev[tid] = s0;
     k.g.w_pos[tid] = s1;
@@ -3830,6 +3857,7 @@ struct FinLeafK {
   const int* status;
   float* gstate;
   long long nx, ns;
+  RecParts rec;
 };
 
 // Every output this thread owns, NaN (a fused row backward gave up).
@@ -3928,7 +3956,8 @@ __global__ __launch_bounds__(256) void finalize_leaf_kernel(FinLeafK k) {
       dst[e] = 0.f;
       return;
     }
-    const float s = sum_partials_plane(k.rpart + q * HH + (long long)i * Hp + j, 4 * HH, k.NCH);
+    const float s = sum_partials_plane(k.rpart + q * HH + (long long)i * Hp + j, 4 * HH,
+                                       rec_count(k.rec, k.NCH));
     const float dwe = quad_lane<0>(s), dwp = quad_lane<1>(s);
     const float sd = quad_lane<2>(s), sdv = quad_lane<3>(s);
     const float wv = k.lp.w[e];
@@ -5916,6 +5945,11 @@ hipError_t fwd_by_rcp(const Plan& p, const FwdK& a, hipStream_t s) {
   const dim3 grid((p.B + NB - 1) / NB), block(p.Hp * p.KS);
   const size_t lds = fwd_lds_bytes(p);
   const int rcp = (p.RC == 4 || p.RC == 8 || p.RC == 16) ? p.RC : 0;
+  if (a.gate != nullptr) {
+    if (rcp != 0) return hipErrorInvalidValue;
+    LTC_LAUNCH((ode_fwd_kernel<NB, 0, true>), grid, block, lds, s, a);
+    return hipGetLastError();
+  }
   if constexpr (NB == 1) {
     if (row_wave128_fwd(p)) {
       LTC_LAUNCH((ode_fwd_row_wave_kernel<128>), grid, dim3(512), lds, s, a);
@@ -5942,6 +5976,11 @@ hipError_t bwd_by_rcp(const Plan& p, const BwdK& a, hipStream_t s) {
   const dim3 grid((p.B + NB - 1) / NB), block(p.Hp * p.KSB);
   const size_t lds = bwd_lds_bytes(p);
   const int rcp = (p.RCB == 4 || p.RCB == 8 || p.RCB == 16) ? p.RCB : 0;
+  if (a.gate != nullptr) {
+    if (rcp != 0 || p.FUSE) return hipErrorInvalidValue;
+    LTC_LAUNCH((ode_bwd_kernel<NB, 0, false, true>), grid, block, lds, s, a);
+    return hipGetLastError();
+  }
 #define LTC_BWD(R, F) LTC_LAUNCH((ode_bwd_kernel<NB, R, F>), grid, block, lds, s, a)
   if constexpr (NB == 1) {
     if (row_kernels(p)) {
@@ -6232,6 +6271,14 @@ hipError_t launch_sens_fwd_ln(const Plan& p, const float* x, Strides3 xs, const 
 hipError_t launch_ode_fwd(const Plan& p, const Prepped& pp, const float* sn, const float* sd,
                           const float* state0, float eps, float* out, float* hfin,
                           float* vsave, float* densave, const ClusterBuf& cb, hipStream_t s) {
+  return launch_ode_fwd_after(p, pp, sn, sd, state0, eps, out, hfin, vsave, densave, cb, nullptr, s);
+}
+
+hipError_t launch_ode_fwd_after(const Plan& p, const Prepped& pp, const float* sn,
+                                const float* sd, const float* state0, float eps, float* out,
+                                float* hfin, float* vsave, float* densave, const ClusterBuf& cb,
+                                const int* gate, hipStream_t s) {
+  if (gate != nullptr && (p.rf.CP > 0 || p.CP > 0)) return hipErrorInvalidValue;
   if (p.rf.CP > 0) {
     if (pp.cF == nullptr || pp.cFi == nullptr || pp.cFn == nullptr) return hipErrorInvalidValue;
     const RegCluster& g = p.rf;
@@ -6277,7 +6324,7 @@ hipError_t launch_ode_fwd(const Plan& p, const Prepped& pp, const float* sn, con
     return hipSuccess;
   }
   FwdK a{pp.recF, pp.neuron, sn, sd, state0, out, hfin, vsave, densave,
-         p.B, p.T, p.H, p.Hp, p.U, p.KS, p.RC, eps, pp.cF, pp.cFi, pp.cFn};
+         p.B, p.T, p.H, p.Hp, p.U, p.KS, p.RC, eps, pp.cF, pp.cFi, pp.cFn, gate};
   if (cmp_fwd(p) && (pp.cF == nullptr || pp.cFi == nullptr || pp.cFn == nullptr))
     return hipErrorInvalidValue;
   switch (p.NB) {
@@ -6294,6 +6341,16 @@ hipError_t launch_ode_bwd(const Plan& p, const Prepped& pp, const float* vsave,
                           const float* ghfin, float2* absave, float* dsn, float* dsd,
                           float* npart, float* gstate, float* rpart, const ClusterBuf& cb,
                           hipStream_t s) {
+  return launch_ode_bwd_after(p, pp, vsave, densave, gout, gs, ghfin, absave, dsn, dsd, npart,
+                              gstate, rpart, cb, nullptr, s);
+}
+
+hipError_t launch_ode_bwd_after(const Plan& p, const Prepped& pp, const float* vsave,
+                                const float* densave, const float* gout, Strides3 gs,
+                                const float* ghfin, float2* absave, float* dsn, float* dsd,
+                                float* npart, float* gstate, float* rpart, const ClusterBuf& cb,
+                                const int* gate, hipStream_t s) {
+  if (gate != nullptr && (p.rb.CP > 0 || p.CP > 0 || absave == nullptr)) return hipErrorInvalidValue;
   if (p.rb.CP > 0) {
     if (pp.cB == nullptr || pp.cBi == nullptr || pp.cBn == nullptr) return hipErrorInvalidValue;
     const RegCluster& g = p.rb;
@@ -6338,7 +6395,7 @@ hipError_t launch_ode_bwd(const Plan& p, const Prepped& pp, const float* vsave,
     return hipSuccess;
   }
   BwdK a{pp.recB, pp.neuron, vsave, densave, gout, gs, ghfin, absave, dsn, dsd, npart, gstate,
-         rpart, p.B, p.T, p.H, p.Hp, p.U, p.KSB, p.RCB, pp.cB, pp.cBi, pp.cBn, nullptr};
+         rpart, p.B, p.T, p.H, p.Hp, p.U, p.KSB, p.RCB, pp.cB, pp.cBi, pp.cBn, nullptr, gate};
   if (cmp_bwd(p) && (pp.cB == nullptr || pp.cBi == nullptr || pp.cBn == nullptr))
     return hipErrorInvalidValue;
   switch (p.NB) {
@@ -6422,9 +6479,10 @@ hipError_t launch_ode_bwd_row_fused(const Plan& p, const Prepped& pp, const floa
 }
 
 hipError_t launch_rec_grad(const Plan& p, const Prepped& pp, const float* vsave,
-                           const float2* absave, float* rpart, hipStream_t s, const float* mask) {
+                           const float2* absave, float* rpart, hipStream_t s, const float* mask,
+                           const int* gate) {
   const long long nper = (p.N + p.NCH - 1) / p.NCH;
-  RecGK a{pp.recF, vsave, absave, mask, rpart, p.H, p.Hp, p.N, nper};
+  RecGK a{pp.recF, vsave, absave, mask, rpart, p.H, p.Hp, p.N, nper, gate};
   LTC_LAUNCH(rec_grad_kernel, dim3(p.Hp / 64, p.Hp / 32, p.NCH), dim3(256), 0, s, a);
   return hipGetLastError();
 }
@@ -6475,7 +6533,8 @@ hipError_t presum(const Plan& p, const float* rpart, const float* npart, const P
 
 hipError_t launch_finalize(const Plan& p, const RawParams& rp, const float* rpart,
                            const float* spart, const float* dxpart, const float* npart,
-                           const PresumBuf& ps, const GradOut& g, hipStream_t s, int segs) {
+                           const PresumBuf& ps, const GradOut& g, hipStream_t s, int segs,
+                           const RecParts& rec) {
   const int BT = p.B * p.T;
   Partials pt{rpart, p.NCH, npart, p.B};
   if (segs & kFinRec) {
@@ -6488,7 +6547,9 @@ hipError_t launch_finalize(const Plan& p, const RawParams& rp, const float* rpar
   const long long count = ((segs & kFinRec) ? nrn : 0) + ((segs & kFinSens) ? nsx : 0);
   if (count == 0) return hipSuccess;
   FinK a{rp, pt.rpart, spart, dxpart, pt.npart, g, pt.nneuron, p.D, p.H, p.Hp, p.Dp, pt.nrec,
-         p.NRC, p.Hp / 32, BT, base, count};
+         p.NRC, p.Hp / 32, BT, base, count, rec};
+  if (rec.status != nullptr && (presum_parts(p.NCH) > 0 || presum_parts(rec.nch) > 0))
+    return hipErrorInvalidValue;
   const unsigned blocks = (unsigned)((count + 255) / 256);
   LTC_LAUNCH(finalize_kernel, dim3(blocks), dim3(256), 0, s, a);
   return hipGetLastError();
@@ -6565,7 +6626,9 @@ hipError_t launch_ln_bwd(const Plan& p, const LeafParams& lp, const LnBuf& ln,
 hipError_t launch_finalize_leaf(const Plan& p, const LeafParams& lp, const float* rpart,
                                 const float* spart, const float* npart, const float* lnpart,
                                 const PresumBuf& ps, const LeafGrads& g, hipStream_t s,
-                                const int* status, float* gstate) {
+                                const int* status, float* gstate, const RecParts& rec) {
+  if (rec.status != nullptr && (presum_parts(p.NCH) > 0 || presum_parts(rec.nch) > 0))
+    return hipErrorInvalidValue;
   Partials pt;
   hipError_t e = presum(p, rpart, npart, ps, s, pt);
   if (e != hipSuccess) return e;
@@ -6584,7 +6647,7 @@ hipError_t launch_finalize_leaf(const Plan& p, const LeafParams& lp, const float
   const long long nx = status ? (long long)p.B * p.T * p.D : 0;
   const long long ns = status && gstate ? (long long)p.B * p.H : 0;
   FinLeafK a{lp, pt.rpart, spart, pt.npart, lnpart, g, pt.nneuron, p.D, p.H, p.Hp, p.Dp,
-             pt.nrec, p.NRC, nln, status, gstate, nx, ns};
+             pt.nrec, p.NRC, nln, status, gstate, nx, ns, rec};
   // four threads per output element, or one per output when a gave-up status
   // turns them all into NaN
   const long long nel = (long long)p.H * p.H + (long long)p.D * p.H + p.H + p.D;
@@ -6606,7 +6669,7 @@ hipError_t launch_finalize_leaf_fused(const Plan& p, const LeafParams& lp, const
   const long long nx = (long long)p.B * p.T * p.D, ns = (long long)p.B * p.H;
   // one sensory and one LayerNorm partial per batch row (B <= 64)
   FinLeafK a{lp, pt.rpart, spart, pt.npart, lnpart, g, pt.nneuron, p.D, p.H, p.Hp, p.Dp,
-             pt.nrec, p.B, p.B, status, gstate, nx, ns};
+             pt.nrec, p.B, p.B, status, gstate, nx, ns, RecParts{nullptr, 0}};
   // four threads per output element, or one per output (every leaf gradient,
   // dL/dx and dL/dh0) when a gave-up status turns them all into NaN
   const long long nel = (long long)p.H * p.H + (long long)p.D * p.H + p.H + p.D;

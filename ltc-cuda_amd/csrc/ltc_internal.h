@@ -356,6 +356,16 @@ inline bool bwd_clusters(const Plan& p) { return p.rb.CP > 0 || p.CP > 0; }
 // how many partials of them the backward's finalize sums.
 inline bool chain_fused(const Plan& p) { return p.rb.CP > 0 || p.FUSE; }
 inline int rec_parts(const Plan& p) { return p.rb.CP > 0 ? p.rb.NCL : p.NCH; }
+// Register-resident clusters where the plan itself has none (H <= 192, and
+// batches past one launch of its clusters): these sizes never depended on other
+// workgroups, so when a member gives up waiting, the plan's own kernels, launched
+// behind the clusters and gated by their status word, make the results.
+inline bool fwd_after(const Plan& p) { return p.rf.CP > 0 && p.CP == 0; }
+inline bool bwd_after(const Plan& p) { return p.rb.CP > 0 && p.CP == 0; }
+inline Plan own_plan(Plan p) {
+  p.rf = p.rb = RegCluster{};
+  return p;
+}
 inline long long cluster_words_bwd(const Plan& p) {
   if (p.rb.CP > 0) return 2LL * p.rb.NCL * p.rb.CP * p.rb.NB * p.rb.JW;
   return 2LL * p.NCLB * p.CPB * p.NBB * p.JWB;
@@ -565,6 +575,17 @@ inline long long chain_launch_lds(const Plan& p) {
 hipError_t launch_ode_fwd(const Plan& p, const Prepped& pp, const float* sn, const float* sd,
                           const float* state0, float eps, float* out, float* hfin,
                           float* vsave, float* densave, const ClusterBuf& cb, hipStream_t s);
+// The plan's own kernels behind register-resident clusters (fwd_after,
+// bwd_after): they run only when the status word `gate` is set.
+hipError_t launch_ode_fwd_after(const Plan& p, const Prepped& pp, const float* sn,
+                                const float* sd, const float* state0, float eps, float* out,
+                                float* hfin, float* vsave, float* densave, const ClusterBuf& cb,
+                                const int* gate, hipStream_t s);
+hipError_t launch_ode_bwd_after(const Plan& p, const Prepped& pp, const float* vsave,
+                                const float* densave, const float* gout, Strides3 gs,
+                                const float* ghfin, float2* absave, float* dsn, float* dsd,
+                                float* npart, float* gstate, float* rpart, const ClusterBuf& cb,
+                                const int* gate, hipStream_t s);
 hipError_t launch_ode_bwd(const Plan& p, const Prepped& pp, const float* vsave,
                           const float* densave, const float* gout, Strides3 gs,
                           const float* ghfin, float2* absave, float* dsn, float* dsd,
@@ -574,7 +595,7 @@ hipError_t launch_ode_bwd(const Plan& p, const Prepped& pp, const float* vsave,
 // whose partials stay unwritten.
 hipError_t launch_rec_grad(const Plan& p, const Prepped& pp, const float* vsave,
                            const float2* absave, float* rpart, hipStream_t s,
-                           const float* mask = nullptr);
+                           const float* mask = nullptr, const int* gate = nullptr);
 // smask (the module path's sensory mask, (D,H)): skip the masked synapses
 // (sens_bwd_cmp_kernel), whose partials stay unwritten.
 hipError_t launch_sens_bwd(const Plan& p, const float* x, Strides3 xs, const Prepped& pp,
@@ -609,6 +630,12 @@ struct PresumBuf {
   float* neuron;  // presum_parts(B) x 3*Hp
   float* ln;      // module path: presum_parts(ln_bwd_blocks) x 4*Dp
 };
+// With `status` set, the recurrent partials are `nch` instead (those of the
+// kernels behind the clusters, bwd_after).
+struct RecParts {
+  const int* status;
+  int nch;
+};
 // Gradient groups a finalize launch writes: the recurrent and per-neuron
 // gradients (from rpart, npart) and the sensory and input gradients (from
 // spart, dxpart).
@@ -616,7 +643,7 @@ constexpr int kFinRec = 1, kFinSens = 2, kFinAll = kFinRec | kFinSens;
 hipError_t launch_finalize(const Plan& p, const RawParams& rp, const float* rpart,
                            const float* spart, const float* dxpart, const float* npart,
                            const PresumBuf& ps, const GradOut& g, hipStream_t s,
-                           int segs = kFinAll);
+                           int segs = kFinAll, const RecParts& rec = RecParts{nullptr, 0});
 
 // Module path backward.
 struct LeafGrads {
@@ -647,7 +674,8 @@ hipError_t launch_ln_bwd(const Plan& p, const LeafParams& lp, const LnBuf& ln,
 hipError_t launch_finalize_leaf(const Plan& p, const LeafParams& lp, const float* rpart,
                                 const float* spart, const float* npart, const float* lnpart,
                                 const PresumBuf& ps, const LeafGrads& g, hipStream_t s,
-                                const int* status = nullptr, float* gstate = nullptr);
+                                const int* status = nullptr, float* gstate = nullptr,
+                                const RecParts& rec = RecParts{nullptr, 0});
 
 // Fused row backward (row_bwd_fused): the chain of every batch row plus one
 // companion workgroup per row for its sensory and LayerNorm backward. The

@@ -740,7 +740,8 @@ def require_kernels():
 def device_status(clear: bool = True) -> None:
     """Raise RuntimeError if a launch on the current device gave up waiting
     for its partner workgroups since the last check: a cluster launch
-    (H > 128), or the companion workgroups of a module backward with one batch
+    (H > 128 and plan field CP > 0; where it is 0 other kernels then make the
+    results and nothing is raised), or the companion workgroups of a module backward with one batch
     row per workgroup (the sensory and LayerNorm companions at H <= 64, the
     recurrent-gradient and sensory companions at 64 < H <= 128). The outputs
     of that call were set to NaN. Synchronises the device."""
