@@ -303,12 +303,9 @@ __device__ __forceinline__ void stream_rows(__amdgpu_buffer_rsrc_t rs, int lane_
 // chunk the rows ks, ks + nch, ... and all lanes of a chunk the same row per
 // slot. The image has nrows rows (slots of all chunks) of `stride` columns.
 // The kernels evaluate slots past a column's count too (a wave runs as many as
-// its fullest lane), with a weight of zero, so such a slot's gate must not be
-// NaN where the column's own gates are not: it repeats the row, slope and
-// offset of the column's first entry. (With zero operands an infinite state of
-// row 0 gave 0 * inf = NaN in every column.) In a column without entries it
-// takes row 0 with a slope so small that every finite state's gate is 1/2,
-// and an infinite state's 0 or 1.
+// its fullest lane): those hold zero weights at row 0, and a slope so small that
+// every finite state's gate is 1/2 and an infinite state's 0 or 1. (With a zero
+// slope an infinite state of row 0 gave 0 * inf = NaN in every column.)
 // ---------------------------------------------------------------------------
 constexpr float kMinSlope = 1e-20f;
 
@@ -317,20 +314,13 @@ __device__ __forceinline__ void compact_column(int col, int nrows, int stride, i
                                                float4* cimg, int* cidx, int* ccnt, Op op) {
   const int sc = nrows / nch;
   auto at = [&](int e) { return (long long)((e % nch) * sc + e / nch) * stride + col; };
-  int n = 0, pad_row = 0;
-  float4 pad = make_float4(kMinSlope, 0.f, 0.f, 0.f);
+  int n = 0;
   for (int r0 = 0; r0 < nrows; r0 += 64) {
     const int r = r0 + lane;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     bool act = false;
     op(r, v, act);
     const unsigned long long m = __ballot(act);
-    if (n == 0 && m != 0) {  // wave-uniform
-      const int l = __ffsll(m) - 1;
-      pad_row = r0 + l;
-      pad.x = __shfl(v.x, l, 64);
-      pad.y = __shfl(v.y, l, 64);
-    }
     if (act) {
       const long long a = at(n + __popcll(m & ((1ULL << lane) - 1ULL)));
       cimg[a] = v;
@@ -340,8 +330,8 @@ __device__ __forceinline__ void compact_column(int col, int nrows, int stride, i
   }
   for (int e = n + lane; e < nrows; e += 64) {
     const long long a = at(e);
-    cimg[a] = pad;
-    cidx[a] = pad_row;
+    cimg[a] = make_float4(kMinSlope, 0.f, 0.f, 0.f);
+    cidx[a] = 0;
   }
   if (lane == 0) ccnt[col] = n;
 }

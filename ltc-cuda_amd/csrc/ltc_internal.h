@@ -126,11 +126,10 @@ struct Plan {
 //   cB[(ks*Hp/NC + s)*Hp + i]  chain operand of column i (presynaptic), rows j: every
 //                           real synapse, or on the module path only those whose
 //                           mask entry is nonzero (the others have zero gradients);
-//   cFi / cBi               the row index of each slot;
+//   cFi / cBi               the row index of each slot (0 in padding slots);
 //   cFn / cBn               the entry count of each column.
-// Padding slots hold zero weights, which add exact zeros, at the row and with
-// the gate argument of the column's first entry (compact_column). Null when
-// the plan does not use the compacted kernels.
+// Padding slots hold zero weights, which add exact zeros (compact_column). Null
+// when the plan does not use the compacted kernels.
 struct Prepped {
   float4* recF;
   float4* recB;
