@@ -820,7 +820,12 @@ struct FwdK {
   const float4* cimg;
   const int* cidx;
   const int* ccnt;
-  const int* gate;  // AFTER: the status word of the clusters before this launch
+};
+// AFTER: with the status word of the clusters before the launch. (Types of their
+// own: one more member of FwdK or BwdK changes the code of every kernel that
+// takes them, the Hp = 128 row chain 144 -> 150 us.)
+struct FwdAfterK : FwdK {
+  const int* gate;
 };
 
 template <int NB>
@@ -928,8 +933,11 @@ __device__ __forceinline__ void fwd_synapses_cmp(const float4* p, const float* v
 // AFTER: behind register-resident clusters whose members gave up waiting, this
 // launch makes the call's results instead; otherwise it leaves at once.
 template <int NB, int RCP, bool AFTER = false>
-__global__ __launch_bounds__(ode_max_threads(NB)) void ode_fwd_kernel(FwdK k) {
-  if (AFTER && !gate_open(k.gate)) return;
+__global__ __launch_bounds__(ode_max_threads(NB)) void ode_fwd_kernel(
+    std::conditional_t<AFTER, FwdAfterK, FwdK> k) {
+  if constexpr (AFTER) {
+    if (!gate_open(k.gate)) return;
+  }
   constexpr int MO = ode_owned_rows(NB);
   constexpr bool CMP = RCP > 0;
   extern __shared__ float4 lds4[];
@@ -1107,7 +1115,9 @@ struct BwdK {
   // dsd; the Hp = 128 chain with recurrent-gradient companions sends each
   // unfold's alpha/beta as [B][T*U][2][128] words instead of into absave.
   unsigned long long* rbw;
-  const int* gate;  // AFTER: the status word of the clusters before this launch
+};
+struct BwdAfterK : BwdK {
+  const int* gate;
 };
 
 // The recurrent-gradient companions of the Hp = 128 chain: the forward image
@@ -1243,10 +1253,13 @@ __device__ __forceinline__ void bwd_load_gout(const BwdK& k, int t, int b0, int 
 // AFTER: as in ode_fwd_kernel. The clusters' image is not folded: the operands
 // are folded here as they arrive.
 template <int NB, int RCP, bool FUSE, bool AFTER = false>
-__global__ __launch_bounds__(ode_max_threads(NB)) void ode_bwd_kernel(BwdK k) {
+__global__ __launch_bounds__(ode_max_threads(NB)) void ode_bwd_kernel(
+    std::conditional_t<AFTER, BwdAfterK, BwdK> k) {
   static_assert(!FUSE || RCP > 0, "fused gradients need register-resident operands");
   static_assert(!AFTER || RCP == 0, "the launch behind clusters streams its operands");
-  if (AFTER && !gate_open(k.gate)) return;
+  if constexpr (AFTER) {
+    if (!gate_open(k.gate)) return;
+  }
   constexpr int MO = ode_owned_rows(NB);
   constexpr bool CMP = !FUSE && RCP > 0;
   extern __shared__ float4 lds4[];
@@ -5931,13 +5944,13 @@ size_t fwd_lds_bytes(const Plan& p) { return (size_t)fwd_lds(p); }
 size_t bwd_lds_bytes(const Plan& p) { return (size_t)chain_lds(p); }
 
 template <int NB>
-hipError_t fwd_by_rcp(const Plan& p, const FwdK& a, hipStream_t s) {
+hipError_t fwd_by_rcp(const Plan& p, const FwdK& a, const int* gate, hipStream_t s) {
   const dim3 grid((p.B + NB - 1) / NB), block(p.Hp * p.KS);
   const size_t lds = fwd_lds_bytes(p);
   const int rcp = (p.RC == 4 || p.RC == 8 || p.RC == 16) ? p.RC : 0;
-  if (a.gate != nullptr) {
+  if (gate != nullptr) {
     if (rcp != 0) return hipErrorInvalidValue;
-    LTC_LAUNCH((ode_fwd_kernel<NB, 0, true>), grid, block, lds, s, a);
+    LTC_LAUNCH((ode_fwd_kernel<NB, 0, true>), grid, block, lds, s, FwdAfterK{a, gate});
     return hipGetLastError();
   }
   if constexpr (NB == 1) {
@@ -5962,13 +5975,13 @@ hipError_t fwd_by_rcp(const Plan& p, const FwdK& a, hipStream_t s) {
 }
 
 template <int NB>
-hipError_t bwd_by_rcp(const Plan& p, const BwdK& a, hipStream_t s) {
+hipError_t bwd_by_rcp(const Plan& p, const BwdK& a, const int* gate, hipStream_t s) {
   const dim3 grid((p.B + NB - 1) / NB), block(p.Hp * p.KSB);
   const size_t lds = bwd_lds_bytes(p);
   const int rcp = (p.RCB == 4 || p.RCB == 8 || p.RCB == 16) ? p.RCB : 0;
-  if (a.gate != nullptr) {
+  if (gate != nullptr) {
     if (rcp != 0 || p.FUSE) return hipErrorInvalidValue;
-    LTC_LAUNCH((ode_bwd_kernel<NB, 0, false, true>), grid, block, lds, s, a);
+    LTC_LAUNCH((ode_bwd_kernel<NB, 0, false, true>), grid, block, lds, s, BwdAfterK{a, gate});
     return hipGetLastError();
   }
 #define LTC_BWD(R, F) LTC_LAUNCH((ode_bwd_kernel<NB, R, F>), grid, block, lds, s, a)
@@ -6314,15 +6327,15 @@ hipError_t launch_ode_fwd_after(const Plan& p, const Prepped& pp, const float* s
     return hipSuccess;
   }
   FwdK a{pp.recF, pp.neuron, sn, sd, state0, out, hfin, vsave, densave,
-         p.B, p.T, p.H, p.Hp, p.U, p.KS, p.RC, eps, pp.cF, pp.cFi, pp.cFn, gate};
+         p.B, p.T, p.H, p.Hp, p.U, p.KS, p.RC, eps, pp.cF, pp.cFi, pp.cFn};
   if (cmp_fwd(p) && (pp.cF == nullptr || pp.cFi == nullptr || pp.cFn == nullptr))
     return hipErrorInvalidValue;
   switch (p.NB) {
-    case 16: return fwd_by_rcp<16>(p, a, s);
-    case 8: return fwd_by_rcp<8>(p, a, s);
-    case 4: return fwd_by_rcp<4>(p, a, s);
-    case 2: return fwd_by_rcp<2>(p, a, s);
-    default: return fwd_by_rcp<1>(p, a, s);
+    case 16: return fwd_by_rcp<16>(p, a, gate, s);
+    case 8: return fwd_by_rcp<8>(p, a, gate, s);
+    case 4: return fwd_by_rcp<4>(p, a, gate, s);
+    case 2: return fwd_by_rcp<2>(p, a, gate, s);
+    default: return fwd_by_rcp<1>(p, a, gate, s);
   }
 }
 
@@ -6385,15 +6398,15 @@ hipError_t launch_ode_bwd_after(const Plan& p, const Prepped& pp, const float* v
     return hipSuccess;
   }
   BwdK a{pp.recB, pp.neuron, vsave, densave, gout, gs, ghfin, absave, dsn, dsd, npart, gstate,
-         rpart, p.B, p.T, p.H, p.Hp, p.U, p.KSB, p.RCB, pp.cB, pp.cBi, pp.cBn, nullptr, gate};
+         rpart, p.B, p.T, p.H, p.Hp, p.U, p.KSB, p.RCB, pp.cB, pp.cBi, pp.cBn, nullptr};
   if (cmp_bwd(p) && (pp.cB == nullptr || pp.cBi == nullptr || pp.cBn == nullptr))
     return hipErrorInvalidValue;
   switch (p.NB) {
-    case 16: return bwd_by_rcp<16>(p, a, s);
-    case 8: return bwd_by_rcp<8>(p, a, s);
-    case 4: return bwd_by_rcp<4>(p, a, s);
-    case 2: return bwd_by_rcp<2>(p, a, s);
-    default: return bwd_by_rcp<1>(p, a, s);
+    case 16: return bwd_by_rcp<16>(p, a, gate, s);
+    case 8: return bwd_by_rcp<8>(p, a, gate, s);
+    case 4: return bwd_by_rcp<4>(p, a, gate, s);
+    case 2: return bwd_by_rcp<2>(p, a, gate, s);
+    default: return bwd_by_rcp<1>(p, a, gate, s);
   }
 }
 
