@@ -326,10 +326,12 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
  * chain (members of 32 columns, parameter gradients fused): workgroups per
  * cluster (0: not used), rows per cluster, launches per call, LDS bytes per
  * workgroup, and unfolds between the moves of its gradient sums out of the
- * registers (0: none). Returns the number of values written, or -1 for invalid
- * sizes. The plan depends on the current device's CU count.
+ * registers (0: none); then 1 when the register-resident forward, and 1 when the
+ * chain, takes its synapses from the dense image (few unfolds; a backward over
+ * the boundary tensors always does). Returns the number of values written, or -1
+ * for invalid sizes. The plan depends on the current device's CU count.
  */
-#define LTC_PLAN_FIELDS 38
+#define LTC_PLAN_FIELDS 40
 int ltc_launch_plan(int B, int T, int D, int H, int ode_unfolds, long long* out, int n);
 
 /*

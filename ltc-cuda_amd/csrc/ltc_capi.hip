@@ -219,6 +219,23 @@ void reg_cluster_counts(ltc::RegCluster& g, int B, int slots, int ncu) {
   g.xcd = (g.NCL + 7) / 8 * 8 * g.CP <= ncu;
 }
 
+// Unfolds times rows of a cluster over all launches up to which the clusters
+// take their synapses from the dense image.
+constexpr long long kRegDenseRows = 24;
+
+// Calls of several launches and few unfolds: each launch clears its words and
+// loads every operand again, about 12 us, against 15 to 25 us an unfold that the
+// plan's own kernels lose. Two unfolds never pay for it (B1024 H192 to H512
+// without gradients 1.3 to 1.6 times the own kernels' time); three do where those
+// leave many CUs idle (B600: 300 workgroups of two rows; 0.78 to 0.90 times, and
+// 1.05 to 1.39 at B1024 and B256, where they fill the chip).
+bool reg_too_short(const ltc::Plan& p, int launches) {
+  const long long n = (long long)p.T * p.U;
+  if (launches <= 1 || n > 3) return false;
+  const int wgs = (p.B + p.NB - 1) / p.NB, rounds = (wgs + 255) / 256;
+  return n <= 2 || p.CP > 0 || wgs * 10 >= rounds * 256 * 9;
+}
+
 // Register-resident clusters for 128 < Hp <= 512 where the plan above has no
 // register-resident form: a forward member's 1024 threads hold the compacted
 // synapses of 64 columns or 32, at most 20 or 16 each at any mask density, so
@@ -255,6 +272,16 @@ void plan_reg_forward(ltc::Plan& p, int ncu) {
     }
   }
   reg_cluster_counts(g, p.B, ncu / g.CP, ncu);
+  if (reg_too_short(p, g.L)) return;
+  // Compacting an image takes longer than the dense one (Hp = 320 ... 512: 13 to
+  // 20 us of a prep launch's 30), which few unfolds do not win back; one row per
+  // cluster is bound by the exchange, not by its slots, and hardly needs it.
+  // Compacted / dense, us a call without gradients: B1 H512 T1 61.6 / 35.9, T8
+  // 157 / 135; B16 H320 T4 89.8 / 87.0, T8 141 / 151; several rows, B64 H320 T1
+  // 43.8 / 41.1, T2 59.0 / 60.7; B256 H192 T1 39.4 / 44.0.
+  const long long n = (long long)p.T * p.U;
+  g.dense = g.NB == 1 ? n <= (p.Hp > 320 ? 64 : 24)
+                      : p.Hp > 256 && n * g.NB * g.L <= kRegDenseRows;
   if (ltc::reg_fwd_lds(g, p.Hp) <= chain_lds_limit()) p.rf = g;
 }
 
@@ -296,6 +323,13 @@ void plan_reg_chain(ltc::Plan& p, int ncu) {
     if ((p.B + nb - 1) / nb <= slots) break;
   }
   reg_cluster_counts(g, p.B, slots, ncu);
+  if (reg_too_short(p, g.L)) return;
+  // The same for the chains that would stream a dense mask: step B1 H512 T1 154
+  // us with the compacted image, 133 streaming; T2 191 / 181, T4 271 / 288; B64
+  // H320 T1 147 / 140, T2 197 / 203; B256 H320, one unfold 198 / 180, three 251 /
+  // 253. Up to Hp = 256 the compacted form is the faster at one unfold already
+  // (B16 H192 68 / 73).
+  g.dense = g.RC > 16 && (long long)p.T * p.U * g.NB * g.L <= kRegDenseRows;
   const long long nch = (g.RC == 32 ? 2 : 4) * rec_grad_chunks(p);
   const long long terms = std::max<long long>((p.N + nch - 1) / nch, kRegSumTerms);
   const long long fl = (terms + g.NB - 1) / g.NB;
@@ -459,6 +493,13 @@ ltc::Plan make_plan(int B, int T, int D, int H, int U, bool reg = true) {
   next = (next + 1) % kEntries;
   if (used < kEntries) ++used;
   return e.p;
+}
+
+// The plan of a backward over the boundary tensors: its chain image would hold
+// every synapse (their gradients are all wanted), so there is nothing to compact.
+ltc::Plan boundary_plan(ltc::Plan p) {
+  p.rb.dense = p.rb.CP > 0;
+  return p;
 }
 
 // Carves 256-byte aligned regions out of one workspace in a fixed order; the
@@ -897,7 +938,7 @@ long long ltc_fwd_workspace_bytes(int B, int T, int D, int H, int ode_unfolds) {
 
 long long ltc_bwd_workspace_bytes(int B, int T, int D, int H, int ode_unfolds) {
   if (check_dims(B, T, D, H, ode_unfolds) != LTC_OK) return -1;
-  const ltc::Plan p = make_plan(B, T, D, H, ode_unfolds);
+  const ltc::Plan p = boundary_plan(make_plan(B, T, D, H, ode_unfolds));
   Carver c{nullptr};
   carve_bwd(p, c);
   return round_up(c.off, 256);
@@ -1044,7 +1085,7 @@ int ltc_full_backward(const float* x, long long sxb, long long sxt, long long sx
   if (B > 0 && !grad_state) return fail(LTC_EINVAL, "grad_state pointer is NULL");
   if ((long long)B * T > 0 && (!x || !grad_out || !grad_x || !saved))
     return fail(LTC_EINVAL, "x/grad_out/grad_x/saved pointer is NULL");
-  const ltc::Plan p = make_plan(B, T, D, H, ode_unfolds);
+  const ltc::Plan p = boundary_plan(make_plan(B, T, D, H, ode_unfolds));
   Carver need{nullptr};
   carve_bwd(p, need);
   if (workspace_bytes < need.off || (need.off > 0 && !workspace))
@@ -1483,7 +1524,7 @@ long long ltc_sensory_bwd_workspace_bytes(int B, int D, int H) {
 
 long long ltc_ode_unfold_fwd_workspace_bytes(int B, int H, int ode_unfolds) {
   if (check_step_dims(B, 1, H, ode_unfolds) != LTC_OK) return -1;
-  const ltc::Plan p = make_plan(B, 1, 1, H, ode_unfolds);
+  const ltc::Plan p = boundary_plan(make_plan(B, 1, 1, H, ode_unfolds));
   Carver c{nullptr};
   carve_unfold(p, c, false);
   return round_up(c.off, 256);
@@ -1491,7 +1532,7 @@ long long ltc_ode_unfold_fwd_workspace_bytes(int B, int H, int ode_unfolds) {
 
 long long ltc_ode_unfold_bwd_workspace_bytes(int B, int H, int ode_unfolds) {
   if (check_step_dims(B, 1, H, ode_unfolds) != LTC_OK) return -1;
-  const ltc::Plan p = make_plan(B, 1, 1, H, ode_unfolds);
+  const ltc::Plan p = boundary_plan(make_plan(B, 1, 1, H, ode_unfolds));
   Carver c{nullptr};
   carve_unfold(p, c, true);
   return round_up(c.off, 256);
@@ -1605,7 +1646,7 @@ int ltc_ode_unfold_fwd(const float* state, const float* w_pos, const float* w_er
     return fail(LTC_EINVAL, "state/w_num_sensory/w_den_sensory/state_out pointer is NULL");
   if (B > 0 && save_intermediates && !v_buffer)
     return fail(LTC_EINVAL, "v_buffer pointer is NULL");
-  const ltc::Plan p = make_plan(B, 1, 1, H, ode_unfolds);
+  const ltc::Plan p = boundary_plan(make_plan(B, 1, 1, H, ode_unfolds));
   Carver need{nullptr};
   carve_unfold(p, need, false);
   rc = check_ws(need.off, workspace, workspace_bytes);
@@ -1667,7 +1708,7 @@ int ltc_ode_unfold_bwd(const float* v_buffer, const float* w_pos, const float* w
   if (B > 0 && (!v_buffer || !w_num_sensory || !w_den_sensory || !grad_output || !grad_v ||
                 !grad_w_num_sensory || !grad_w_den_sensory))
     return fail(LTC_EINVAL, "v_buffer/sensory/grad_output/grad_v pointer is NULL");
-  const ltc::Plan p = make_plan(B, 1, 1, H, ode_unfolds);
+  const ltc::Plan p = boundary_plan(make_plan(B, 1, 1, H, ode_unfolds));
   Carver need{nullptr};
   carve_unfold(p, need, true);
   rc = check_ws(need.off, workspace, workspace_bytes);
@@ -1763,7 +1804,8 @@ int ltc_launch_plan(int B, int T, int D, int H, int ode_unfolds, long long* out,
       ltc::row_bwd_fused(p) ? 1 : 0, ltc::row128_rec_fused(p) ? 1 : 0, p.LCH, p.LCHB,
       ltc::sens_full_list(p) ? 1 : 0,
       p.rf.CP, p.rf.JW, p.rf.NB, p.rf.L, p.rf.CP > 0 ? ltc::reg_fwd_lds(p.rf, p.Hp) : 0,
-      p.rb.CP, p.rb.NB, p.rb.L, p.rb.CP > 0 ? ltc::reg_bwd_lds(p.rb, p.Hp) : 0, p.rb.FL};
+      p.rb.CP, p.rb.NB, p.rb.L, p.rb.CP > 0 ? ltc::reg_bwd_lds(p.rb, p.Hp) : 0, p.rb.FL,
+      p.rf.dense ? 1 : 0, p.rb.dense ? 1 : 0};
   const int m = n < LTC_PLAN_FIELDS ? n : LTC_PLAN_FIELDS;
   for (int i = 0; i < m; ++i) out[i] = v[i];
   return m;

@@ -4370,13 +4370,14 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
   int nslot, sks, so;
   {
     int* perm = reinterpret_cast<int*>(slot_tab + (RCP / 4) * nthr);
-    const int cnt0 = k.ccnt[c];
+    const bool dense = NF && k.cimg == nullptr;
+    const int cnt0 = dense ? Hp : k.ccnt[c];
     const int lane_id = balanced_lane(cnt0 > ks ? (cnt0 - 1 - ks) / NCK + 1 : 0, tid,
                                       nthr, perm, perm + nthr);
     sks = lane_id / JW;
     so = lane_id % JW;
     const int sc = p * JW + so;
-    const int cnt = k.ccnt[sc];
+    const int cnt = dense ? Hp : k.ccnt[sc];
     nslot = wave_max(cnt > sks ? (cnt - 1 - sks) / NCK + 1 : 0);
     int ix[RCP];
 #pragma unroll
@@ -4386,9 +4387,10 @@ __global__ __launch_bounds__(1024) void ode_fwd_cl2_kernel(FwdCK k) {
         ix[rr] = 0;
         continue;
       }
-      const long long a = (long long)(sks * RC + rr) * Hp + sc;
-      preg[rr] = k.cimg[a];
-      ix[rr] = k.cidx[a] * NB * 4;
+      const int row = rr * NCK + sks;
+      const long long a = (long long)(dense ? row : sks * RC + rr) * Hp + sc;
+      preg[rr] = dense ? k.recF[a] : k.cimg[a];
+      ix[rr] = (dense ? row : k.cidx[a]) * NB * 4;
     }
 #pragma unroll
     for (int q = 0; q < RCP / 4; ++q)
@@ -4618,22 +4620,29 @@ __global__ __launch_bounds__(1024) void ode_fwd_own_kernel(FwdCK k) {
   unsigned long long* xbase = k.xch + (long long)cl * 2 * Hp;
   const float C = k.neuron[c], G = k.neuron[Hp + c], L = k.neuron[2 * Hp + c];
   const float GL = G * L, CG = C + G;
-  const int cnt = k.ccnt[c];
+  const bool dense = k.cimg == nullptr;
+  const int cnt = dense ? Hp : k.ccnt[c];
   const int nslot = wave_max(cnt > ck ? (cnt - 1 - ck) / LPC + 1 : 0);
   float4 preg[RCP];
   unsigned ix[RCP / 2];
+  auto load = [&](const float4* img, bool dense) {
 #pragma unroll
-  for (int rr = 0; rr < RCP; ++rr) {
-    // slots past the image's RC but within the last group of ZG
-    preg[rr] = make_float4(kMinSlope, 0.f, 0.f, 0.f);
-    unsigned o = 0;
-    if (rr < RC) {
-      const int a = (ck * RC + rr) * Hp + c;
-      preg[rr] = k.cimg[a];
-      o = (unsigned)k.cidx[a] * 4u;
+    for (int rr = 0; rr < RCP; ++rr) {
+      // slots past the image's RC but within the last group of ZG
+      preg[rr] = make_float4(kMinSlope, 0.f, 0.f, 0.f);
+      unsigned o = 0;
+      if (rr < RC) {
+        const int row = rr * LPC + ck, a = (dense ? row : ck * RC + rr) * Hp + c;
+        preg[rr] = img[a];
+        o = (unsigned)(dense ? row : k.cidx[a]) * 4u;
+      }
+      ix[rr >> 1] = (rr & 1) ? (ix[rr >> 1] | (o << 16)) : o;
     }
-    ix[rr >> 1] = (rr & 1) ? (ix[rr >> 1] | (o << 16)) : o;
-  }
+  };
+  if (dense)
+    load(k.recF, true);
+  else
+    load(k.cimg, false);
   if (tid == 0) gave_up = nanrow[0] = nanrow[1] = 0;
   __syncthreads();
   for (int j = tid; j < Hp; j += NT) {
@@ -5507,7 +5516,10 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   }
   const int RC = REG ? k.RC : RCP;  // slots of a chunk
   if ((CP - 1) * PERG > XW * 512) return;  // the host's geometry keeps to it
-  const int cntc = REG ? k.ccnt[c] : 0;
+  // REG without a compacted image (RegCluster::dense): entry e of a column is row e
+  const bool dense = REG && !FACT && k.cimg == nullptr;
+  auto count = [&](int col) { return dense ? Hp : k.ccnt[col]; };
+  const int cntc = REG ? count(c) : 0;
   auto pden_at = [&](long long m) { return pden + (m & 1) * NB * Hp; };
   auto pv_at = [&](long long m) { return pv + (m % 3) * NB * Hp; };
   // v slot r (an unfold index mod 3, kept by the loop instead of divided)
@@ -5525,18 +5537,19 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   unsigned ix[PACK ? RCP / 2 : RCP];
   int nmine, nslot, sks, so;
   {
-    const int cnt0 = k.ccnt[c];
+    const int cnt0 = count(c);
     const int lane_id = balanced_lane<RCP <= 16 ? 16 : RCP>(cnt0 > ks ? (cnt0 - 1 - ks) / kCmpChunks + 1 : 0, tid,
                                       nthr, perm, perm + nthr);
     sks = lane_id / JW;
     so = lane_id - sks * JW;
-    const int cnt = k.ccnt[p * JW + so];
+    const int cnt = count(p * JW + so);
     nmine = cnt > sks ? (cnt - 1 - sks) / kCmpChunks + 1 : 0;
     nslot = wave_max(nmine);
 #pragma unroll
     for (int rr = 0; rr < RCP; ++rr) {
-      const long long a = (long long)(sks * RC + rr) * Hp + p * JW + so;
-      const float4 q = k.cimg[a];
+      const int row = rr * kCmpChunks + sks;
+      const long long a = (long long)(dense ? row : sks * RC + rr) * Hp + p * JW + so;
+      const float4 q = dense ? k.recB[a] : k.cimg[a];
       // image operands (x, y, w E, w) -> (x, y, E, w x); an entry with
       // w = 0 (a padding slot) contributes nothing either way
       preg[rr] = FACT ? make_float4(q.x, q.y, q.w != 0.f ? q.z / q.w : 0.f, q.w * q.x) : q;
@@ -5544,7 +5557,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
         preg[rr].x = kMinSlope;
         preg[rr].y = 0.f;
       }
-      const unsigned of = (unsigned)(k.cidx[a] * ABS * 8);
+      const unsigned of = (unsigned)((dense ? row : k.cidx[a]) * ABS * 8);
       if constexpr (PACK)
         ix[rr >> 1] = (rr & 1) ? (ix[rr >> 1] | (of << 16)) : of;
       else
@@ -5888,7 +5901,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   for (int rr = 0; rr < RCP; ++rr) {
     if (rr < nmine) {
       const long long a = (long long)(sks_end * RC + rr) * Hp + sc;
-      const int j = k.cidx[a];
+      const int j = dense ? rr * kCmpChunks + sks_end : k.cidx[a];
       const float w = FACT ? k.cimg[a].w : 1.f;  // the factor the last two sums left out
       float4 s = make_float4(gacc[rr].x, gacc[rr].y, gacc[rr].z * w, gacc[rr].w * w);
       if (REG && k.R0 > 0) {  // a later launch of the call adds to the cluster's partial
@@ -6092,9 +6105,11 @@ hipError_t launch_reg_bwd_mv(const Plan& p, BwdCK a, hipStream_t s) {
     return hipGetLastError();
   }
   // The kernel over at most reg_chain_slots synapses a thread, then the one
-  // that streams them all: one of the two leaves at its first check.
-  a.maxcnt = 16 * reg_chain_slots(g.RC);
-  if (reg_chain_slots(g.RC) == 16)
+  // that streams them all: one of the two leaves at its first check. Without a
+  // compacted image only the latter.
+  a.maxcnt = g.dense ? 0 : 16 * reg_chain_slots(g.RC);
+  if (g.dense) {
+  } else if (reg_chain_slots(g.RC) == 16)
     LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 16, true, true, MOVE>), grid, block, lds, s, a);
   else
     LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 20, true, true, MOVE>), grid, block, lds, s, a);
@@ -6283,11 +6298,12 @@ hipError_t launch_ode_fwd_after(const Plan& p, const Prepped& pp, const float* s
                                 const int* gate, hipStream_t s) {
   if (gate != nullptr && (p.rf.CP > 0 || p.CP > 0)) return hipErrorInvalidValue;
   if (p.rf.CP > 0) {
-    if (pp.cF == nullptr || pp.cFi == nullptr || pp.cFn == nullptr) return hipErrorInvalidValue;
     const RegCluster& g = p.rf;
+    if (!g.dense && (pp.cF == nullptr || pp.cFi == nullptr || pp.cFn == nullptr))
+      return hipErrorInvalidValue;
     FwdCK a{pp.recF, pp.neuron, sn, sd, state0, out, hfin, vsave, densave, cb.xch, cb.status,
             cb.spin, p.B, p.T, p.H, p.Hp, p.U, g.KS, g.RC, g.CP, 0, eps,
-            pp.cF, pp.cFi, pp.cFn, 0, g.NCL};
+            g.dense ? nullptr : pp.cF, pp.cFi, pp.cFn, 0, g.NCL};
     for (int l = 0; l < g.L; ++l) {
       hipError_t e = clear_cluster(p, cb, false, s, l == 0);
       if (e != hipSuccess) return e;
@@ -6355,11 +6371,13 @@ hipError_t launch_ode_bwd_after(const Plan& p, const Prepped& pp, const float* v
                                 const int* gate, hipStream_t s) {
   if (gate != nullptr && (p.rb.CP > 0 || p.CP > 0 || absave == nullptr)) return hipErrorInvalidValue;
   if (p.rb.CP > 0) {
-    if (pp.cB == nullptr || pp.cBi == nullptr || pp.cBn == nullptr) return hipErrorInvalidValue;
     const RegCluster& g = p.rb;
+    if (!g.dense && (pp.cB == nullptr || pp.cBi == nullptr || pp.cBn == nullptr))
+      return hipErrorInvalidValue;
     BwdCK a{pp.recB, pp.neuron, vsave, densave, gout, gs, ghfin, absave, dsn, dsd, npart,
             gstate, rpart, cb.xch, cb.status, cb.spin, p.B, p.T, p.H, p.Hp, p.U, g.KS, g.RC,
-            g.CP, g.xcd ? 1 : 0, pp.cB, pp.cBi, pp.cBn, 0, g.NCL, 0, cb.gsum, g.FL};
+            g.CP, g.xcd ? 1 : 0, g.dense ? nullptr : pp.cB, pp.cBi, pp.cBn, 0, g.NCL, 0, cb.gsum,
+            g.FL};
     if (g.FL > 0 && cb.gsum == nullptr) return hipErrorInvalidValue;
     for (int l = 0; l < g.L; ++l) {
       hipError_t e = clear_cluster(p, cb, true, s, l == 0);

@@ -70,9 +70,11 @@ enum KernelId : int {
 // whole rounds of eight clusters, still holds at most one workgroup per CU).
 // FL (chain): unfolds after which the gradient sums move from the registers to
 // ClusterBuf::gsum, 0 for never.
+// dense: no compacted image; the threads take their synapses from the dense one
+// (a chain of more than 16 slots a thread streams it).
 struct RegCluster {
   int CP, JW, KS, RC, NB, NCL, L, FL;
-  bool xcd;
+  bool xcd, dense;
 };
 
 // Workgroups of a register-resident launch: with every cluster on one XCD the
@@ -465,8 +467,8 @@ inline long long row_bwd_words(const Plan& p) {
 }
 // Whether the forward launch reads a compacted image: the plan's own forms
 // (cmp_fwd) or the register-resident clusters.
-inline bool fwd_image_cmp(const Plan& p) { return p.rf.CP > 0 || cmp_fwd(p); }
-inline bool bwd_image_cmp(const Plan& p) { return p.rb.CP > 0 || cmp_bwd(p); }
+inline bool fwd_image_cmp(const Plan& p) { return p.rf.CP > 0 ? !p.rf.dense : cmp_fwd(p); }
+inline bool bwd_image_cmp(const Plan& p) { return p.rb.CP > 0 ? !p.rb.dense : cmp_bwd(p); }
 inline int cmp_chunks_fwd(const Plan& p) {
   if (p.rf.CP > 0) return p.rf.KS;
   return (row_kernels(p) || row_wave128_fwd(p)) ? 4 : (p.CP > 0 ? kCmpChunks : p.KS);

@@ -78,7 +78,7 @@ class CApi:
                    "module_row128_rec_fused", "launches_fwd", "launches_bwd", "sens_full_list",
                    "reg_fwd_members", "reg_fwd_cols", "reg_fwd_rows", "reg_fwd_launches",
                    "reg_fwd_lds", "reg_bwd_members", "reg_bwd_rows", "reg_bwd_launches",
-                   "reg_bwd_lds", "reg_bwd_move")
+                   "reg_bwd_lds", "reg_bwd_move", "reg_fwd_dense", "reg_bwd_dense")
 
     def __init__(self, path: str = LIB_PATH):
         self.path = path

@@ -497,3 +497,19 @@ def test_chain_sums_are_bounded(capi, B, T, H):
     parts = max(1, min(64, -(-1024 // ((p["Hp"] // 64) * (p["Hp"] // 32))), -(-n // 32)))
     assert terms <= max(48, -(-n // parts)) + nb
     assert fl == 0 or 48 <= nb * fl and fl < T * 6
+
+
+@pytest.mark.parametrize("H", [192, 256, 320, 448, 512])
+def test_short_calls(capi, H):
+    """Calls of several launches and two unfolds run the plan's own kernels, of
+    three only where those leave the chip idle; what was one launch stays so."""
+    for B in (600, 1024):
+        for T, U in ((1, 1), (1, 2), (2, 1), (1, 3), (4, 1), (1, 6)):
+            p, q = capi.plan(B, T, 8, H, U), capi.plan(B, 8, 8, H, U)
+            short = T * U <= 2 or (T * U == 3 and B == 1024)
+            for way in ("fwd", "bwd"):
+                if q[f"reg_{way}_launches"] > 1:
+                    assert (p[f"reg_{way}_members"] == 0) == short, (B, T, U, p)
+    for B in (1, 16, 64):
+        p = capi.plan(B, 1, 8, H, 1)
+        assert p["reg_fwd_members"] > 0 or H == 256

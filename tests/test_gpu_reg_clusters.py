@@ -90,15 +90,18 @@ def test_nan_state_reaches_its_whole_row(shape, U):
     assert torch.isfinite(out[:B - 1]).all()
 
 
-@pytest.mark.parametrize("shape", [(1, 1, 8, 192), (90, 1, 4, 192), (1, 1, 4, 300),
-                                   (60, 1, 4, 320), (5, 1, 4, 448), (300, 1, 4, 256)],
-                         ids=lambda s: "B%dT%dD%dH%d" % s)
+# (B, T, D, H, whether the forward reads the dense image)
+@pytest.mark.parametrize("shape", [(1, 5, 8, 192, 0), (1, 1, 8, 192, 1), (90, 1, 4, 192, 0),
+                                   (1, 5, 4, 300, 0), (60, 2, 4, 320, 0), (60, 1, 4, 320, 1),
+                                   (5, 11, 4, 448, 0), (5, 1, 4, 448, 1), (300, 1, 4, 256, 0)],
+                         ids=lambda s: "B%dT%dD%dH%ddense%d" % s)
 @pytest.mark.parametrize("i", [0, 7])
 def test_infinite_state_saturates_its_gates(shape, i):
     """An infinite v_i makes the gates of its synapses 0 or 1, whatever slot holds
     them or pads a column: every other neuron stays finite and equals the oracle."""
-    B, T, D, H = shape
-    assert ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)["reg_fwd_members"] > 0
+    B, T, D, H, dense = shape
+    p = ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)
+    assert p["reg_fwd_members"] > 0 and p["reg_fwd_dense"] == dense
     args = _edge_masks(boundary(B, T, D, H, seed=14))
     h0 = args[1].clone()
     h0[0, i] = float("inf")
@@ -113,8 +116,9 @@ def test_infinite_state_saturates_its_gates(shape, i):
         assert (got - ref[..., keep]).abs().max().item() <= 5e-6
 
 
-@pytest.mark.parametrize("shape", [(2, 1, 4, 192), (90, 1, 4, 192), (2, 1, 4, 320),
-                                   (60, 1, 4, 320), (300, 1, 4, 256)],
+@pytest.mark.parametrize("shape", [(2, 1, 4, 192), (2, 30, 4, 192), (90, 1, 4, 192), (2, 1, 4, 320),
+                                   (2, 30, 4, 320), (60, 1, 4, 320), (60, 10, 4, 320),
+                                   (300, 1, 4, 256)],
                          ids=lambda s: "B%dT%dD%dH%d" % s)
 @pytest.mark.parametrize("leaf,value", [("mu", float("nan")), ("sigma", float("nan")),
                                         ("mu", float("inf"))])
@@ -126,7 +130,7 @@ def test_non_finite_operand_at_a_masked_synapse(shape, leaf, value):
     m = _perturbed_module(D, H, seed=6).to(DEV)
     m.ode_unfolds = 1
     p = ltc_cuda._cuda_module.capi.plan(B, T, D, H, 1)
-    assert p["reg_fwd_members"] > 0
+    assert p["reg_fwd_members"] > 0 and p["reg_fwd_dense"] == (T == 1 and B < 90)
     with torch.no_grad():
         m.sparsity_mask[5, 9] = m.sparsity_mask[H - 1, H - 1] = 0.0
         getattr(m, leaf)[5, 9] = value
@@ -246,7 +250,7 @@ def test_non_finite_gradient_reaches_its_whole_row(shape, value):
     assert torch.equal(dirty[keep], clean[keep])
 
 
-@pytest.mark.parametrize("shape", [(5, 2, 6, 192), (40, 1, 4, 320)], ids=lambda s: "B%dT%dD%dH%d" % s)
+@pytest.mark.parametrize("shape", [(5, 2, 6, 192), (40, 3, 4, 320)], ids=lambda s: "B%dT%dD%dH%d" % s)
 @pytest.mark.parametrize("sigma,mu", [(0.0, 0.5), (1e-22, 0.5), (1e-22, 1e22), (-1e-21, 2e21),
                                       (1e-15, 1e15)])
 def test_gradients_at_a_vanishing_slope(shape, sigma, mu):
@@ -296,3 +300,103 @@ def test_gradient_sums_of_long_sequences(shape):
         err = ((q - r_g[n]).norm() / r_g[n].norm()).item()
         print(f"{shape} {n}: {err:.2e}", flush=True)
         assert err <= 4.3e-7, f"{n}: {err:.1e}"
+
+
+# (B, T, D, H, density, dense forward, dense chain, register chain): both sides of
+# the rules for the image that forward and chain read, and of the slot limit
+IMAGES = [(1, 4, 8, 192, 0.5, 1, 0, 1), (1, 5, 8, 192, 0.5, 0, 0, 1), (86, 1, 5, 130, 0.5, 0, 0, 1),
+          (3, 2, 70, 257, 0.5, 1, 1, 0), (3, 3, 70, 257, 0.5, 1, 0, 1), (3, 5, 70, 257, 0.5, 0, 0, 1),
+          (52, 1, 5, 320, 0.5, 1, 1, 0), (52, 2, 5, 320, 0.5, 0, 0, 1), (52, 2, 5, 320, 1.0, 0, 0, 0),
+          (5, 10, 5, 400, 0.5, 1, 0, 1), (5, 11, 5, 400, 0.5, 0, 0, 1), (9, 3, 5, 500, 0.5, 1, 0, 1),
+          (33, 1, 5, 512, 0.5, 1, 1, 0), (33, 2, 5, 512, 0.5, 0, 0, 1)]
+
+
+@pytest.mark.parametrize("shape", IMAGES, ids=lambda s: "B%dT%dD%dH%dp%g" % s[:5])
+def test_dense_and_compacted_images(shape):
+    B, T, D, H, density, df, db, reg = shape
+    p = ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)
+    assert (p["reg_fwd_dense"], p["reg_bwd_dense"]) == (df, db), p
+    m = _perturbed_module(D, H, seed=B + T, sparsity=density).to(DEV)
+    # the register chain takes columns (rows of the mask) of at most 16 slots a
+    # thread in 16 chunks, 20 above Hp = 448
+    limit = p["Hp"] if p["Hp"] <= 256 else (256 if p["Hp"] <= 448 else 320)
+    fits = int((m.sparsity_mask != 0).sum(1).max()) <= limit
+    assert reg == (fits and not db)
+    g = torch.Generator().manual_seed(23)
+    x = torch.randn(B, T, D, generator=g)
+    h0 = torch.randn(B, H, generator=g) * 0.2
+    G = torch.randn(B, T, H, generator=g)
+    xg, hg = x.to(DEV).requires_grad_(True), h0.to(DEV).requires_grad_(True)
+    out, _ = m(xg, (hg, hg))
+    (out * G.to(DEV)).sum().backward()
+    r_out, _, r_g, r_gx, r_gh = _oracle_module_grads(m, x, h0, G, torch.zeros(B, H))
+    assert (out.detach().cpu().double() - r_out).abs().max().item() <= 5e-6
+    for name, a, b in ([("x", xg.grad, r_gx), ("h0", hg.grad, r_gh)]
+                       + [(n, q.grad, r_g[n]) for n, q in m.named_parameters()]):
+        err = ((a.cpu().double() - b).norm() / b.norm()).item()
+        assert err <= 2e-5, f"{name}: {err:.1e}"
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 8, 192), (64, 2, 8, 320), (40, 1, 8, 500), (3, 10, 4, 512)],
+                         ids=lambda s: "B%dT%dD%dH%d" % s)
+def test_boundary_gradients(shape):
+    """A backward over the boundary tensors wants every synapse's gradients: dense
+    columns, whatever the image rule says."""
+    B, T, D, H = shape
+    args = _edge_masks(boundary(B, T, D, H, seed=7))
+    dev_args, (out, h, saved) = gpu_forward(args, save=True)
+    g = torch.Generator().manual_seed(8)
+    g_out, g_h = torch.randn(B, T, H, generator=g), torch.randn(B, H, generator=g)
+    got = gpu_backward(dev_args, saved, g_out.to(DEV), g_h.to(DEV))
+    assert_grads_close(got, oracle_grads(args, g_out, g_h), f"{shape}")
+
+
+@pytest.mark.parametrize("shape", [(60, 2, 4, 384), (6, 3, 4, 320)], ids=lambda s: "B%dT%dD%dH%d" % s)
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_non_finite_gradient_in_the_compacted_chain(shape, value):
+    """As test_non_finite_gradient_reaches_its_whole_row, at the last of several
+    steps."""
+    B, T, D, H = shape
+    assert ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)["reg_bwd_dense"] == 0
+    m = _perturbed_module(D, H, seed=4).to(DEV)
+    x = torch.randn(B, T, D, generator=torch.Generator().manual_seed(1)).to(DEV)
+    h0 = torch.zeros(B, H, device=DEV, requires_grad=True)
+    out, _ = m(x, (h0, h0))
+    G = torch.ones(B, T, H, device=DEV)
+    clean, = torch.autograd.grad(out, h0, G, retain_graph=True)
+    G[3, T - 1, 0] = value
+    dirty, = torch.autograd.grad(out, h0, G)
+    assert not torch.isfinite(dirty[3]).any()
+    keep = [b for b in range(B) if b != 3]
+    assert torch.equal(dirty[keep], clean[keep])
+
+
+@pytest.mark.parametrize("shape", [(6, 4, 5, 320), (6, 4, 5, 512)], ids=lambda s: "B%dT%dD%dH%d" % s)
+def test_a_weight_that_cannot_be_factored_out_takes_the_streaming_chain(shape):
+    """|erev| above 1e18 at a weight of e^-80: a synapse worth 1e-17, so every other
+    gradient is the same to a rounding, but the register chain, which divides by
+    the weight, may not run. Which one ran shows in the last bits."""
+    B, T, D, H = shape
+    assert ltc_cuda._cuda_module.capi.plan(B, T, D, H, 6)["reg_bwd_dense"] == 0
+    m = _perturbed_module(D, H, seed=12).to(DEV)
+    with torch.no_grad():
+        m.sparsity_mask[6, 5] = 1.0
+        m.w[6, 5] = -80.0
+    x = torch.randn(B, T, D, generator=torch.Generator().manual_seed(2)).to(DEV)
+    h0 = torch.zeros(B, H, device=DEV)
+    res = []
+    for erev in (1.0, 5e17, 2e18):
+        with torch.no_grad():
+            m.erev[6, 5] = erev
+        m.zero_grad(set_to_none=True)
+        out, _ = m(x, (h0, h0))
+        out.sum().backward()
+        gs = [m.mu.grad.clone(), m.sigma.grad.clone(), m.erev.grad.clone()]
+        for t in gs:
+            t[6, 5] = 0.0
+        res.append(gs)
+    one, below, above = res
+    for a, b, c in zip(one, below, above):
+        assert torch.equal(a, b)
+        assert not torch.equal(a, c)
+        assert ((a - c).norm() / a.norm()).item() <= 1e-5
