@@ -5448,43 +5448,15 @@ __global__ __launch_bounds__(FUSE ? 512 : 1024) void ode_bwd_cl_kernel(BwdCK k) 
 // sums of each synapse take the rows in the same order as the one-group
 // kernel; a slot's operands are (x, y, E, w x), w factored out of dL/darg
 // (bwd_synapse_cmpe), and its alpha/beta row offset stays in a register.
-//
-// REG: the register-resident clusters beyond that form: 12 or 16 slots cover
-// Hp = 192 or 256, 16 slots Hp = 320 ... 448 and 20 Hp = 512 while no column
-// has more than 16 * RCP entries (half-dense masks; a second launch, of
-// ode_bwd_cl_kernel, covers the rest). Bound by the slot loops at two waves per
-// SIMD and the exchange of up to 16 members: B64 T32 H192 554 us (chain 996
-// and rec_grad 205 before), H512 1104 us (1868). Partials are written slot by
-// slot: through store_partials32's tile, whole planes of which half is padding,
-// B64 T32 H512 took 1124 instead of 1111 us and B256 T4 H512, whose two
-// launches add, 676 instead of 640. FACT factors w out as above, which needs
-// w != 0 wherever wE is (kChainIrregular otherwise); without it the operands
-// stay (x, y, wE, w).
-// REG's fourth sum is that of dl * zp, zp = x v + y the gate's argument, not of
-// dl * v: the sigma gradient is sum dl (v - mu), and summed as sum dl v less mu
-// sum dl its terms cancel only after hundreds of rounded additions (B64 T32
-// H192: error against float64 2.2e-6, 1.3e-6 with rec_grad_kernel's shorter
-// sums). A slope x below kMinSlope is raised to it so that sum dl v can be
-// taken out again at the end, unless the offset y counts beside it: then
-// |mu| = |y / x| > 1e12, and sum dl v, nothing beside mu sum dl, is left out.
-// (A gate argument past the float range, |sigma (v - mu)| > 2e38, makes that
-// synapse's sigma gradient NaN.)
-// REG keeps the dense kernels' treatment of a non-finite alpha or beta: the
-// synapses left out have weight zero, and zero times it is NaN, so dL/dv of
-// every neuron of that row that has such a synapse becomes NaN. A row flag by
-// unfold parity carries it, as the forward's does a NaN state.
-template <int NB, int RCP = 16, bool FACT = true, bool REG = false, bool MOVE = false>
+template <int NB>
 __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   static_assert(NB == 2 || NB == 4 || NB == 8, "two groups of rows");
-  constexpr int JW = 32, HB = NB / 2, PER = NB * JW, PERG = HB * JW;
+  constexpr int JW = 32, RCP = 16, HB = NB / 2, PER = NB * JW, PERG = HB * JW;
   constexpr int ABS = NB + 2;  // padded alpha/beta rows, as in ode_bwd_cl_kernel
-  constexpr int HPC = 16 * RCP;  // Hp, without REG
-  // gather words per thread and group: (CP - 1) * PERG <= XW * 512
-  // (CP = 8 without REG, at most 8 without FACT, 16 with both)
-  constexpr int XW = !REG ? 2 : (FACT ? NB / 2 : (NB == 8 ? 2 : 1));
+  constexpr int HPC = 16 * RCP;  // Hp = 256
+  constexpr int XW = 2;          // gather words per thread and group: (CP-1)*PERG <= 2*512
   extern __shared__ float4 lds4[];
   __shared__ int gave_up;
-  __shared__ int badrow[2][NB];  // REG: alpha/beta of that unfold parity not finite
   const int Hp = k.Hp, H = k.H, KS = k.KS, B = k.B, T = k.T, U = k.U, CP = k.CP;
   float2* ab = reinterpret_cast<float2*>(lds4);                  // [Hp][ABS]
   float* red = reinterpret_cast<float*>(ab + ABS * Hp);         // [2][KS][HB][JW]
@@ -5493,9 +5465,6 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   // [4][threads] int4 of the compacted kernels' slot table, of which this
   // kernel only uses the space after it (balanced_lane's scratch)
   int4* slot_tab = reinterpret_cast<int4*>(pv + 3 * NB * Hp);
-  // REG: balanced_lane's scratch directly
-  int* perm = REG ? reinterpret_cast<int*>(slot_tab)
-                  : reinterpret_cast<int*>(slot_tab + (RCP / 4) * 512);
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int ks = tid / JW, o = tid % JW;
   int p, cl;
@@ -5509,17 +5478,396 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   const long long BHp = (long long)B * Hp;
   const float C = k.neuron[c];
   if (T == 0) return;
-  if constexpr (REG) {
-    if (cl >= k.NCL) return;  // grid padded to whole rounds of the XCDs
-    if (k.maxcnt > 0 && !chain_counts_fit(k.ccnt, Hp, k.maxcnt)) return;
-    if (tid < 2 * NB) badrow[tid / NB][tid % NB] = 0;  // before balanced_lane's barriers
+  auto pden_at = [&](long long m) { return pden + (m & 1) * NB * Hp; };
+  auto pv_at = [&](long long m) { return pv + (m % 3) * NB * Hp; };
+  // v slot r (an unfold index mod 3, kept by the loop instead of divided)
+  auto pv_slot = [&](int r) { return pv + r * NB * Hp; };
+  auto mod3_next = [](int r) { return r == 2 ? 0 : r + 1; };
+  auto mod3_prev = [](int r) { return r == 0 ? 2 : r - 1; };
+
+  float4 preg[RCP];
+  int ix[RCP];  // slot row offsets, in registers
+  int nmine, nslot, sks, so;
+  {
+    int* perm = reinterpret_cast<int*>(slot_tab + (RCP / 4) * nthr);
+    const int cnt0 = k.ccnt[c];
+    const int lane_id = balanced_lane(cnt0 > ks ? (cnt0 - 1 - ks) / kCmpChunks + 1 : 0, tid,
+                                      nthr, perm, perm + nthr);
+    sks = lane_id / JW;
+    so = lane_id - sks * JW;
+    const int cnt = k.ccnt[p * JW + so];
+    nmine = cnt > sks ? (cnt - 1 - sks) / kCmpChunks + 1 : 0;
+    nslot = wave_max(nmine);
+#pragma unroll
+    for (int rr = 0; rr < RCP; ++rr) {
+      const long long a = (long long)(sks * RCP + rr) * Hp + p * JW + so;
+      // image operands (x, y, w E, w) -> (x, y, E, w x); an entry with
+      // w = 0 (a padding slot) contributes nothing either way
+      const float4 q = k.cimg[a];
+      preg[rr] = make_float4(q.x, q.y, q.w != 0.f ? q.z / q.w : 0.f, q.w * q.x);
+      ix[rr] = k.cidx[a] * ABS * 8;
+    }
   }
-  const int RC = REG ? k.RC : RCP;  // slots of a chunk
-  if ((CP - 1) * PERG > XW * 512) return;  // the host's geometry keeps to it
-  // REG without a compacted image (RegCluster::dense): entry e of a column is row e
-  const bool dense = REG && !FACT && k.cimg == nullptr;
+  const int sc = p * JW + so;
+  float4 gacc[RCP];
+#pragma unroll
+  for (int rr = 0; rr < RCP; ++rr) gacc[rr] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (tid == 0) gave_up = 0;
+
+  // Owner state, as in ode_bwd_cl_kernel.
+  float g = 0.f, gdir = 0.f, accA = 0.f, accB = 0.f, pC = 0.f, pGv = 0.f, pA = 0.f;
+  auto own_ab = [&](float den, float vk, float vk1) {
+    float al = 0.f, be = 0.f;
+    gdir = 0.f;
+    if (live && c < H) {
+      al = g * den;  // saved 1/den
+      be = -g * vk1 * den;
+      accA += al;
+      accB += be;
+      pC += al * (vk - vk1);
+      pGv += al * vk1;
+      pA += al;
+      gdir = al * C;
+    }
+    ab[c * ABS + bo] = make_float2(al, be);
+  };
+  auto gout_at = [&](int b, int t, int col) {
+    return k.gout[(long long)(b0 + b) * k.gs.b + (long long)t * k.gs.t + (long long)col * k.gs.c];
+  };
+  auto prefetch = [&](long long m) {  // 1/den of unfold m, v of slot m
+    rows_to_lds_fixed<NB, HPC, 512>(k.densave + m * BHp, b0, B, pden_at(m), tid);
+    rows_to_lds_fixed<NB, HPC, 512>(k.vsave + m * BHp, b0, B, pv_at(m), tid);
+  };
+
+  const long long n_last = (long long)T * U - 1;
+  // Unfold n_last's alpha/beta of every column from the output gradients.
+  if (owner) {
+    if (live && c < H) {
+      g = gout_at(bo, T - 1, c);
+      if (k.ghfin != nullptr) g += k.ghfin[(long long)(b0 + bo) * H + c];
+    }
+    float den = 1.f, vk = 0.f, vk1 = 0.f;
+    if (live) {
+      const long long e = (n_last * B + b0 + bo) * Hp + c;
+      den = k.densave[e];
+      vk = k.vsave[e];
+      vk1 = k.vsave[e + BHp];
+    }
+    own_ab(den, vk, vk1);
+  }
+  for (int e = tid; e < (CP - 1) * PER; e += nthr) {
+    const int q = e / PER, r = e - q * PER, b = r / JW;
+    const int col = (q + (q >= p ? 1 : 0)) * JW + (r - b * JW);
+    float al = 0.f, be = 0.f;
+    if (b0 + b < B && col < H) {
+      float gg = gout_at(b, T - 1, col);
+      if (k.ghfin != nullptr) gg += k.ghfin[(long long)(b0 + b) * H + col];
+      const long long ee = (n_last * B + b0 + b) * Hp + col;
+      const float rden = k.densave[ee];
+      al = gg * rden;
+      be = -gg * k.vsave[ee + BHp] * rden;
+    }
+    ab[col * ABS + b] = make_float2(al, be);
+  }
+  // The prefetched rows the first three phases read: v of slots n_last and
+  // n_last - 1, 1/den of unfold n_last - 1.
+  rows_to_lds_fixed<NB, HPC, 512>(k.vsave + n_last * BHp, b0, B, pv_at(n_last), tid);
+  if (n_last > 0) prefetch(n_last - 1);
+  wait_vm();
+  lds_barrier();
+
+  // This thread's gather words (x < XW): partner member, row of the group, column.
+  int gm[XW], gr[XW], gcl[XW];
+  bool gth[XW];
+#pragma unroll
+  for (int x = 0; x < XW; ++x) {
+    const int e = tid + x * nthr;
+    // With two or more rows per group the word count (CP - 1) * PERG is a
+    // multiple of 64, so a wave gathers all its words or none: a scalar
+    // branch instead of a lane mask.
+    if constexpr (HB >= 2)
+      gth[x] = __builtin_amdgcn_readfirstlane(e) < (CP - 1) * PERG;
+    else
+      gth[x] = e < (CP - 1) * PERG;
+    const int q = e / PERG, r = e - q * PERG;
+    gm[x] = q + (q >= p ? 1 : 0);
+    gr[x] = r / JW;
+    gcl[x] = gm[x] * JW + (r - gr[x] * JW);
+  }
+  bool pend = false;  // owners: their group's finish is due
+  long long pn = 0;
+  int pn3 = 0, pt = 0, pu = 0;  // pn mod 3, its step and unfold within the step
+  float gnext = 0.f;
+  // step t, unfold u within it and n mod 3, stepped with n
+  int t = T - 1, u = U - 1, n3 = (int)(n_last % 3);
+  for (long long n = n_last; n >= 0; --n) {
+#pragma unroll
+    for (int gi = 0; gi < 2; ++gi) {
+      // (e) the owners of the previous phase's group: dL/dv^{pn}, published
+      // for the partners' alpha/beta of unfold pn - 1.
+      bool own_next = false;
+      if (pend) {
+        pend = false;
+        const float* rg = red + og * KS * HB * JW;
+        const float s = ks_sum_wide(rg + (bo - og * HB) * JW + o, HB * JW, KS);
+        g = c < H ? fmaf(kNegLn2, s, gdir) : 0.f;
+        if (pn > 0) {
+          g += gnext;
+          const unsigned tag = (unsigned)pn;
+          xch_put(xbase + (long long)(tag & 1) * CP * PER + p * PER + bo * JW + o, g, tag);
+          own_next = true;
+        }
+        if (pu == 0 && live) {
+          const long long e = ((long long)(b0 + bo) * T + pt) * Hp + c;
+          k.dsn[e] = accA;
+          k.dsd[e] = accB;
+        }
+        if (pu == 0) accA = accB = 0.f;
+      }
+      // The output gradient entering at this unfold's step boundary.
+      if (owner && og == gi) gnext = (n > 0 && u == 0 && live && c < H) ? gout_at(bo, t - 1, c) : 0.f;
+      // (a) group gi's synapses at unfold n; the other group's newest words
+      // are loaded halfway: group 0's dL/dv^n while running group 1, group
+      // 1's dL/dv^{n+1} while running group 0.
+      const int gg = 1 - gi;
+      const long long gtag = gi == 1 ? n : n + 1;
+      const bool need = gi == 1 ? n > 0 : n < n_last;
+      const long long am = gtag - 1;  // the unfold whose alpha/beta the words rebuild
+      unsigned long long* gslot = xbase + (long long)(gtag & 1) * CP * PER;
+      unsigned long long w[XW];
+      // 1/den and v^{am+1} of the gathered words' rows and columns, read
+      // from LDS when the word loads are issued, so that the rebuild after
+      // the poll does not wait for LDS
+      float rdn[XW], rvk[XW], odn = 0.f, ovk = 0.f, ovk1 = 0.f;
+      const float* dn = pden_at(am);
+      const float* vk1 = pv_slot(gi == 1 ? n3 : mod3_next(n3));  // slot am + 1 = gtag
+      float cvi[HB], acc[HB];
+      // The slot count, opaque to the compiler here: otherwise it keeps the
+      // slot branches' conditions as lane masks across the loop, which spill
+      // and are reloaded every phase.
+      int nsl = nslot;
+      asm volatile("" : "+s"(nsl));
+      const float* vn = pv_slot(n3);
+#pragma unroll
+      for (int b = 0; b < HB; ++b) {
+        cvi[b] = b0 + gi * HB + b < B ? vn[(gi * HB + b) * Hp + sc] : 0.f;
+        acc[b] = 0.f;
+      }
+#pragma unroll
+      for (int q = 0; q < RCP / 4; ++q) {
+        if (q == RCP / 8) {
+#pragma unroll
+          for (int x = 0; x < XW; ++x)
+            if (need && gth[x])
+              w[x] = xch_get(gslot + gm[x] * PER + (gg * HB + gr[x]) * JW + (gcl[x] - gm[x] * JW));
+#pragma unroll
+          for (int x = 0; x < XW; ++x) {
+            rdn[x] = rvk[x] = 0.f;
+            if (need && gth[x]) {
+              const int e = (gg * HB + gr[x]) * Hp + gcl[x];
+              rdn[x] = dn[e];
+              rvk[x] = vk1[e];
+            }
+          }
+          // the owners' own entry likewise
+          if (own_next) {
+            odn = pden_at(pn - 1)[bo * Hp + c];
+            ovk = pv_slot(mod3_prev(pn3))[bo * Hp + c];
+            ovk1 = pv_slot(pn3)[bo * Hp + c];
+          }
+          // group 1's phases issue the prefetch of unfold n - 2, after the
+          // word loads
+          if (gi == 1 && n >= 2) {
+            // 1/den of unfold n - 2, v of slot n - 2 (n - 2 = n + 1 mod 3)
+            rows_to_lds_fixed<NB, HPC, 512>(k.densave + (n - 2) * BHp, b0, B, pden_at(n), tid);
+            rows_to_lds_fixed<NB, HPC, 512>(k.vsave + (n - 2) * BHp, b0, B,
+                                            pv_slot(mod3_next(n3)), tid);
+          }
+        }
+        if (4 * q < nsl) {
+          const int off[4] = {ix[4 * q], ix[4 * q + 1], ix[4 * q + 2], ix[4 * q + 3]};
+#pragma unroll
+          for (int h = 0; h < 4; h += 2) {
+            if (4 * q + h < nsl) {
+#pragma unroll
+              for (int i = 0; i < 2; ++i) {
+                const int rr = 4 * q + h + i;
+                bwd_synapse_cmpe<HB>(preg[rr], ab + gi * HB, off[h + i], cvi, acc, gacc[rr]);
+                asm volatile("" : "+v"(gacc[rr].x), "+v"(gacc[rr].y), "+v"(gacc[rr].z),
+                             "+v"(gacc[rr].w));
+              }
+            }
+          }
+        }
+      }
+      // (b) the group's partials
+      float* rgi = red + gi * KS * HB * JW;
+#pragma unroll
+      for (int b = 0; b < HB; ++b) rgi[(sks * HB + b) * JW + so] = acc[b];
+      // (c) the other group's alpha/beta of unfold am from the partners'
+      // words, and the owners' own entry of the group they just finished
+      if (k.spin <= 0) {
+        gave_up = 1;  // a budget of 0: give up at the first wait, as xch_gather does
+      } else if (need) {
+#pragma unroll
+        for (int x = 0; x < XW; ++x) {
+          if (!gth[x]) continue;
+          const long long t0 = wall_clock64();
+          bool ok = true;
+          unsigned long long* wa =
+              gslot + gm[x] * PER + (gg * HB + gr[x]) * JW + (gcl[x] - gm[x] * JW);
+          while ((unsigned)(w[x] >> 32) != (unsigned)gtag) {
+            if (wall_clock64() - t0 > k.spin) {
+              ok = false;
+              break;
+            }
+            w[x] = xch_get(wa);
+          }
+          if (!ok) {
+            gave_up = 1;
+            continue;
+          }
+          const int b = gg * HB + gr[x], col = gcl[x];
+          float al = 0.f, be = 0.f;
+          if (b0 + b < B && col < H) {
+            const float gv = __uint_as_float((unsigned)w[x]);
+            const float rden = rdn[x];
+            al = gv * rden;
+            be = -gv * rvk[x] * rden;
+          }
+          ab[col * ABS + b] = make_float2(al, be);
+        }
+      }
+      if (own_next) own_ab(odn, ovk, ovk1);
+      // the prefetch issued in the previous (group 1) phase, visible to
+      // every wave after this barrier
+      if (gi == 0) wait_vm();
+      lds_barrier();
+      if (gave_up) {
+        if (k.gstate != nullptr && live && c < H)
+          k.gstate[(long long)(b0 + bo) * H + c] = __builtin_nanf("");
+        if (tid == 0) __hip_atomic_store(k.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return;
+      }
+      if (owner && og == gi) {
+        pn = n;
+        pn3 = n3;
+        pt = t;
+        pu = u;
+        pend = true;
+      }
+    }
+    n3 = mod3_prev(n3);
+    if (--u < 0) {
+      u = U - 1;
+      --t;
+    }
+  }
+  // group 1's finish of unfold 0 (nothing is published at unfold 0)
+  if (pend) {
+    const float* rg = red + og * KS * HB * JW;
+    const float s = ks_sum_wide(rg + (bo - og * HB) * JW + o, HB * JW, KS);
+    g = c < H ? fmaf(kNegLn2, s, gdir) : 0.f;
+    if (live) {
+      const long long e = ((long long)(b0 + bo) * T) * Hp + c;
+      k.dsn[e] = accA;
+      k.dsd[e] = accB;
+    }
+  }
+  if (live) {
+    if (k.gstate != nullptr && c < H) k.gstate[(long long)(b0 + bo) * H + c] = g;
+    float* np = k.npart + (long long)(b0 + bo) * 3 * Hp + c;
+    np[0] = pC;
+    np[Hp] = pGv;
+    np[2 * Hp] = pA;
+  }
+  // This cluster's share of the recurrent parameter gradients, layout
+  // [cluster][4][i][j], as ode_bwd_cl_kernel writes it.
+  const long long HH = (long long)Hp * Hp;
+  float* out = k.rpart + (long long)(k.R0 / NB + cl) * 4 * HH + (long long)sc * Hp;
+  // The image entries are indexed again from a copy of sks the compiler
+  // cannot match with the preload's, so that it does not keep the preload's
+  // addresses (or every w) live across the loop.
+  int sks_end = sks;
+  asm volatile("" : "+v"(sks_end));
+#pragma unroll
+  for (int rr = 0; rr < RCP; ++rr) {
+    if (rr < nmine) {
+      const long long a = (long long)(sks_end * RCP + rr) * Hp + sc;
+      const int j = k.cidx[a];
+      const float w = k.cimg[a].w;  // the factor the last two sums left out
+      out[j] = gacc[rr].x;
+      out[HH + j] = gacc[rr].y;
+      out[2 * HH + j] = gacc[rr].z * w;
+      out[3 * HH + j] = gacc[rr].w * w;
+    }
+  }
+}
+
+// The register-resident fused chain for the other sizes of 128 < Hp <= 512, the
+// two-group form of ode_bwd_cl2_kernel (a kernel of its own: compiled as one
+// template with it, that kernel's slot loop was scheduled 0.7% slower at B256 T64
+// H256): 12 or 16 slots cover Hp = 192 or 256, 16 slots Hp = 320 ... 448 and 20
+// Hp = 512 while no column
+// has more than 16 * RCP entries (half-dense masks; a second launch, of
+// ode_bwd_cl_kernel, covers the rest). Bound by the slot loops at two waves per
+// SIMD and the exchange of up to 16 members: B64 T32 H192 554 us (chain 996
+// and rec_grad 205 before), H512 1104 us (1868). Partials are written slot by
+// slot: through store_partials32's tile, whole planes of which half is padding,
+// B64 T32 H512 took 1124 instead of 1111 us and B256 T4 H512, whose two
+// launches add, 676 instead of 640. FACT factors w out as above, which needs
+// w != 0 wherever wE is (kChainIrregular otherwise); without it the operands
+// stay (x, y, wE, w).
+// The fourth sum is that of dl * zp, zp = x v + y the gate's argument, not of
+// dl * v: the sigma gradient is sum dl (v - mu), and summed as sum dl v less mu
+// sum dl its terms cancel only after hundreds of rounded additions (B64 T32
+// H192: error against float64 2.2e-6, 1.3e-6 with rec_grad_kernel's shorter
+// sums). A slope x below kMinSlope is raised to it so that sum dl v can be
+// taken out again at the end, unless the offset y counts beside it: then
+// |mu| = |y / x| > 1e12, and sum dl v, nothing beside mu sum dl, is left out.
+// (A gate argument past the float range, |sigma (v - mu)| > 2e38, makes that
+// synapse's sigma gradient NaN.)
+// It keeps the dense kernels' treatment of a non-finite alpha or beta: the
+// synapses left out have weight zero, and zero times it is NaN, so dL/dv of
+// every neuron of that row that has such a synapse becomes NaN. A row flag by
+// unfold parity carries it, as the forward's does a NaN state.
+template <int NB, int RCP, bool FACT, bool MOVE>
+__global__ __launch_bounds__(512) void ode_bwd_reg_kernel(BwdCK k) {
+  static_assert(NB == 2 || NB == 4 || NB == 8, "two groups of rows");
+  constexpr int JW = 32, HB = NB / 2, PER = NB * JW, PERG = HB * JW;
+  constexpr int ABS = NB + 2;  // padded alpha/beta rows, as in ode_bwd_cl_kernel
+  // gather words per thread and group: (CP - 1) * PERG <= XW * 512
+  constexpr int XW = reg_chain_words(NB, FACT);
+  extern __shared__ float4 lds4[];
+  __shared__ int gave_up;
+  __shared__ int badrow[2][NB];  // alpha/beta of that unfold parity not finite
+  const int Hp = k.Hp, H = k.H, KS = k.KS, B = k.B, T = k.T, U = k.U, CP = k.CP;
+  float2* ab = reinterpret_cast<float2*>(lds4);                  // [Hp][ABS]
+  float* red = reinterpret_cast<float*>(ab + ABS * Hp);         // [2][KS][HB][JW]
+  float* pden = red + 2 * KS * HB * JW;                         // [2][NB][Hp] by unfold parity
+  float* pv = pden + 2 * NB * Hp;                               // [3][NB][Hp] by slot mod 3
+  int* perm = reinterpret_cast<int*>(pv + 3 * NB * Hp);  // balanced_lane's scratch
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  const int ks = tid / JW, o = tid % JW;
+  int p, cl;
+  cluster_coords(blockIdx.x, CP, k.xcd_local != 0, p, cl);
+  const int c = p * JW + o;
+  const int b0 = k.R0 + cl * NB;
+  const bool owner = ks < NB;
+  const int bo = ks, og = ks / HB;
+  const bool live = owner && b0 + bo < B;
+  unsigned long long* xbase = k.xch + (long long)cl * 2 * CP * PER;
+  const long long BHp = (long long)B * Hp;
+  const float C = k.neuron[c];
+  if (T == 0) return;
+  if (cl >= k.NCL) return;  // grid padded to whole rounds of the XCDs
+  if (k.maxcnt > 0 && !chain_counts_fit(k.ccnt, Hp, k.maxcnt)) return;
+  if (tid < 2 * NB) badrow[tid / NB][tid % NB] = 0;  // before balanced_lane's barriers
+  const int RC = k.RC;  // slots of a chunk
+  // without a compacted image (RegCluster::dense) entry e of a column is row e
+  const bool dense = !FACT && k.cimg == nullptr;
   auto count = [&](int col) { return dense ? Hp : k.ccnt[col]; };
-  const int cntc = REG ? count(c) : 0;
+  const int cntc = count(c);
   auto pden_at = [&](long long m) { return pden + (m & 1) * NB * Hp; };
   auto pv_at = [&](long long m) { return pv + (m % 3) * NB * Hp; };
   // v slot r (an unfold index mod 3, kept by the loop instead of divided)
@@ -5553,7 +5901,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
       // image operands (x, y, w E, w) -> (x, y, E, w x); an entry with
       // w = 0 (a padding slot) contributes nothing either way
       preg[rr] = FACT ? make_float4(q.x, q.y, q.w != 0.f ? q.z / q.w : 0.f, q.w * q.x) : q;
-      if (REG && fabsf(q.x) < kMinSlope && fabsf(q.y) < 1e-8f) {  // the gate is 1/2 either way
+      if (fabsf(q.x) < kMinSlope && fabsf(q.y) < 1e-8f) {  // the gate is 1/2 either way
         preg[rr].x = kMinSlope;
         preg[rr].y = 0.f;
       }
@@ -5586,16 +5934,13 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
       gdir = al * C;
     }
     ab[c * ABS + bo] = make_float2(al, be);
-    if (REG && not_finite(al, be)) badrow[par][bo] = 1;
+    if (not_finite(al, be)) badrow[par][bo] = 1;
   };
   auto gout_at = [&](int b, int t, int col) {
     return k.gout[(long long)(b0 + b) * k.gs.b + (long long)t * k.gs.t + (long long)col * k.gs.c];
   };
   auto stage = [&](const float* slice, float* dst) {
-    if constexpr (REG)
-      rows_to_lds<NB, 512>(slice, b0, B, Hp, dst, tid);
-    else
-      rows_to_lds_fixed<NB, HPC, 512>(slice, b0, B, dst, tid);
+    rows_to_lds<NB, 512>(slice, b0, B, Hp, dst, tid);
   };
   auto prefetch = [&](long long m) {  // 1/den of unfold m, v of slot m
     stage(k.densave + m * BHp, pden_at(m));
@@ -5631,7 +5976,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
       be = -gg * k.vsave[ee + BHp] * rden;
     }
     ab[col * ABS + b] = make_float2(al, be);
-    if (REG && not_finite(al, be)) badrow[n_last & 1][b] = 1;
+    if (not_finite(al, be)) badrow[n_last & 1][b] = 1;
   }
   // The prefetched rows the first three phases read: v of slots n_last and
   // n_last - 1, 1/den of unfold n_last - 1.
@@ -5682,7 +6027,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
         const float* rg = red + og * KS * HB * JW;
         const float s = ks_sum_wide(rg + (bo - og * HB) * JW + o, HB * JW, KS);
         g = c < H ? fmaf(kNegLn2, s, gdir) : 0.f;
-        if (REG && badrow[pn & 1][bo] != 0 && cntc < H && c < H) g = __builtin_nanf("");
+        if (badrow[pn & 1][bo] != 0 && cntc < H && c < H) g = __builtin_nanf("");
         if (pn > 0) {
           g += gnext;
           const unsigned tag = (unsigned)pn;
@@ -5773,9 +6118,9 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
               for (int i = 0; i < 2; ++i) {
                 const int rr = 4 * q + h + i;
                 if constexpr (FACT)
-                  bwd_synapse_cmpe<HB, REG>(preg[rr], ab + gi * HB, off[h + i], cvi, acc, gacc[rr]);
+                  bwd_synapse_cmpe<HB, true>(preg[rr], ab + gi * HB, off[h + i], cvi, acc, gacc[rr]);
                 else
-                  bwd_synapse_cmp<HB, REG>(preg[rr], ab + gi * HB, off[h + i], cvi, acc, gacc[rr]);
+                  bwd_synapse_cmp<HB, true>(preg[rr], ab + gi * HB, off[h + i], cvi, acc, gacc[rr]);
                 asm volatile("" : "+v"(gacc[rr].x), "+v"(gacc[rr].y), "+v"(gacc[rr].z),
                              "+v"(gacc[rr].w));
               }
@@ -5819,7 +6164,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
             be = -gv * (EARLY ? rvk[x] : vk1[e]) * rden;
           }
           ab[col * ABS + b] = make_float2(al, be);
-          if (REG && not_finite(al, be)) badrow[am & 1][b] = 1;
+          if (not_finite(al, be)) badrow[am & 1][b] = 1;
         }
       }
       if (own_next) {
@@ -5865,7 +6210,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
     const float* rg = red + og * KS * HB * JW;
     const float s = ks_sum_wide(rg + (bo - og * HB) * JW + o, HB * JW, KS);
     g = c < H ? fmaf(kNegLn2, s, gdir) : 0.f;
-    if (REG && badrow[0][bo] != 0 && cntc < H && c < H) g = __builtin_nanf("");
+    if (badrow[0][bo] != 0 && cntc < H && c < H) g = __builtin_nanf("");
     if (live) {
       const long long e = ((long long)(b0 + bo) * T) * Hp + c;
       k.dsn[e] = accA;
@@ -5886,15 +6231,13 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
   // live across the loop.
   int sks_end = sks;
   asm volatile("" : "+v"(sks_end));
-  // REG: sum dl*v from sum dl*(x*v + y)
-  if constexpr (REG) {
-    if constexpr (MOVE) move_sums<false>(gacc, k.gsum, true);
+  if constexpr (MOVE) move_sums<false>(gacc, k.gsum, true);
+  // sum dl*v from sum dl*(x*v + y)
 #pragma unroll
-    for (int rr = 0; rr < RCP; ++rr)
-      gacc[rr].w = fabsf(preg[rr].x) < kMinSlope
-                       ? 0.f
-                       : (gacc[rr].w - preg[rr].y * gacc[rr].z) / preg[rr].x;
-  }
+  for (int rr = 0; rr < RCP; ++rr)
+    gacc[rr].w = fabsf(preg[rr].x) < kMinSlope
+                     ? 0.f
+                     : (gacc[rr].w - preg[rr].y * gacc[rr].z) / preg[rr].x;
   const long long HH = (long long)Hp * Hp;
   float* out = k.rpart + (long long)cl * 4 * HH + (long long)sc * Hp;
 #pragma unroll
@@ -5904,7 +6247,7 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
       const int j = dense ? rr * kCmpChunks + sks_end : k.cidx[a];
       const float w = FACT ? k.cimg[a].w : 1.f;  // the factor the last two sums left out
       float4 s = make_float4(gacc[rr].x, gacc[rr].y, gacc[rr].z * w, gacc[rr].w * w);
-      if (REG && k.R0 > 0) {  // a later launch of the call adds to the cluster's partial
+      if (k.R0 > 0) {  // a later launch of the call adds to the cluster's partial
         s.x += out[j];
         s.y += out[HH + j];
         s.z += out[2 * HH + j];
@@ -6097,11 +6440,14 @@ hipError_t launch_reg_bwd_mv(const Plan& p, BwdCK a, hipStream_t s) {
   const RegCluster& g = p.rb;
   const dim3 grid(reg_grid(g)), block(512);
   const size_t lds = (size_t)reg_bwd_lds(g, p.Hp);
+  // the partners' words of a row group over 512 threads
+  if ((g.CP - 1) * (NB / 2) * 32 > reg_chain_words(NB, g.RC > 16) * 512)
+    return hipErrorInvalidConfiguration;
   if (g.RC == 12 || g.RC == 16) {
     if (g.RC == 12)
-      LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 12, false, true, MOVE>), grid, block, lds, s, a);
+      LTC_LAUNCH((ode_bwd_reg_kernel<NB, 12, false, MOVE>), grid, block, lds, s, a);
     else
-      LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 16, false, true, MOVE>), grid, block, lds, s, a);
+      LTC_LAUNCH((ode_bwd_reg_kernel<NB, 16, false, MOVE>), grid, block, lds, s, a);
     return hipGetLastError();
   }
   // The kernel over at most reg_chain_slots synapses a thread, then the one
@@ -6110,9 +6456,9 @@ hipError_t launch_reg_bwd_mv(const Plan& p, BwdCK a, hipStream_t s) {
   a.maxcnt = g.dense ? 0 : 16 * reg_chain_slots(g.RC);
   if (g.dense) {
   } else if (reg_chain_slots(g.RC) == 16)
-    LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 16, true, true, MOVE>), grid, block, lds, s, a);
+    LTC_LAUNCH((ode_bwd_reg_kernel<NB, 16, true, MOVE>), grid, block, lds, s, a);
   else
-    LTC_LAUNCH((ode_bwd_cl2_kernel<NB, 20, true, true, MOVE>), grid, block, lds, s, a);
+    LTC_LAUNCH((ode_bwd_reg_kernel<NB, 20, true, MOVE>), grid, block, lds, s, a);
   const size_t lds2 = (size_t)std::max(cluster_chain_lds(NB, p.Hp, 16, 32, false),
                                        partial_tile_lds(p.Hp));
   a.xcd_local = 0;  // streamed operands: members spread over the XCDs (cluster_coords)

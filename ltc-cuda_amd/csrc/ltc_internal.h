@@ -511,6 +511,10 @@ constexpr int kRegChainSlots = 20;
 // to 16 (Hp <= 256); beyond, enough for half-dense masks (at Hp = 512 the
 // fullest of 512 columns has about 290 entries, 19 a thread; at 448, 256).
 inline int reg_chain_slots(int rc) { return rc <= 16 ? rc : (rc <= 28 ? 16 : 20); }
+// Exchange words a thread of the register-resident chain gathers per row group:
+// (CP - 1) * NB / 2 * 32 over 512 threads, with CP = 6 or 8, or up to 16 beyond
+// 16 slots a thread.
+constexpr int reg_chain_words(int nb, bool wide) { return wide ? nb / 2 : (nb == 8 ? 2 : 1); }
 inline long long reg_bwd_lds(const RegCluster& g, int hp) {
   const long long n = (g.NB + 2LL) * hp * 8 + (long long)g.KS * g.NB * g.JW * 4 +
                       chain_pf_bytes(g.NB) * g.NB * hp + 512 * 4 + 8 * (kRegChainSlots + 1) * 4;
