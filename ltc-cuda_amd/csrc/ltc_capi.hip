@@ -293,8 +293,8 @@ void plan_reg_forward(ltc::Plan& p, int ncu) {
 // least kRegSumTerms. Largest 2-norm error of the w, mu and erev gradients
 // against float64, rec_grad_kernel / never moved / moved, in units of 1e-7: B2
 // T100 H192 2.9 / 9.6 / 3.0, B64 T32 H192 3.5 / 5.5 / 3.2, B300 T16 H256 4.7 /
-// 7.4 / 4.3, B128 T8 H384 3.9 / 5.6 / 3.0. A move costs about 2 us a launch
-// (12 slots; 4 with 16 or 20): those four steps took 1.9, 1.7, 2.3 and 0%
+// 7.4 / 4.3, B128 T8 H384 3.9 / 5.6 / 3.0. A move takes 2 to 4 us (12 to 20
+// slots): those four steps take 2.0, 1.6, 1.2 and 0%
 // longer for it.
 constexpr int kRegSumTerms = 48;
 

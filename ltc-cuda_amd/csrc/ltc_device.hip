@@ -4907,7 +4907,7 @@ __device__ __forceinline__ void move_sums(float4 (&gacc)[N], float4* gsum, bool 
   const __amdgpu_buffer_rsrc_t r = image_rsrc(gsum + (long long)g * N * 512, N * 512LL * 16);
   int lane_bytes = threadIdx.x * 16;
   asm volatile("" : "+v"(lane_bytes));
-  constexpr int G = N <= 16 ? 4 : 2;
+  constexpr int G = N == 12 ? 12 : (N == 16 ? 4 : 2);
 #pragma unroll
   for (int q = 0; q < N; q += G) {
     if (moved) {
