@@ -2611,6 +2611,7 @@ constexpr int RG_NT = 32;
 // Entries up to which a tile of 2048 goes by its list: six slots a thread cost
 // about what the dense form's eight do.
 constexpr int kRecListMax = 1536;
+static_assert(kRecListMax <= 6 * 256, "six slots a thread");
 
 struct RecGK {
   const float4* recF;
@@ -2623,22 +2624,58 @@ struct RecGK {
   const int* gate;  // behind clusters: run only when their status word is set
 };
 
+// A listed synapse's operands, the LDS positions of its v_i and alpha/beta_j, and
+// its sums.
+struct RecSyn {
+  float4 p;
+  int lv, lab;
+  float sWE, sWP, sD, sDv;
+};
+
+// The staged chunk of `cnt` instances for this thread's first NS synapses.
+template <int NS, int N>
+__device__ __forceinline__ void rec_grad_chunk(RecSyn (&y)[N], const float (*vsh)[32],
+                                               const float2 (*absh)[64], int cnt) {
+  // UN instances at a time at constant LDS offsets; those past the chunk
+  // hold alpha = beta = 0 and add zero. (With 2 or 1 of them and three waves
+  // a SIMD instead of two: 88 -> 98 us.)
+  constexpr int UN = 4;
+#pragma unroll 1
+  for (int nn = 0; nn < cnt; nn += UN) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+#pragma unroll
+      for (int q = 0; q < NS; ++q) {
+        const float v = (&vsh[nn][0])[u * 32 + y[q].lv];
+        const float2 c = (&absh[nn][0])[u * 64 + y[q].lab];
+        const float4 p = y[q].p;
+        const float a = gate(fmaf(p.x, v, p.y));
+        const float a2 = fmaf(-a, a, a);
+        y[q].sWE = fmaf(c.x, a, y[q].sWE);
+        y[q].sWP = fmaf(c.y, a, y[q].sWP);
+        const float dl = fmaf(c.x, p.z, c.y * p.w) * a2;
+        y[q].sD += dl;
+        y[q].sDv = fmaf(dl, v, y[q].sDv);
+      }
+    }
+  }
+}
+
+// The listed synapses of a tile that needs NS slots: its first waves run NS, the
+// others (not `full`) NS - 1. NS is uniform over the workgroup, whose barriers
+// every wave passes at the same place.
 template <int NS>
 __device__ __forceinline__ void rec_grad_rows(const RecGK& k, const unsigned short* list, int total,
-                                              float (*vsh)[32], float2 (*absh)[64]) {
+                                              bool full, float (*vsh)[32], float2 (*absh)[64]) {
   const int Hp = k.Hp, tid = threadIdx.x;
   const int jb = blockIdx.x * 64, ib = blockIdx.y * 32;
-  float4 p[NS];
-  int lv[NS], lab[NS];  // LDS positions of the entry's v_i and alpha/beta_j
-  float sWE[NS], sWP[NS], sD[NS], sDv[NS];
+  RecSyn y[NS];
 #pragma unroll
   for (int q = 0; q < NS; ++q) {
-    sWE[q] = sWP[q] = sD[q] = sDv[q] = 0.f;
     const int e = tid + 256 * q;
     const int c = e < total ? list[e] : 0, i = c >> 6, j = c & 63;
-    lv[q] = i;
-    lab[q] = j;
-    p[q] = e < total ? k.recF[(ib + i) * Hp + jb + j] : make_float4(0.f, 0.f, 0.f, 0.f);
+    y[q] = RecSyn{e < total ? k.recF[(ib + i) * Hp + jb + j] : make_float4(0.f, 0.f, 0.f, 0.f),
+                  i, j, 0.f, 0.f, 0.f, 0.f};
   }
   const long long nb = (long long)blockIdx.z * k.nper;
   const long long ne = min(k.N, nb + k.nper);
@@ -2672,29 +2709,11 @@ __device__ __forceinline__ void rec_grad_rows(const RecGK& k, const unsigned sho
     for (int q = 0; q < NA; ++q) absh[q * 4 + (tid >> 6)][tid & 63] = nab[q];
     __syncthreads();
     if (n0 + RG_NT < ne) fetch(n0 + RG_NT);
-    // UN instances at a time at constant LDS offsets; those past the chunk
-    // hold alpha = beta = 0 and add zero. (With 2 or 1 of them and three waves
-    // a SIMD instead of two: 88 -> 98 us.)
-    constexpr int UN = 4;
     const int cnt = (int)min((long long)RG_NT, ne - n0);
-#pragma unroll 1
-    for (int nn = 0; nn < cnt; nn += UN) {
-#pragma unroll
-      for (int u = 0; u < UN; ++u) {
-#pragma unroll
-        for (int q = 0; q < NS; ++q) {
-          const float v = (&vsh[nn][0])[u * 32 + lv[q]];
-          const float2 c = (&absh[nn][0])[u * 64 + lab[q]];
-          const float a = gate(fmaf(p[q].x, v, p[q].y));
-          const float a2 = fmaf(-a, a, a);
-          sWE[q] = fmaf(c.x, a, sWE[q]);
-          sWP[q] = fmaf(c.y, a, sWP[q]);
-          const float dl = fmaf(c.x, p[q].z, c.y * p[q].w) * a2;
-          sD[q] += dl;
-          sDv[q] = fmaf(dl, v, sDv[q]);
-        }
-      }
-    }
+    if (full)
+      rec_grad_chunk<NS>(y, vsh, absh, cnt);
+    else if constexpr (NS > 1)
+      rec_grad_chunk<NS - 1>(y, vsh, absh, cnt);
     __syncthreads();
   }
   const long long HH = (long long)Hp * Hp;
@@ -2702,11 +2721,11 @@ __device__ __forceinline__ void rec_grad_rows(const RecGK& k, const unsigned sho
 #pragma unroll
   for (int q = 0; q < NS; ++q) {
     if (tid + 256 * q < total) {
-      float* o = out + (ib + lv[q]) * Hp + jb + lab[q];
-      o[0] = sWE[q];
-      o[HH] = sWP[q];
-      o[2 * HH] = sD[q];
-      o[3 * HH] = sDv[q];
+      float* o = out + (ib + y[q].lv) * Hp + jb + y[q].lab;
+      o[0] = y[q].sWE;
+      o[HH] = y[q].sWP;
+      o[2 * HH] = y[q].sD;
+      o[3 * HH] = y[q].sDv;
     }
   }
 }
@@ -2835,13 +2854,14 @@ __global__ __launch_bounds__(256) void rec_grad_kernel(RecGK k) {
     list[at++] = (unsigned short)((i << 6) | (j0 + q));
   }
   __syncthreads();
-  // slots of this wave: its first entry is 64 w
-  const int ns = __builtin_amdgcn_readfirstlane(total > 64 * w ? (total - 64 * w + 255) / 256 : 0);
+  // whether this wave, whose first entry is 64 w, has as many slots as the first
+  const int ns = __builtin_amdgcn_readfirstlane((total + 255) / 256);
+  const bool full = __builtin_amdgcn_readfirstlane(total > 256 * (ns - 1) + 64 * w);
   switch (ns) {
 #define LTC_RG(N) \
-  case N: rec_grad_rows<N>(k, list, total, vsh, absh); break;
-    LTC_RG(2) LTC_RG(3) LTC_RG(4) LTC_RG(5) LTC_RG(6)
-    default: rec_grad_rows<1>(k, list, total, vsh, absh); break;
+  case N: rec_grad_rows<N>(k, list, total, full, vsh, absh); break;
+    LTC_RG(1) LTC_RG(2) LTC_RG(3) LTC_RG(4) LTC_RG(5) LTC_RG(6)
+    default: break;  // no synapse in the tile
 #undef LTC_RG
   }
 }
