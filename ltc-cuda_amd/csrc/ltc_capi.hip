@@ -624,7 +624,7 @@ BwdWs carve_bwd(const ltc::Plan& p, Carver& c, bool images = true) {
   w.spart = c.take<float>(nrc * 4 * p.Dp * p.Hp);
   w.dxpart = c.take<float>((long long)(p.Hp / 32) * p.B * p.T * p.Dp);
   w.cb = carve_cluster(p, c, true);
-  w.ps.rec = c.take<float>((long long)ltc::presum_parts(p.NCH) * 4 * p.Hp * p.Hp);
+  w.ps.rec = c.take<float>((long long)ltc::presum_parts((int)nch) * 4 * p.Hp * p.Hp);
   w.ps.neuron = c.take<float>((long long)ltc::presum_parts(p.B) * 3 * p.Hp);
   w.ps.ln = c.take<float>((long long)ltc::presum_parts(ltc::ln_bwd_blocks(p)) * 4 * p.Dp);
   return w;

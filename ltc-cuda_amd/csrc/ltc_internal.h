@@ -623,15 +623,15 @@ struct GradOut {
 // Long partial sums (the per-row neuron partials over B, the recurrent
 // gradient partials over NCH) get a parallel first pass into at most 64
 // partials each: presum_parts(M) of them, or 0 when M is small enough to sum
-// directly. The scratch buffers hold presum_parts(NCH) * 4*Hp*Hp and
-// presum_parts(B) * 3*Hp floats.
+// directly. The scratch buffers hold presum_parts(recurrent partials) * 4*Hp*Hp
+// and presum_parts(B) * 3*Hp floats.
 inline int presum_parts(int m) {
   if (m <= 64) return 0;
   const int rpb = (m + 63) / 64 > 32 ? (m + 63) / 64 : 32;
   return (m + rpb - 1) / rpb;
 }
 struct PresumBuf {
-  float* rec;     // presum_parts(NCH) x 4*Hp*Hp
+  float* rec;     // presum_parts(recurrent partials) x 4*Hp*Hp
   float* neuron;  // presum_parts(B) x 3*Hp
   float* ln;      // module path: presum_parts(ln_bwd_blocks) x 4*Dp
 };
