@@ -6506,15 +6506,13 @@ hipError_t bwd_cl_by_rcp(const Plan& p, const BwdCK& a, hipStream_t s) {
   const dim3 grid(p.NCLB * p.CPB), block(p.JWB * p.KSB);
   const size_t lds = bwd_cl_lds_bytes(p);
   if (p.FUSE) {
-    // 32-column members, 512 threads: 16 register-resident synapses each
-    // (Hp = 256) or 32 streamed ones (Hp = 512).
+    // 32-column members, 512 threads, 16 register-resident synapses each (Hp =
+    // 256; at 512 the register-resident clusters run every batch).
     if (p.JWB != 32 || p.KSB != 16) return hipErrorInvalidConfiguration;
     if (p.RCB == 16 && NB >= 2)
       LTC_LAUNCH((ode_bwd_cl2_kernel<(NB >= 2 ? NB : 2)>), grid, block, lds, s, a);
     else if (p.RCB == 16)
       LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 16, true>), grid, block, lds, s, a);
-    else if (p.RCB == 32)
-      LTC_LAUNCH((ode_bwd_cl_kernel<NB, 32, 0, true, 32>), grid, block, lds, s, a);
     else
       return hipErrorInvalidConfiguration;
   } else {

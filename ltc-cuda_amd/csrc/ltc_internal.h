@@ -508,8 +508,11 @@ inline long long reg_fwd_lds(const RegCluster& g, int hp) {
 // slots, and the balanced lane order's scratch (counts up to kRegChainSlots).
 constexpr int kRegChainSlots = 20;
 // Synapses a chain thread of Hp / 16 = rc holds in registers: all of them up
-// to 16 (Hp <= 256); beyond, enough for half-dense masks (at Hp = 512 the
-// fullest of 512 columns has about 290 entries, 19 a thread; at 448, 256).
+// to 16 (Hp <= 256); beyond, what half-dense masks need: 20 at Hp = 512, where
+// the fullest of 512 columns has about 290 entries, and 16 up to Hp = 448. There
+// the limit of 256 entries is met by nearly every mask to H = 430 or so, but some
+// column exceeds it in about one half-dense mask of ten at H = 440 and of three
+// at 448, and such a call takes the streaming chain.
 inline int reg_chain_slots(int rc) { return rc <= 16 ? rc : (rc <= 28 ? 16 : 20); }
 // Exchange words a thread of the register-resident chain gathers per row group:
 // (CP - 1) * NB / 2 * 32 over 512 threads, with CP = 6 or 8, or up to 16 beyond
