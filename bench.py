@@ -188,7 +188,7 @@ def kernel_times(capi, fn, iters):
 
 
 def _kernel_flops_by_launch(c, plan, ktimes, counts=None):
-    fl = kernel_flops(c, bool(plan["fuse"]), counts)
+    fl = kernel_flops(c, bool(plan["fuse"] or plan.get("reg_bwd_members")), counts)
     if ((plan.get("module_row_bwd_fused") or plan.get("module_row128_rec_fused"))
             and "ltc_sens_bwd" not in ktimes):
         # the chain launch also runs the sensory backward (its companions)
@@ -204,8 +204,8 @@ def _kernel_flops_by_launch(c, plan, ktimes, counts=None):
 
 def roofline(c, ktimes, plan, traffic=None, counts=None):
     """Dominant kernel of the step against the FP32 peak. `frac` prices the
-    unit's dense work (every synapse, masked or not: SURVEY's FLOP_fwd = 10 and
-    FLOP_bwd = 22 per synapse); `frac_evaluated` the synapses the kernels
+    unit's dense work (every synapse, masked or not: 10 FLOP forward and 22
+    backward per synapse); `frac_evaluated` the synapses the kernels
     actually evaluate (the compacted kernels skip masked ones)."""
     fl = _kernel_flops_by_launch(c, plan, ktimes)
     fle = _kernel_flops_by_launch(c, plan, ktimes, counts)
@@ -238,7 +238,21 @@ def mask_density(m):
             float((m.sensory_sparsity_mask != 0).float().mean()))
 
 
-def syn_counts(c, plan=None, density=(1.0, 1.0)):
+def skips_masked(m, plan):
+    """Whether the forward and the chain of a call skip masked recurrent synapses:
+    the plan's compacted kernels (cmp_fwd / cmp_bwd), or the register-resident
+    clusters when they read compacted images; the chain above 256 columns only
+    while every neuron has at most 256 outgoing synapses (320 above 448), else the
+    kernel that streams dense operands runs."""
+    fwd = plan.get("cmp_fwd") or (plan.get("reg_fwd_members") and not plan.get("reg_fwd_dense"))
+    limit = plan["Hp"] if plan["Hp"] <= 256 else (256 if plan["Hp"] <= 448 else 320)
+    fits = int((m.sparsity_mask != 0).sum(1).max()) <= limit
+    bwd = plan.get("cmp_bwd") or (plan.get("reg_bwd_members") and not plan.get("reg_bwd_dense")
+                                  and fits)
+    return {"forward": bool(fwd), "chain": bool(bwd)}
+
+
+def syn_counts(c, plan=None, density=(1.0, 1.0), skips=None):
     """Synapse evaluations per step as the kernels run them, and the layer's
     active-only count (both masks' densities):
     - sens_fwd: the compacted sensory launch skips masked sensory synapses
@@ -249,23 +263,26 @@ def syn_counts(c, plan=None, density=(1.0, 1.0)):
       module_row_bwd_fused, and module_row128_rec_fused with D <= 128)
       evaluate every one;
     - rec_fwd / rec_dv: the compacted forward and chain skip masked recurrent
-      synapses (plan fields cmp_fwd / cmp_bwd);
-    - rec_bwd: the parameter-gradient sums, skipped with the chain only when
-      the chain forms them itself (fuse); an unfused chain's rec_grad pass
-      evaluates every synapse."""
+      synapses (`skips`, skips_masked);
+    - rec_bwd: the parameter-gradient sums, skipped with the chain when the chain
+      forms them itself; an unfused chain's rec_grad pass lists the unmasked ones
+      of each tile that is not nearly full, its companions evaluate every one."""
     rho_r, rho_s = density
     sens = c["B"] * c["T"] * c["D"] * c["H"]
     rec = c["B"] * c["T"] * c["U"] * c["H"] ** 2
     plan = plan or {}
-    skip_bwd = plan.get("cmp_bwd") and plan.get("fuse")
+    skips = skips or {"forward": False, "chain": False}
+    fused = plan.get("fuse") or plan.get("reg_bwd_members")
+    skip_bwd = (skips["chain"] if fused or not plan
+                else rho_r <= 0.75 and not plan.get("module_row128_rec_fused"))
     sens_cmp = bool(plan) and not plan.get("module_sens_in_prep")
     sens_bwd_dense = (not plan or plan.get("module_row_bwd_fused")
                       or (plan.get("module_row128_rec_fused") and plan.get("Dp", 0) <= 128))
     return {"sens_fwd": sens * (rho_s if sens_cmp else 1.0),
             "sens_bwd": sens * (1.0 if sens_bwd_dense else rho_s),
-            "rec_fwd": rec * (rho_r if plan.get("cmp_fwd") else 1.0),
+            "rec_fwd": rec * (rho_r if skips["forward"] else 1.0),
             "rec_bwd": rec * (rho_r if skip_bwd else 1.0),
-            "rec_dv": rec * (rho_r if plan.get("cmp_bwd") else 1.0),
+            "rec_dv": rec * (rho_r if skips["chain"] else 1.0),
             "active": sens * rho_s + rec * rho_r}
 
 
@@ -637,10 +654,11 @@ def measure_config(name, c, capi, cpu, probe=None):
     train = c["loss"] is not None
     plan = capi.plan(c["B"], c["T"], c["D"], c["H"], c["U"])
     dens = mask_density(m)
-    counts = syn_counts(c, plan, dens)
+    skips = skips_masked(m, plan)
+    counts = syn_counts(c, plan, dens, skips)
     rec = {"shape": {k: c[k] for k in ("B", "T", "D", "H", "U")}, "n_syn": n_syn(c),
            "loss": c["loss"], "x": c["x"]}
-    rec.update(sparsity_record(plan, dens, counts))
+    rec.update(sparsity_record(skips, dens, counts))
 
     if train:
         def fn():
@@ -703,11 +721,10 @@ def measure_config(name, c, capi, cpu, probe=None):
     return rec
 
 
-def sparsity_record(plan, dens, counts):
+def sparsity_record(skips, dens, counts):
     """What the kernels skip, and the active-only count beside the dense one."""
     return {"mask_density": {"recurrent": round(dens[0], 5), "sensory": round(dens[1], 5)},
-            "skips_masked_recurrent": {"forward": bool(plan.get("cmp_fwd")),
-                                       "chain": bool(plan.get("cmp_bwd"))},
+            "skips_masked_recurrent": dict(skips),
             "n_syn_active": int(round(counts["active"])),
             "n_syn_evaluated_fwd": int(round(counts["sens_fwd"] + counts["rec_fwd"])),
             "n_syn_evaluated_bwd": int(round(counts["sens_bwd"] + counts["rec_bwd"]))}
@@ -816,7 +833,8 @@ def main():
     m, x, target = make_inputs(c, "cuda:0")
     plan = capi.plan(c["B"], c["T"], c["D"], c["H"], c["U"])
     dens = mask_density(m)
-    counts = syn_counts(c, plan, dens)
+    skips = skips_masked(m, plan)
+    counts = syn_counts(c, plan, dens, skips)
 
     for _ in range(max(args.warmup, 200)):
         step(m, x, target)
@@ -864,7 +882,7 @@ def main():
                    "step": "whole step replayed as one HIP graph" if use_graph
                            else "eager module forward + loss.backward()"},
         "active_synapse_updates_per_s": counts["active"] / (ms * 1e-3),
-        **sparsity_record(plan, dens, counts),
+        **sparsity_record(skips, dens, counts),
         "eager_ms_per_step": round(eager_ms, 5),
         "eager_synapse_updates_per_s": n_syn(c) / (eager_ms * 1e-3),
         "graphed_ms_per_step": None if graph_ms is None else round(graph_ms, 5),
