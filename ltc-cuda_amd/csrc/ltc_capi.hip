@@ -288,14 +288,13 @@ void plan_reg_forward(ltc::Plan& p, int ncu) {
 // A gradient sum kept over a whole launch is T * U * NB rounded additions long,
 // however small the batch, and what one row adds keeps its sign for long: the
 // sums move out of the registers, and start again, after as many unfolds as
-// make a quarter of the terms of one of rec_grad_kernel's partials (rec_grad_
-// chunks; half at Hp = 512, whose chains kept whole sums before too), and at
-// least kRegSumTerms. Largest 2-norm error of the w, mu and erev gradients
-// against float64, rec_grad_kernel / never moved / moved, in units of 1e-7: B2
-// T100 H192 2.9 / 9.6 / 3.0, B64 T32 H192 3.5 / 5.5 / 3.2, B300 T16 H256 4.7 /
-// 7.4 / 4.3, B128 T8 H384 3.9 / 5.6 / 3.0. A move takes 2 to 4 us (12 to 20
-// slots): those four steps take 2.0, 1.6, 1.2 and 0%
-// longer for it.
+// make half the terms of one of rec_grad_kernel's partials (rec_grad_chunks),
+// shorter still where later launches of the call add theirs, and at least
+// kRegSumTerms. 2-norm error of the w gradient against float64, rec_grad_kernel /
+// never moved / moved, in units of 1e-7: B2 T100 H192 2.9 / 9.6 / 3.0, B64 T32
+// H192 3.5 / 5.5 / 3.6, B300 T16 H256 4.7 / 7.4 / 4.3, B128 T8 H384 3.9 / 5.6 /
+// 4.0 (mu and erev alike, sigma lower than either). A move takes 2 to 4 us (12 to
+// 20 slots): those four steps take 2.3, 1.6, 0.7 and 0% longer for it.
 constexpr int kRegSumTerms = 48;
 
 // The chain: members of 32 columns and 512 threads, whose registers hold the
@@ -330,7 +329,7 @@ void plan_reg_chain(ltc::Plan& p, int ncu) {
   // 253. Up to Hp = 256 the compacted form is the faster at one unfold already
   // (B16 H192 68 / 73).
   g.dense = g.RC > 16 && (long long)p.T * p.U * g.NB * g.L <= kRegDenseRows;
-  const long long nch = (g.RC == 32 ? 2 : 4) * rec_grad_chunks(p);
+  const long long nch = 2LL * (g.RC == 32 ? 1 : g.L) * rec_grad_chunks(p);
   const long long terms = std::max<long long>((p.N + nch - 1) / nch, kRegSumTerms);
   const long long fl = (terms + g.NB - 1) / g.NB;
   g.FL = fl < (long long)p.T * p.U ? (int)fl : 0;
