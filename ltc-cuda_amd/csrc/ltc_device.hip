@@ -2600,8 +2600,8 @@ __global__ __launch_bounds__(512) void ode_bwd_row_fused_kernel(BwdK k, RowCompa
 // and nothing for the padding of H to Hp. Neighbouring threads mostly share i
 // and have neighbouring j, so their LDS reads of v_i and alpha/beta_j stay
 // broadcasts and nearly conflict-free. Nearly full tiles take every synapse
-// (rec_grad_dense). VALU-bound (B128 T25 H100 half-dense: 128 us with every
-// synapse of the padded tile evaluated, 88 us this way).
+// (rec_grad_dense). VALU-bound (B128 T25 H100 half-dense, kernel trace: 129
+// us with every synapse of the padded tile evaluated, 96 us this way).
 // Per synapse and n:  a = gate, a2 = a(1-a), h = alpha*WE + beta*WP,
 //   sWE += alpha*a, sWP += beta*a, sD += h*a2, sDv += h*a2*v_i
 // and the finalize kernel forms dM = -S*sD and dS = sDv - M*sD. Partials of
@@ -5831,8 +5831,8 @@ __global__ __launch_bounds__(512) void ode_bwd_cl2_kernel(BwdCK k) {
 // Hp = 512 while no column
 // has more than 16 * RCP entries (half-dense masks; a second launch, of
 // ode_bwd_cl_kernel, covers the rest). Bound by the slot loops at two waves per
-// SIMD and the exchange of up to 16 members: B64 T32 H192 554 us (chain 996
-// and rec_grad 205 before), H512 1104 us (1868). Partials are written slot by
+// SIMD and the exchange of up to 16 members: B64 T32 H192 565 us, 550 without
+// moving its sums (chain 996 and rec_grad 205 before), H512 1084 us (1868). Partials are written slot by
 // slot: through store_partials32's tile, whole planes of which half is padding,
 // B64 T32 H512 took 1124 instead of 1111 us and B256 T4 H512, whose two
 // launches add, 676 instead of 640. FACT factors w out as above, which needs
