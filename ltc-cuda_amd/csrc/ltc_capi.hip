@@ -229,11 +229,11 @@ constexpr long long kRegDenseRows = 24;
 // without gradients 1.3 to 1.6 times the own kernels' time); three do where those
 // leave many CUs idle (B600: 300 workgroups of two rows; 0.78 to 0.90 times, and
 // 1.05 to 1.39 at B1024 and B256, where they fill the chip).
-bool reg_too_short(const ltc::Plan& p, int launches) {
+bool reg_too_short(const ltc::Plan& p, int launches, int ncu) {
   const long long n = (long long)p.T * p.U;
   if (launches <= 1 || n > 3) return false;
-  const int wgs = (p.B + p.NB - 1) / p.NB, rounds = (wgs + 255) / 256;
-  return n <= 2 || p.CP > 0 || wgs * 10 >= rounds * 256 * 9;
+  const int wgs = (p.B + p.NB - 1) / p.NB, rounds = (wgs + ncu - 1) / ncu;
+  return n <= 2 || p.CP > 0 || wgs * 10 >= rounds * ncu * 9;
 }
 
 // Register-resident clusters for 128 < Hp <= 512 where the plan above has no
@@ -272,7 +272,7 @@ void plan_reg_forward(ltc::Plan& p, int ncu) {
     }
   }
   reg_cluster_counts(g, p.B, ncu / g.CP, ncu);
-  if (reg_too_short(p, g.L)) return;
+  if (reg_too_short(p, g.L, ncu)) return;
   // Compacting an image takes longer than the dense one (Hp = 320 ... 512: 13 to
   // 20 us of a prep launch's 30), which few unfolds do not win back; one row per
   // cluster is bound by the exchange, not by its slots, and hardly needs it.
@@ -322,7 +322,7 @@ void plan_reg_chain(ltc::Plan& p, int ncu) {
     if ((p.B + nb - 1) / nb <= slots) break;
   }
   reg_cluster_counts(g, p.B, slots, ncu);
-  if (reg_too_short(p, g.L)) return;
+  if (reg_too_short(p, g.L, ncu)) return;
   // The same for the chains that would stream a dense mask: step B1 H512 T1 154
   // us with the compacted image, 133 streaming; T2 191 / 181, T4 271 / 288; B64
   // H320 T1 147 / 140, T2 197 / 203; B256 H320, one unfold 198 / 180, three 251 /
